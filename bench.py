@@ -66,7 +66,7 @@ def collide_kernel_bytes(spheres: float, wall_contacts: float) -> float:
     return 480.0 * spheres + 40.0 * wall_contacts
 
 
-# The library walks the pairs inside k_collide (k_pairs returns at once) when the step's full
+# A library with a pair pass of its own walks the pairs inside k_collide when the step's full
 # pass holds fewer spheres than this.
 MERGE_PAIRS_BELOW = 65536
 
@@ -74,11 +74,11 @@ MERGE_PAIRS_BELOW = 65536
 def kernel_rooflines(tm, n, info, n_pp, n_wall, fuse):
     """Per-step time and achieved HBM bandwidth of the step's kernels from the event-timed
     steps: k_lite_move (spheres outside the full pass), k_pairs and k_collide (the full-pass
-    spheres, contact_spheres of the last step). On a small full pass k_collide also walks the
-    pairs (their bytes count for it) and k_pairs only reads the queue counters."""
+    spheres, contact_spheres of the last step). Without a pair pass of its own (no time for it, or a
+    small full pass) k_collide walks the pairs and their bytes count for it."""
     steps = max(tm["steps"], 1)
     full = info["contact_spheres"]
-    merged = full < MERGE_PAIRS_BELOW
+    merged = full < MERGE_PAIRS_BELOW or not tm.get("pair_pass_ms", 0) > 0
     out = {}
     if fuse and tm["lite_move_ms"] > 0:
         ms = tm["lite_move_ms"] / steps

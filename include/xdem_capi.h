@@ -164,14 +164,14 @@ typedef struct xdem_ctx_config {
                                     so results do not change. Small values exist to test that
                                     path. */
     unsigned int full_blocks;    /* blocks of the full-pass kernels (pair, triangle and contact
-                                    passes), rounded down to a multiple of 64 (0 = 1024). They
+                                    passes), taken to a multiple of 64 (0 = two per CU). They
                                     stride over the queued spheres, so results do not depend on
-                                    it; a few blocks per CU keep several waves per SIMD to hide
-                                    the neighbour gathers. */
-    unsigned int merge_pairs_below; /* below this many spheres in a step's full pass the contact
-                                    kernel walks their pairs itself instead of a pair pass of
-                                    its own (0 = 65536; 1 = never). Results do not depend on
                                     it. */
+    unsigned int merge_pairs_below; /* a step's full pass of fewer spheres than this is divided
+                                    into groups of 4 to 64 spheres to a wave, as few as fill the
+                                    device; from this size on every wave takes 64 (0 = the
+                                    first rule for every size; 1 = the second). Results do not
+                                    depend on it. */
     int keep_order;              /* 0 (default): the context stores each scene's spheres in the
                                     bucket order of their initial positions (a stable sort on
                                     the bucket key at commit), so that the neighbours a kernel
@@ -366,8 +366,7 @@ int xdem_ctx_graph_launch(xdem_ctx* ctx, unsigned int nlaunch);
  * into the contact passes), out[4] = per-step pair test (k_touch) ms, out[5] = k_lite_move
  * ms (fused mode; 0 otherwise), out[6] = k_collide ms and out[7] = the triangle pass before it
  * (k_mesh_pass, with the wait for the fork; about 0 without meshes) ms, both on the second
- * stream, out[8] = the sphere-pair pass (k_pairs, on the second stream between the two; it
- * returns at once on a small full pass, whose pairs k_collide walks) ms. */
+ * stream, out[8] = 0 (the sphere pairs are part of k_collide). */
 int xdem_ctx_set_timing(xdem_ctx* ctx, int on);
 int xdem_ctx_timing(xdem_ctx* ctx, double out[9]);
 

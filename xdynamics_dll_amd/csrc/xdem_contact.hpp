@@ -101,11 +101,12 @@ __device__ __forceinline__ void sphere_contact(const ContactConst& cc, double dt
     acc.M = acc.M + cvt3<double>(cross(dc, fnt));
 }
 
-// One contact of sphere i with sphere j evaluated on its own (the pair pass): the parts of
-// sphere_contact that do not depend on the earlier pairs of the sphere. out = Fn (3), Ft (3),
-// the lever arm dc (3), in T and stored as double, and the rolling-resistance term; returns
-// whether Ft was set (|e| != 0). sphere_pair_sum then adds the pairs in visiting order with
-// the same operations as sphere_contact, carrying Ft over where it was not set (quirk Q4).
+// One contact of sphere i with sphere j evaluated on its own: the parts of sphere_contact that do
+// not depend on the earlier pairs of the sphere. Returns whether Ft was set (|e| != 0). Set: out =
+// Fn + Ft (3), its moment about the centre (3), the rolling-resistance term, Ft (3). Not set (the
+// force needs the previous pair's Ft, quirk Q4): out = Fn (3), the lever arm (3), the
+// rolling-resistance term. All in T, stored as double. sphere_pair_add then adds the pairs in
+// visiting order with sphere_contact's operations.
 template <class T, int MODEL, bool GPU_LAW>
 __device__ __forceinline__ bool sphere_pair_eval(const ContactConst& cc, double dt, V4<double> ipos, V3<double> ivel,
                                                  V3<double> iom, double im, V4<double> jpos, V3<double> jvel,
@@ -123,26 +124,36 @@ __device__ __forceinline__ bool sphere_pair_eval(const ContactConst& cc, double 
     V3<T> Fn, Ft = mk3(T(0), T(0), T(0));
     const bool set = force_law<T, MODEL, GPU_LAW>(cc, c, g.cdist, dt, sd0, sd1, rv, unit, Ft, Fn);
     const V3<T> dc = cvt3<T>(dcpr);
-    out[0] = (double)Fn.x; out[1] = (double)Fn.y; out[2] = (double)Fn.z;
-    out[3] = (double)Ft.x; out[4] = (double)Ft.y; out[5] = (double)Ft.z;
-    out[6] = (double)dc.x; out[7] = (double)dc.y; out[8] = (double)dc.z;
-    out[9] = (double)(c.eq_r * T(cc.rfric) * length(Fn));
+    const V3<T> f = set ? Fn + Ft : Fn;
+    const V3<T> m = set ? cross(dc, f) : dc;
+    out[0] = (double)f.x; out[1] = (double)f.y; out[2] = (double)f.z;
+    out[3] = (double)m.x; out[4] = (double)m.y; out[5] = (double)m.z;
+    out[6] = (double)(c.eq_r * T(cc.rfric) * length(Fn));
+    out[7] = (double)Ft.x; out[8] = (double)Ft.y; out[9] = (double)Ft.z;
     return set;
 }
 
-// Adds one evaluated contact to the sphere's sums: sphere_contact's accumulation, in its order.
+// Sums of a sphere's pairs: the rolling torque sum of sphere contacts is their moment sum.
+struct PairSums {
+    V3<double> F, M;
+    double R;
+};
+
+// Adds one evaluated contact (out[0..6] of sphere_pair_eval) to the sphere's sums:
+// sphere_contact's accumulation, in its order. Ft: the tangential force a pair without one of
+// its own takes over.
 template <class T>
-__device__ __forceinline__ void sphere_pair_sum(const double v[10], bool set, bool stale_ft, V3<T>& Ft, Accum& acc)
+__device__ __forceinline__ void sphere_pair_add(const double v[7], bool set, V3<T> Ft, PairSums& acc)
 {
-    if (!stale_ft) Ft = mk3(T(0), T(0), T(0));
-    if (set) Ft = mk3(T(v[3]), T(v[4]), T(v[5]));
-    const V3<T> Fn = mk3(T(v[0]), T(v[1]), T(v[2]));
-    const V3<T> dc = mk3(T(v[6]), T(v[7]), T(v[8]));
-    const V3<T> fnt = Fn + Ft;
-    acc.T = acc.T + cvt3<double>(cross(dc, fnt));
-    acc.R += v[9];
-    acc.F = acc.F + cvt3<double>(fnt);
-    acc.M = acc.M + cvt3<double>(cross(dc, fnt));
+    V3<double> f = mk3(v[0], v[1], v[2]), m = mk3(v[3], v[4], v[5]);
+    if (!set) {
+        const V3<T> fnt = mk3(T(v[0]), T(v[1]), T(v[2])) + Ft;
+        f = cvt3<double>(fnt);
+        m = cvt3<double>(cross(mk3(T(v[3]), T(v[4]), T(v[5])), fnt));
+    }
+    acc.R += v[6];
+    acc.F = acc.F + f;
+    acc.M = acc.M + m;
 }
 
 // Cohesion-only attraction of a separated pair (impl:708-718), FP64 for every precision.

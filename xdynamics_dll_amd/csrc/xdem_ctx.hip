@@ -240,7 +240,8 @@ struct xdem_ctx {
     uint32_t *work2 = nullptr, *seg_count2 = nullptr;
     uint32_t* grid_bar = nullptr;                        // k_rebuild's phase cursors and flags
     uint32_t rebuild_blocks = 0;                         // k_rebuild's grid
-    uint32_t resident_blocks = kQueueSegs;               // k_touch's and k_pairs' grid
+    uint32_t resident_blocks = kQueueSegs;               // k_touch's grid
+    uint32_t collide_blocks = kQueueSegs;                // k_collide's default grid
     unsigned long long* pass_mask = nullptr;
     // stored order: stored sphere -> the caller's global index (scene begin + caller's index)
     // and back; the same ranges per scene as the caller's
@@ -286,7 +287,6 @@ struct xdem_ctx {
     // meshes (all scenes' triangles concatenated)
     MeshDev* d_meshes = nullptr;
     double *d_vlist = nullptr, *d_plocal = nullptr, *d_prad = nullptr, *d_prox = nullptr, *msum = nullptr;
-    double* ppsum = nullptr;
     xdem_triangle_info* d_tri = nullptr;
     uint32_t *d_mcell_start = nullptr, *d_mcell_tris = nullptr;
     uint32_t *tri_count = nullptr, *tri_list = nullptr, *mesh_work = nullptr, *mesh_count = nullptr;
@@ -316,7 +316,7 @@ struct xdem_ctx {
     bool timing = false;
     std::vector<hipEvent_t> events;  // kEventsPerStep per timed step
     double t_contact = 0.0, t_grid = 0.0, t_finish = 0.0, t_pairs = 0.0, t_lite_move = 0.0, t_collide = 0.0;
-    double t_pairpass = 0.0, t_meshpass = 0.0;
+    double t_meshpass = 0.0;
     unsigned t_steps = 0;
     unsigned long long steps_done = 0;
 
@@ -364,15 +364,14 @@ struct xdem_ctx {
         A.tri_count = tri_count; A.tri_list = tri_list; A.msum = msum;
         A.ms_count = ms_count; A.ms_id = ms_id; A.ms_tsd = ms_tsd;
         A.mesh_work = mesh_work; A.mesh_count = mesh_count;
-        A.ppsum = ppsum;
         A.has_mesh = meshes.empty() ? 0 : 1;
         A.np = np; A.nsorted = np; A.cap = cap; A.nwslot = nwslot; A.nbucket = nbucket;
         A.stale_ft = cfg.quirks.stale_ft; A.flat_inertia = cfg.quirks.flat_inertia;
         A.keep_velocity = cfg.quirks.velocity_not_updated; A.tmax_persist = tmax_persist;
         A.zero_force = 1;
-        A.full_blocks = cfg.full_blocks ? std::max(cfg.full_blocks, kQueueSegs) : 1024u;
+        A.full_blocks = cfg.full_blocks ? std::max(cfg.full_blocks, kQueueSegs) : collide_blocks;
         A.resident_blocks = resident_blocks;
-        A.merge_below = cfg.merge_pairs_below ? cfg.merge_pairs_below : kMergePairsBelow;
+        A.group_max_from = cfg.merge_pairs_below ? cfg.merge_pairs_below : UINT32_MAX;
         A.has_cyl = cyls.empty() ? 0 : 1;
         return A;
     }
@@ -398,15 +397,11 @@ struct xdem_ctx {
         if (ev && (e = hipEventRecord(ev[2], stream)) != hipSuccess) return e;
         // the full pass (spheres k_touch queued) on the second stream, concurrently with the
         // lite pass (all others) on the first; the first stream waits for both: the triangle
-        // pass, the pair pass (on a small full pass it returns at once: k_collide walks the
-        // pairs; on the second stream its launch overlaps the lite pass instead of lengthening
-        // the step), the contact kernel
+        // pass, the contact kernel
         const bool gpu_law = cfg.quirks.gpu_force_law != 0;
         if ((e = hipEventRecord(fork_ev, stream)) != hipSuccess) return e;
         if ((e = hipStreamWaitEvent(stream2, fork_ev, 0)) != hipSuccess) return e;
         if (!meshes.empty() && (e = collide_fn(A, multi, fuse, model, gpu_law, 2, stream2)) != hipSuccess) return e;
-        if (ev && (e = hipEventRecord(ev[9], stream2)) != hipSuccess) return e;
-        if ((e = collide_fn(A, multi, fuse, model, gpu_law, 3, stream2)) != hipSuccess) return e;
         if (ev && (e = hipEventRecord(ev[7], stream2)) != hipSuccess) return e;
         if ((e = collide_fn(A, multi, fuse, model, gpu_law, 1, stream2)) != hipSuccess) return e;
         if (ev && (e = hipEventRecord(ev[8], stream2)) != hipSuccess) return e;
@@ -505,7 +500,7 @@ struct xdem_ctx {
     }
 };
 
-constexpr unsigned kEventsPerStep = 10;
+constexpr unsigned kEventsPerStep = 9;
 
 static int hip_status(hipError_t e) { return e == hipSuccess ? XDEM_OK : XDEM_E_HIP; }
 
@@ -759,7 +754,8 @@ int xdem_ctx_commit(xdem_ctx* c)
     {
         int cus = 0;
         CTX_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device));
-        c->resident_blocks = resident_grid(cus);
+        c->resident_blocks = resident_grid(cus, 3);
+        c->collide_blocks = resident_grid(cus, 2);
     }
     if (c->rebuild_blocks == 0) return XDEM_E_HIP;
     CTX_CHECK(c->alloc(&c->nbr, sizeof(uint32_t) * n * c->list_cap));
@@ -779,7 +775,6 @@ int xdem_ctx_commit(xdem_ctx* c)
         CTX_CHECK(c->alloc(&c->pp_id[b], sizeof(uint32_t) * n * c->cap));
         CTX_CHECK(c->alloc(&c->pp_tsd[b], sizeof(double2) * n * c->cap));
     }
-    CTX_CHECK(c->alloc(&c->ppsum, sizeof(double) * 10 * n));
     CTX_CHECK(c->alloc(&c->pl_count, sizeof(uint32_t) * n));
     CTX_CHECK(c->alloc(&c->pl_id, sizeof(uint32_t) * n * XDEM_MAX_P2PL_COUNT));
     CTX_CHECK(c->alloc(&c->pl_tsd, sizeof(double2) * n * XDEM_MAX_P2PL_COUNT));
@@ -849,7 +844,7 @@ int xdem_ctx_commit(xdem_ctx* c)
         CTX_CHECK(c->alloc(&c->mesh_count, sizeof(uint32_t)));
     }
     CTX_CHECK(c->alloc(&c->err, sizeof(uint32_t)));
-    CTX_CHECK(c->alloc(&c->counters, sizeof(unsigned long long) * 4));
+    CTX_CHECK(c->alloc(&c->counters, sizeof(unsigned long long) * kQueueSegs * kCounterStride));
 
     // host staging of the initial state (xDiscreteElementMethodSimulation.cpp:60-83)
     std::vector<double> pos(4 * n), vel(3 * n), acc(3 * n, 0.0), ep(4 * n, 0.0), mass(n), inertia(3 * n);
@@ -953,7 +948,7 @@ int xdem_ctx_commit(xdem_ctx* c)
     CTX_CHECK(hipMemsetAsync(c->pl_id, 0, sizeof(uint32_t) * n * XDEM_MAX_P2PL_COUNT, s));
     CTX_CHECK(hipMemsetAsync(c->pl_tsd, 0, sizeof(double2) * n * XDEM_MAX_P2PL_COUNT, s));
     CTX_CHECK(hipMemsetAsync(c->err, 0, sizeof(uint32_t), s));
-    CTX_CHECK(hipMemsetAsync(c->counters, 0, sizeof(unsigned long long) * 4, s));
+    CTX_CHECK(hipMemsetAsync(c->counters, 0, sizeof(unsigned long long) * kQueueSegs * kCounterStride, s));
     CTX_CHECK(hipMemsetAsync(c->n_rebuild, 0, sizeof(unsigned long long), s));
     {
         ListCtl L;
@@ -1081,7 +1076,6 @@ static int run_steps(xdem_ctx* c, unsigned nsteps)
         c->t_pairs = 0.0;
         c->t_lite_move = 0.0;
         c->t_collide = 0.0;
-        c->t_pairpass = 0.0;
         c->t_meshpass = 0.0;
         c->t_steps = std::min(nsteps, kmax);
         for (unsigned k = 0; k < c->t_steps; k++) {
@@ -1092,13 +1086,11 @@ static int run_steps(xdem_ctx* c, unsigned nsteps)
             CTX_CHECK(hipEventElapsedTime(&b, ev[2], ev[3]));
             CTX_CHECK(hipEventElapsedTime(&f, ev[3], ev[4]));
             CTX_CHECK(hipEventElapsedTime(&m, ev[5], ev[6]));
-            float kc = 0.f, kp = 0.f, km = 0.f;
+            float kc = 0.f, km = 0.f;
             CTX_CHECK(hipEventElapsedTime(&kc, ev[7], ev[8]));
-            CTX_CHECK(hipEventElapsedTime(&km, ev[2], ev[9]));
-            CTX_CHECK(hipEventElapsedTime(&kp, ev[9], ev[7]));
+            CTX_CHECK(hipEventElapsedTime(&km, ev[2], ev[7]));
             c->t_collide += kc;
             c->t_meshpass += km;
-            c->t_pairpass += kp;
             c->t_grid += a;
             c->t_pairs += p;
             c->t_contact += b;
@@ -1868,12 +1860,16 @@ int xdem_ctx_contact_count(xdem_ctx* c, unsigned long long* n_p2p, unsigned long
 {
     if (!c || !n_p2p || !n_wall) return XDEM_E_INVALID;
     if (!c->committed) return XDEM_E_NOT_READY;
-    unsigned long long h[2];
+    unsigned long long h[kQueueSegs * kCounterStride];   // the partial counts
     CTX_CHECK(hipSetDevice(c->cfg.device));
     CTX_CHECK(hipMemcpyAsync(h, c->counters, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     CTX_CHECK(hipStreamSynchronize(c->stream));
-    *n_p2p = h[0];
-    *n_wall = h[1];
+    *n_p2p = 0;
+    *n_wall = 0;
+    for (uint32_t k = 0; k < kQueueSegs; k++) {
+        *n_p2p += h[k * kCounterStride];
+        *n_wall += h[k * kCounterStride + 1];
+    }
     return XDEM_OK;
 }
 
@@ -1931,7 +1927,7 @@ int xdem_ctx_timing(xdem_ctx* c, double out[9])
     if (!c || !out) return XDEM_E_INVALID;
     out[6] = c->t_collide;
     out[7] = c->t_meshpass;
-    out[8] = c->t_pairpass;
+    out[8] = 0.0;   // the pairs are part of k_collide
     out[5] = c->t_lite_move;
     out[0] = c->t_contact;
     out[1] = c->t_grid;

@@ -88,8 +88,9 @@ __device__ __forceinline__ void st_co(uint32_t* p, uint32_t v)
 __device__ __forceinline__ void step_counters(const StepArgs& A)
 {
     if (blockIdx.x != 0) return;
-    if (threadIdx.x < 2) A.counters[threadIdx.x] = 0ull;
     if (threadIdx.x < kQueueSegs) {
+        A.counters[threadIdx.x * kCounterStride] = 0ull;
+        A.counters[threadIdx.x * kCounterStride + 1u] = 0ull;
         A.seg_count2[threadIdx.x * kSegStride] = 0u;
         A.dmax_next[threadIdx.x * kSegStride] = 0u;
     }

@@ -36,6 +36,7 @@ constexpr uint32_t kCountMask = 0x01ffffffu;
 // slower: its few thousand full-pass spheres then fell into a few segments, on few XCDs.)
 constexpr uint32_t kQueueSegs = 64;
 constexpr uint32_t kSegStride = 32;           // uint32 entries between two segment counters
+constexpr uint32_t kCounterStride = 16;       // 64-bit entries between two partial contact counts
 constexpr uint32_t kBarFlags = 64;            // release flags of k_rebuild's phases
 constexpr uint32_t kRebuildPhases = 6;        // k_rebuild: count, reduce, parts, apply, scatter, order
 constexpr uint32_t kClaimGroups = 8;          // unit ranges per phase, each with a cursor and a counter
@@ -185,13 +186,13 @@ struct StepArgs {
     uint32_t* tri_count;                     // per sphere: listed triangles (build)
     uint32_t* tri_list;                      // their indices in the mesh, kTriCap per sphere
     double* msum;                            // per sphere: triangle sums F, M, T (3 each), R
-    double* ppsum;                           // per sphere of the full pass: sphere-contact sums F, M, T, R
     uint32_t* ms_count; uint32_t* ms_id; double2* ms_tsd;   // triangle history, 5 slots (in place)
     uint32_t* mesh_work;                     // spheres with listed triangles (build), mesh_count of them
     uint32_t* mesh_count;
     int has_mesh;
     uint32_t* err;
-    unsigned long long* counters;  // [0] stored sphere contacts, [1] stored wall contacts
+    unsigned long long* counters;  // kQueueSegs partial counts, kCounterStride apart: [0] stored sphere
+                                   // contacts, [1] stored wall and cylinder contacts
     uint32_t* seg_count;           // spheres per candidate queue segment (kSegStride apart)
     uint32_t* seg_count2;          // spheres per full-pass queue segment (kSegStride apart)
     uint32_t seg_cap;              // entries per queue segment in work and work2
@@ -203,9 +204,9 @@ struct StepArgs {
     uint32_t nwslot, nbucket;
     uint32_t list_cap;                       // neighbour-list entries per sorted slot
     uint32_t full_blocks;                    // grid of the full-pass kernels (host side: launch shape)
-    uint32_t resident_blocks;                // grid of k_touch and k_pairs: the blocks the device holds
-                                             // at once at three waves per SIMD (host side)
-    uint32_t merge_below;                    // full passes smaller than this: k_collide walks the pairs
+    uint32_t resident_blocks;                // grid of k_touch: the blocks the device holds at once at
+                                             // three waves per SIMD (host side)
+    uint32_t group_max_from;                 // full passes of this size or more: 64 spheres to a wave
     int has_cyl;                             // a scene has cylinders (host side: the CYL kernels)
     int stale_ft, flat_inertia, keep_velocity, tmax_persist;
     int zero_force;  // k_finish leaves force/moment zero (the reference's state after a step)
@@ -775,37 +776,23 @@ __device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S
     }
 }
 
-// ------------------------------------------------------------------------- pair pass
-// The sphere contacts of the full pass, one thread per queued sphere: its passing pairs in
-// rank order (rank = place among the sphere's passing list entries, i.e. the reference's
-// visiting order), each looked up in the previous step's slots, evaluated
-// (sphere_pair_eval), written to its new slot (= rank, up to the capacity) and added with
-// sphere_contact's operations, so the sums are those of the reference's walk over the pairs.
-// The first kPairIdRegs slot ids of the previous step are read once into registers, and the
-// next pair's list entry is loaded while the current pair is evaluated; the neighbour's state
-// and its history entry are then one round trip. The sums go to ppsum for k_collide.
-// Cohesion-only pairs add their attraction.
-constexpr uint32_t kPairIdRegs = 16;
+// ------------------------------------------------------------------------- sphere pairs
+// A pair's place among the passing list entries of its sphere, its rank, is the reference's
+// visiting order. Each pair is looked up in the previous step's slots, evaluated
+// (sphere_pair_eval), written to its new slot (= rank, up to the capacity) and added in rank
+// order with sphere_contact's operations, so the sums are those of the reference's walk.
+// Cohesion-only pairs add their attraction. The first kPairIds slot ids of the previous step
+// are staged in LDS.
+constexpr uint32_t kPairIds = 16;
+constexpr uint32_t kGroupMin = 4;      // k_collide: the fewest spheres to a wave
 constexpr uint32_t kPairSet = 0, kPairStale = 1, kPairCoh = 2;   // kinds of an evaluated pair
-
-// The first slot of the previous step holding sphere k (kInvalid: none).
-__device__ __forceinline__ uint32_t old_slot(const StepArgs& A, uint32_t hb, const uint32_t (&ids)[kPairIdRegs],
-                                             uint32_t old_count, uint32_t k)
-{
-    uint32_t slot = kInvalid;
-#pragma unroll
-    for (int s = (int)kPairIdRegs - 1; s >= 0; s--)   // downwards: the lowest match stays
-        if ((uint32_t)s < old_count && ids[s] == k) slot = (uint32_t)s;
-    for (uint32_t s = kPairIdRegs; s < old_count && slot == kInvalid; s++)
-        if (A.pp_id_in[hb + s] == k) slot = s;
-    return slot;
-}
 
 // Sphere i's pair with neighbour k: the neighbour's state, the history entry of `slot`, the
 // force law; writes the new slot `rank` and returns the kind.
 template <class T, int MODEL, bool GPU_LAW>
-__device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S, uint32_t i, const OwnState& o,
-                                            V3<double> iom, uint32_t k, uint32_t rank, uint32_t slot, double v[10])
+__device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S, uint32_t i, V4<double> ipos,
+                                            V3<double> ivel, V3<double> iom, double imass, uint32_t k, uint32_t rank,
+                                            uint32_t slot, double v[10])
 {
     const uint32_t hb = i * A.cap;
     const V4<double> jpos = ld4(A.pos + 4 * (size_t)k);
@@ -814,17 +801,17 @@ __device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S
     const V4<double> jev = ld4(A.ev + 4 * (size_t)k);
     const double jmass = A.mass[k];
     const double2 h = slot != kInvalid ? A.pp_tsd_in[hb + slot] : make_double2(0.0, 0.0);
-    const PairGeom g = pair_geom(o.pos, jpos);
+    const PairGeom g = pair_geom(ipos, jpos);
     double sd0 = 0.0, sd1 = 0.0;
     uint32_t kind;
     if (g.cdist > 0) {
         sd0 = h.x; sd1 = h.y;
-        const bool set = sphere_pair_eval<T, MODEL, GPU_LAW>(S.cc, S.dt, o.pos, o.vel, iom, o.mass, jpos, jvel,
+        const bool set = sphere_pair_eval<T, MODEL, GPU_LAW>(S.cc, S.dt, ipos, ivel, iom, imass, jpos, jvel,
                                                              omega_of(jep, jev), jmass, g, sd0, sd1, v);
         kind = set ? kPairSet : kPairStale;
     } else {
         // cohesion only: the attraction cf * unit that sphere_cohesion subtracts
-        const double ir = o.pos.w, jr = jpos.w;
+        const double ir = ipos.w, jr = jpos.w;
         const double Req = jr ? (ir * jr) / (ir + jr) : ir;
         const double cf = cohesion_force<double>(S.cc, Req, S.cc.jk * Req);
         const V3<double> u = g.rp / g.dist;
@@ -847,60 +834,6 @@ __device__ __forceinline__ uint32_t full_queue_total(const StepArgs& A)
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
     return c;
-}
-
-// Below StepArgs::merge_below full-pass spheres (default kMergePairsBelow) k_collide walks
-// the pairs itself and k_pairs returns at once: the spheres then fit in one wave per SIMD of
-// k_collide, and the pair sums skip two dependent memory round trips (ppsum, own state).
-// Above it k_pairs (three waves per SIMD) hides the neighbour gathers of dense packs.
-constexpr uint32_t kMergePairsBelow = 65536;
-
-// Sphere i's passing pairs in rank order (the k_pairs walk): the pair sums, the new slots and
-// count, the overflow bits. Returns the stored count.
-template <class T, int MODEL, bool GPU_LAW>
-__device__ __forceinline__ uint32_t pairs_sphere(const StepArgs& A, const SceneDev& S, uint32_t i, const OwnState& o,
-                                                 V3<double> iom, uint32_t flags, Accum& pp)
-{
-    const uint32_t nlist_all = flags & kCountMask;
-    const unsigned long long m = min(nlist_all, A.list_cap) ? A.pass_mask[i] : 0ull;
-    const uint32_t old_count = min(A.pp_count_in[i], A.cap);
-    const uint32_t hb = i * A.cap;
-    // the previous step's slot ids (at most the capacity: the last sphere's slots end the array)
-    uint32_t ids[kPairIdRegs];
-    const uint32_t nid = min(A.cap, kPairIdRegs);
-    if ((A.cap & 3u) == 0u) {
-        const uint4* p4 = reinterpret_cast<const uint4*>(A.pp_id_in + hb);
-#pragma unroll
-        for (uint32_t c = 0; c < kPairIdRegs / 4u; c++) {
-            const uint4 w = 4u * c < nid ? p4[c] : make_uint4(kInvalid, kInvalid, kInvalid, kInvalid);
-            ids[4 * c] = w.x; ids[4 * c + 1] = w.y; ids[4 * c + 2] = w.z; ids[4 * c + 3] = w.w;
-        }
-    } else {
-#pragma unroll
-        for (uint32_t s = 0; s < kPairIdRegs; s++) ids[s] = s < nid ? A.pp_id_in[hb + s] : kInvalid;
-    }
-    const uint32_t* lst = A.nbr + (size_t)i * A.list_cap;
-    V3<T> Ft = mk3(T(0), T(0), T(0));
-    uint32_t rank = 0;
-    unsigned long long mm = m;
-    uint32_t k_next = mm ? lst[(uint32_t)__ffsll((long long)mm) - 1u] : 0u;
-    for (; mm; rank++) {
-        const uint32_t k = k_next;
-        mm &= mm - 1ull;
-        if (mm) k_next = lst[(uint32_t)__ffsll((long long)mm) - 1u];   // in flight during this pair
-        double v[10];
-        const uint32_t kind =
-            pair_of<T, MODEL, GPU_LAW>(A, S, i, o, iom, k, rank, old_slot(A, hb, ids, old_count, k), v);
-        if (kind == kPairCoh) pp.F = pp.F - mk3(v[0], v[1], v[2]);
-        else sphere_pair_sum<T>(v, kind == kPairSet, A.stale_ft != 0, Ft, pp);
-    }
-    const uint32_t n_new = min(rank, A.cap);
-    A.pp_count_out[i] = n_new;
-    uint32_t err = 0;
-    if (rank > A.cap) err |= XDEM_ERR_P2P_OVERFLOW;
-    if (nlist_all > A.list_cap) err |= XDEM_ERR_NBR_OVERFLOW;
-    if (err) atomicOr(A.err, err);
-    return n_new;
 }
 
 // Sphere i against the cylinders of its scene, in order: each looks up the slots as the previous
@@ -948,47 +881,22 @@ __device__ __forceinline__ uint32_t collide_cylinders(const CylDev* cyls, uint32
     return cs.count;
 }
 
-// Full contact pass of sphere i: the near neighbours the pair search listed, in their order, under
-// the exact FP64 predicate; every wall of the scene in id order; then sphere_tail. The
-// sphere's own state and outputs are read and written by id.
+// The rest of sphere i's full contact pass after its sphere pairs (their sums in pp): every wall
+// of the scene in id order, its cylinders, the triangle sums, then sphere_tail. count0: the wall
+// slot count before the step.
 template <class T, bool MULTI, bool FUSE, int MODEL, bool GPU_LAW, bool CYL>
-__device__ __forceinline__ void collide_sphere(const StepArgs& A, uint32_t i, bool merged, uint32_t& n_pp,
-                                               uint32_t& n_wall, float& dmx)
+__device__ __forceinline__ void collide_tail(const StepArgs& A, const SceneDev& S, uint32_t i, uint32_t flags,
+                                             uint32_t count0, OwnState& o, V3<double> iom, const PairSums& pp,
+                                             uint32_t& n_wall, uint32_t err, float& dmx)
 {
-    const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
-    // the sphere's own state, list flags and wall slot count, issued together (the fields
-    // of the velocity update are read just before the tail: fewer registers live across
-    // the pairs)
-    OwnState o = load_own<false>(A, S, i);
-    const uint32_t flags = A.nbr_count[i];
-    n_pp = 0;
     WallSlots ws;
-    const uint32_t count0 = S.nwall ? A.pl_count[i] : 0u;
     ws.init(count0, A.pl_id + XDEM_MAX_P2PL_COUNT * i,
             reinterpret_cast<const double*>(A.pl_tsd + XDEM_MAX_P2PL_COUNT * i));
-    const V3<double> iom = omega_of(o.ep, o.ev);
-    uint32_t err = 0;
-
-    // ---- sphere-sphere (impl:613-733): walked here when the full pass is small, else the
-    // sums of k_pairs, which ran before this kernel
-    Accum pp = {mk3(0.0, 0.0, 0.0), mk3(0.0, 0.0, 0.0), mk3(0.0, 0.0, 0.0), 0.0};
-    if (S.has_pp) {
-        if (merged) {
-            n_pp = pairs_sphere<T, MODEL, GPU_LAW>(A, S, i, o, iom, flags, pp);
-        } else {
-            const double* ps = A.ppsum + (size_t)i * 10;
-            pp.F = mk3(ps[0], ps[1], ps[2]);
-            pp.M = mk3(ps[3], ps[4], ps[5]);
-            pp.T = mk3(ps[6], ps[7], ps[8]);
-            pp.R = ps[9];
-        }
-    }
-
     // ---- walls, in id order (impl:950-1080 once per wall)
     Accum tot;
     tot.F = mk3(0.0, 0.0, 0.0) + pp.F;
     tot.M = mk3(0.0, 0.0, 0.0) + pp.M;
-    tot.T = o.t0 + pp.T;
+    tot.T = o.t0 + pp.M;
     tot.R = 0.0 + pp.R;
     if (S.nwall && !(flags & kWallNear)) {
         // no wall in reach + skin since the list build (the build's exact test): every wall's
@@ -1187,12 +1095,15 @@ __global__ __launch_bounds__(256) void k_mesh_pass(StepArgs A)
     }
 }
 
-// Pair results handed from the lane that evaluated a pair to the lane of its sphere, per wave:
-// ten values (sphere_pair_eval's out[] or the cohesion attraction) and the kind, column-major.
+// What the lanes of a wave hand each other in k_collide, column-major. own: each owner lane's
+// sphere as the pairs need it (position and radius, velocity, angular velocity, mass); v, kind:
+// a pair's ten values (sphere_pair_eval's out[] or the cohesion attraction) and kind, from the
+// lane that evaluated it to the lane of its sphere.
 struct PairStage {
+    double own[11][64];
     double v[10][64];
     uint32_t kind[64];
-    uint32_t ids[64][kPairIdRegs];   // each lane's sphere: its first slot ids of the previous step
+    uint32_t ids[64][kPairIds];   // each owner lane's sphere: its first slot ids of the previous step
 };
 
 // LDS written by some lanes of a wave and then read by others: the wave's own accesses complete
@@ -1204,157 +1115,8 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The pair pass of a large full pass. A wave takes 64 touched spheres, one per lane: when at
-// least half the sorted slots are touched (a dense pack), found in sorted-slot order, each XCD
-// sweeping one contiguous eighth of the slots, so the neighbours a block gathers were mostly
-// fetched into its XCD's L2 by the blocks of adjacent slots; otherwise from the full-pass
-// queue (block b takes segment b mod 64). It numbers their passing pairs consecutively, sphere after sphere, in rank order (an exclusive
-// scan of the pass-mask counts). The lanes then evaluate the pairs 64 at a time: entry x
-// belongs to the lane L whose range [s_L, s_L + c_L) holds it (a binary search over the
-// scanned ends), its rank is x - s_L and its list entry the rank-th set bit of L's mask; the
-// pair's history lookup, force law and new slot are pair_of's, as in pairs_sphere. Each
-// sphere's lane then adds its pairs' results in rank order from LDS with sphere_pair_sum's
-// operations, so the sums, slots and counts are those of the one-thread walk, while no lane
-// idles through the longest walk of its wave.
-template <class T, bool MULTI, int MODEL, bool GPU_LAW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pairs(StepArgs A)
-{
-    const uint32_t nfull = full_queue_total(A);
-    if (nfull < A.merge_below) return;   // k_collide walks the pairs
-    __shared__ PairStage stage_all[4];
-    PairStage& st = stage_all[threadIdx.x >> 6];
-    const uint32_t lane = threadIdx.x & 63u;
-    unsigned long long c0 = 0;
-    // the wave's spheres: sorted slots (it = virtual block) or queue entries (it = the wave's
-    // first entry); either way the loop bounds are the same for the whole wave
-    const bool sweep = 2ull * nfull >= (unsigned long long)A.nsorted;
-    const uint32_t nvb = (A.nsorted + blockDim.x - 1) / blockDim.x;
-    const QueueBlock qb = queue_block(blockIdx.x, gridDim.x);
-    const uint32_t* qseg = A.work2 + (size_t)qb.seg * A.seg_cap;
-    const uint32_t qcnt = sweep ? 0u : A.seg_count2[qb.seg * kSegStride];
-    const uint32_t it0 = sweep ? blockIdx.x : qb.chunk * blockDim.x + (threadIdx.x & ~63u);
-    const uint32_t it_end = sweep ? nvb : qcnt;
-    const uint32_t it_step = sweep ? gridDim.x : qb.nchunk * blockDim.x;
-    for (uint32_t it = it0; it < it_end; it += it_step) {
-        uint32_t i = kInvalid;
-        if (sweep) {
-            const uint32_t j = xcd_block(it, nvb) * blockDim.x + threadIdx.x;
-            if (j < A.nsorted) i = A.svals[j];
-        } else if (it + lane < qcnt) {
-            i = qseg[it + lane];
-        }
-        uint32_t flags = 0;
-        if (i < A.np) {
-            flags = A.nbr_count[i];
-            if (!(flags & kTouch) || !A.scenes[scene_index(A, i, MULTI)].has_pp) i = kInvalid;
-        } else {
-            i = kInvalid;
-        }
-        const uint32_t nlist_all = flags & kCountMask;
-        const unsigned long long m = (i != kInvalid && min(nlist_all, A.list_cap)) ? A.pass_mask[i] : 0ull;
-        const uint32_t c = (uint32_t)__popcll(m);
-        const uint32_t old_count = c ? min(A.pp_count_in[i], A.cap) : 0u;
-        if (c) {
-            const uint32_t hb = i * A.cap;
-            const uint32_t nid = min(old_count, kPairIdRegs);
-            for (uint32_t q = 0; q < nid; q++) st.ids[lane][q] = A.pp_id_in[hb + q];
-        }
-        // inclusive scan of the counts over the wave
-        uint32_t incl = c;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t t = __shfl_up(incl, off, 64);
-            if ((int)lane >= off) incl += t;
-        }
-        const uint32_t total = __shfl(incl, 63, 64);
-        const uint32_t first = incl - c;
-        Accum pp = {mk3(0.0, 0.0, 0.0), mk3(0.0, 0.0, 0.0), mk3(0.0, 0.0, 0.0), 0.0};
-        V3<T> Ft = mk3(T(0), T(0), T(0));
-        wave_lds_sync();
-        // entry x's lane L, rank r and neighbour k; the next chunk's are found (and its list
-        // entry loaded) while this chunk's pairs are evaluated
-        uint32_t L, r, k;
-        auto locate = [&](uint32_t x, uint32_t& L_, uint32_t& r_, uint32_t& k_) {
-            // the lane of entry x: the number of lanes whose range ends at or before x
-            L_ = 0;
-#pragma unroll
-            for (uint32_t w = 32; w; w >>= 1) {
-                const uint32_t e = __shfl(incl, (int)(L_ + w - 1u), 64);
-                if (e <= x) L_ += w;
-            }
-            const uint32_t iq = __shfl(i, (int)L_, 64);
-            r_ = x - __shfl(first, (int)L_, 64);
-            const uint32_t mlo = __shfl((uint32_t)m, (int)L_, 64), mhi = __shfl((uint32_t)(m >> 32), (int)L_, 64);
-            k_ = 0;
-            if (x < total) {
-                unsigned long long mm = ((unsigned long long)mhi << 32) | mlo;
-                for (uint32_t u = 0; u < r_; u++) mm &= mm - 1ull;
-                k_ = A.nbr[(size_t)iq * A.list_cap + ((uint32_t)__ffsll((long long)mm) - 1u)];
-            }
-        };
-        locate(lane, L, r, k);
-        for (uint32_t b = 0; b < total; b += 64u) {
-            const uint32_t x = b + lane;
-            uint32_t Ln = 0, rn = 0, kn = 0;
-            if (b + 64u < total) locate(x + 64u, Ln, rn, kn);
-            const uint32_t iL = __shfl(i, (int)L, 64);
-            const uint32_t ocL = __shfl(old_count, (int)L, 64);
-            if (x < total) {
-                const SceneDev& S = A.scenes[scene_index(A, iL, MULTI)];
-                OwnState o;
-                o.pos = ld4(A.pos + 4 * (size_t)iL);
-                o.vel = ld3(A.vel + 3 * (size_t)iL);
-                o.mass = A.mass[iL];
-                const V3<double> iom = omega_of(ld4(A.ep + 4 * (size_t)iL), ld4(A.ev + 4 * (size_t)iL));
-                const uint32_t hb = iL * A.cap;
-                uint32_t slot = kInvalid;
-#pragma unroll
-                for (int q = (int)kPairIdRegs - 1; q >= 0; q--)   // downwards: the lowest match stays
-                    if ((uint32_t)q < ocL && st.ids[L][q] == k) slot = (uint32_t)q;
-                for (uint32_t q = kPairIdRegs; q < ocL && slot == kInvalid; q++)
-                    if (A.pp_id_in[hb + q] == k) slot = q;
-                double v[10];
-                const uint32_t kind = pair_of<T, MODEL, GPU_LAW>(A, S, iL, o, iom, k, r, slot, v);
-#pragma unroll
-                for (int q = 0; q < 10; q++) st.v[q][lane] = v[q];
-                st.kind[lane] = kind;
-            }
-            wave_lds_sync();
-            // this lane's sphere adds its pairs of this chunk, in rank order
-            const uint32_t lo = max(first, b), hi = min(incl, b + 64u);
-            for (uint32_t y = lo; y < hi; y++) {
-                const uint32_t q = y - b;
-                double v[10];
-#pragma unroll
-                for (int z = 0; z < 10; z++) v[z] = st.v[z][q];
-                const uint32_t kind = st.kind[q];
-                if (kind == kPairCoh) pp.F = pp.F - mk3(v[0], v[1], v[2]);
-                else sphere_pair_sum<T>(v, kind == kPairSet, A.stale_ft != 0, Ft, pp);
-            }
-            wave_lds_sync();
-            L = Ln; r = rn; k = kn;
-        }
-        if (i != kInvalid) {
-            const uint32_t n_new = min(c, A.cap);
-            A.pp_count_out[i] = n_new;
-            c0 += n_new;
-            uint32_t err = 0;
-            if (c > A.cap) err |= XDEM_ERR_P2P_OVERFLOW;
-            if (nlist_all > A.list_cap) err |= XDEM_ERR_NBR_OVERFLOW;
-            if (err) atomicOr(A.err, err);
-            double* ps = A.ppsum + (size_t)i * 10;
-            st3(ps, pp.F);
-            st3(ps + 3, pp.M);
-            st3(ps + 6, pp.T);
-            ps[9] = pp.R;
-        }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) c0 += __shfl_xor(c0, off, 64);
-    if ((threadIdx.x & 63) == 0 && c0) atomicAdd(&A.counters[0], c0);
-}
-
-// Wave-wide sums of the stored-contact counts, one atomic per wave.
+// Wave-wide sums of the stored-contact counts, at most one atomic each per wave, on the wave's line
+// of the counters (adds to one address queue up at about 2 ns each).
 __device__ __forceinline__ void add_contact_counts(const StepArgs& A, unsigned long long c0, unsigned long long c1)
 {
 #pragma unroll
@@ -1363,8 +1125,9 @@ __device__ __forceinline__ void add_contact_counts(const StepArgs& A, unsigned l
         c1 += __shfl_xor(c1, off, 64);
     }
     if ((threadIdx.x & 63) == 0 && (c0 | c1)) {
-        atomicAdd(&A.counters[0], c0);
-        atomicAdd(&A.counters[1], c1);
+        unsigned long long* c = A.counters + ((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kQueueSegs - 1u)) * kCounterStride;
+        if (c0) atomicAdd(c, c0);
+        if (c1) atomicAdd(c + 1, c1);
     }
 }
 
@@ -1467,6 +1230,9 @@ __global__ __launch_bounds__(256) void k_lite_move(StepArgs A)
     lite_spheres(A, [&](uint32_t i, uint32_t skip) {
         const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
         const uint32_t flags = A.nbr_count[i];
+        // a wave of full-pass spheres only (a dense pack) ends here: the loads below would take
+        // bandwidth from the full pass
+        if (__all((flags & skip) != 0u)) return;
         const bool settled = flags & kNoContacts;
         const bool acc_kept = flags & kAccStable;
         const uint32_t count0 = (S.nwall && !settled) ? A.pl_count[i] : 0u;
@@ -1570,28 +1336,203 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
     });
 }
 
-// Full pass over the spheres k_touch queued: block b takes queue segment b mod kQueueSegs,
-// its entries chunk b / kQueueSegs, ... strided by the chunks per segment. The first entry's
-// sphere id is read together with the segment's count.
+// Full pass over the spheres k_touch queued. A wave takes G of them, one per owner lane: when at
+// least half the sorted slots are touched (a dense pack), found in sorted-slot order, each XCD
+// sweeping one contiguous eighth of the slots, so the neighbours a block gathers were mostly
+// fetched into its XCD's L2 by the blocks of adjacent slots; otherwise from the full-pass queue
+// (block b takes segment b mod 64). It numbers their passing pairs consecutively, sphere after
+// sphere, in rank order (an exclusive scan of the pass-mask counts). The lanes then evaluate the
+// pairs 64 at a time: entry x belongs to the lane L whose range [s_L, s_L + c_L) holds it (a
+// binary search over the scanned ends), its rank is x - s_L and its list entry the rank-th set
+// bit of L's mask. Each owner lane then adds its pairs' results in rank order from LDS with
+// sphere_pair_add's operations, so the sums, slots and counts are those of a one-thread walk,
+// and goes on with the walls, the velocity update and the next drift (collide_tail).
+//
+// G: as few spheres as put all of them on half the grid's waves (one per SIMD) in one round,
+// between 4 and 64. A wave issues the same instructions for a few spheres as for 64, so more
+// waves than SIMDs cost issue slots, and fewer cost rounds of pairs one after the other.
+//
+// Bound by the latency of a wave's chain (list entry, neighbour state, the FP64 divisions and
+// roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 29 us for
+// 10,000 touched spheres, 63 us for 61,000 (FP64 and DHS; a thread per sphere walking its own
+// pairs: 44 and 88 us). Beyond, two waves per SIMD wait for the neighbour gathers: 500,000
+// spheres with 3.6M pairs 263 us, half of the line requests missing L2 (a pair pass with a
+// second pass over the spheres for the rest: 172 + 110 us and 160 bytes a sphere between them).
 template <class T, bool MULTI, bool FUSE, int MODEL, bool GPU_LAW, bool CYL>
-__global__ __launch_bounds__(256) void k_collide(StepArgs A)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_collide(StepArgs A)
 {
+    __shared__ PairStage stage_all[4];
+    PairStage& st = stage_all[threadIdx.x >> 6];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t nfull = full_queue_total(A);
+    const bool sweep = 2ull * nfull >= (unsigned long long)A.nsorted;
+    // the wave's spheres: sorted slots (it = virtual block of 4 G slots) or queue entries (it =
+    // the wave's first entry); either way the loop bounds are the same for the whole wave
     const QueueBlock qb = queue_block(blockIdx.x, gridDim.x);
-    const uint32_t stride = qb.nchunk * blockDim.x;
-    const uint32_t* q = A.work2 + (size_t)qb.seg * A.seg_cap;
-    uint32_t e = qb.chunk * blockDim.x + threadIdx.x;
-    uint32_t i = e < A.seg_cap ? q[e] : 0u;
-    const uint32_t cnt = A.seg_count2[qb.seg * kSegStride];
+    const uint32_t* qseg = A.work2 + (size_t)qb.seg * A.seg_cap;
+    const uint32_t qcnt = sweep ? 0u : A.seg_count2[qb.seg * kSegStride];
+    const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;   // a multiple of 4
+    const uint32_t todo = sweep ? A.nsorted : qcnt;
+    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(kGroupMin, (2u * todo + waves - 1u) / waves));
+    const uint32_t nvb = (A.nsorted + 4u * G - 1u) / (4u * G);
+    const uint32_t it0 = sweep ? blockIdx.x : (qb.chunk * 4u + wave) * G;
+    const uint32_t it_end = sweep ? nvb : qcnt;
+    const uint32_t it_step = sweep ? gridDim.x : waves * G;
     unsigned long long c0 = 0, c1 = 0;
     float dmx = 0.0f;
-    const bool merged = full_queue_total(A) < A.merge_below;
-    while (e < cnt) {
-        uint32_t n_pp = 0, n_wall = 0;
-        collide_sphere<T, MULTI, FUSE, MODEL, GPU_LAW, CYL>(A, i, merged, n_pp, n_wall, dmx);
-        c0 += n_pp;
-        c1 += n_wall;
-        e += stride;
-        if (e < cnt) i = q[e];
+    for (uint32_t it = it0; it < it_end; it += it_step) {
+        uint32_t i = kInvalid;
+        if (lane < G) {
+            if (sweep) {
+                const uint32_t j = (xcd_block(it, nvb) * 4u + wave) * G + lane;
+                if (j < A.nsorted) i = A.svals[j];
+            } else if (it + lane < qcnt) {
+                i = qseg[it + lane];
+            }
+        }
+        uint32_t flags = 0;
+        if (i < A.np) {
+            flags = A.nbr_count[i];
+            if (!(flags & kTouch)) i = kInvalid;
+        } else {
+            i = kInvalid;
+        }
+        // what the pairs need of the sphere and its slot counts, issued together
+        const uint32_t nlist_all = flags & kCountMask;
+        unsigned long long m = 0;
+        uint32_t old_count = 0, wall_count0 = 0;
+        bool has_pp = false;
+        if (i != kInvalid) {
+            const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+            has_pp = S.has_pp != 0u;
+            if (has_pp && min(nlist_all, A.list_cap)) m = A.pass_mask[i];
+            old_count = min(A.pp_count_in[i], A.cap);
+            wall_count0 = S.nwall ? A.pl_count[i] : 0u;
+            const V4<double> p = ld4(A.pos + 4 * (size_t)i);
+            const V3<double> v = ld3(A.vel + 3 * (size_t)i);
+            const V4<double> e = ld4(A.ep + 4 * (size_t)i), d = ld4(A.ev + 4 * (size_t)i);
+            const double mass = A.mass[i];
+            const uint32_t hb = i * A.cap;
+            const uint32_t nid = m ? min(old_count, kPairIds) : 0u;
+            if ((A.cap & 3u) == 0u) {
+                const uint4* p4 = reinterpret_cast<const uint4*>(A.pp_id_in + hb);
+                for (uint32_t q = 0; q < nid; q += 4u) *reinterpret_cast<uint4*>(&st.ids[lane][q]) = p4[q / 4u];
+            } else {
+                for (uint32_t q = 0; q < nid; q++) st.ids[lane][q] = A.pp_id_in[hb + q];
+            }
+            const V3<double> w = omega_of(e, d);
+            st.own[0][lane] = p.x; st.own[1][lane] = p.y; st.own[2][lane] = p.z; st.own[3][lane] = p.w;
+            st.own[4][lane] = v.x; st.own[5][lane] = v.y; st.own[6][lane] = v.z;
+            st.own[7][lane] = w.x; st.own[8][lane] = w.y; st.own[9][lane] = w.z;
+            st.own[10][lane] = mass;
+        }
+        const uint32_t c = (uint32_t)__popcll(m);
+        // inclusive scan of the counts over the wave
+        uint32_t incl = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t t = __shfl_up(incl, off, 64);
+            if ((int)lane >= off) incl += t;
+        }
+        const uint32_t total = __shfl(incl, 63, 64);
+        const uint32_t first = incl - c;
+        PairSums pp = {mk3(0.0, 0.0, 0.0), mk3(0.0, 0.0, 0.0), 0.0};
+        V3<T> Ft = mk3(T(0), T(0), T(0));
+        wave_lds_sync();
+        // entry x's lane L, rank r and neighbour k; the next chunk's are found (and its list
+        // entry loaded) while this chunk's pairs are evaluated
+        uint32_t L, r, k;
+        auto locate = [&](uint32_t x, uint32_t& L_, uint32_t& r_, uint32_t& k_) {
+            // the lane of entry x: the number of lanes whose range ends at or before x
+            L_ = 0;
+#pragma unroll
+            for (uint32_t w = 32; w; w >>= 1) {
+                const uint32_t e = __shfl(incl, (int)(L_ + w - 1u), 64);
+                if (e <= x) L_ += w;
+            }
+            const uint32_t iq = __shfl(i, (int)L_, 64);
+            r_ = x - __shfl(first, (int)L_, 64);
+            const uint32_t mlo = __shfl((uint32_t)m, (int)L_, 64), mhi = __shfl((uint32_t)(m >> 32), (int)L_, 64);
+            k_ = 0;
+            if (x < total) {
+                unsigned long long mm = ((unsigned long long)mhi << 32) | mlo;
+                for (uint32_t u = 0; u < r_; u++) mm &= mm - 1ull;
+                k_ = A.nbr[(size_t)iq * A.list_cap + ((uint32_t)__ffsll((long long)mm) - 1u)];
+            }
+        };
+        locate(lane, L, r, k);
+        for (uint32_t b = 0; b < total; b += 64u) {
+            const uint32_t x = b + lane;
+            uint32_t Ln = 0, rn = 0, kn = 0;
+            if (b + 64u < total) locate(x + 64u, Ln, rn, kn);
+            const uint32_t iL = __shfl(i, (int)L, 64);
+            const uint32_t ocL = __shfl(old_count, (int)L, 64);
+            if (x < total) {
+                const SceneDev& S = A.scenes[scene_index(A, iL, MULTI)];
+                const V4<double> ipos = {st.own[0][L], st.own[1][L], st.own[2][L], st.own[3][L]};
+                const V3<double> ivel = mk3(st.own[4][L], st.own[5][L], st.own[6][L]);
+                const V3<double> wL = mk3(st.own[7][L], st.own[8][L], st.own[9][L]);
+                const uint32_t hb = iL * A.cap;
+                uint32_t slot = kInvalid;
+#pragma unroll
+                for (int q = (int)kPairIds - 1; q >= 0; q--)   // downwards: the lowest match stays
+                    if ((uint32_t)q < ocL && st.ids[L][q] == k) slot = (uint32_t)q;
+                for (uint32_t q = kPairIds; q < ocL && slot == kInvalid; q++)
+                    if (A.pp_id_in[hb + q] == k) slot = q;
+                double v[10];
+                const uint32_t kind =
+                    pair_of<T, MODEL, GPU_LAW>(A, S, iL, ipos, ivel, wL, st.own[10][L], k, r, slot, v);
+#pragma unroll
+                for (int q = 0; q < 10; q++) st.v[q][lane] = v[q];
+                st.kind[lane] = kind;
+            }
+            wave_lds_sync();
+            // this lane's sphere adds its pairs of this chunk, in rank order; Ft: the last
+            // tangential force set, for a pair without one of its own (quirk Q4)
+            const uint32_t lo = max(first, b), hi = min(incl, b + 64u);
+            uint32_t last = kInvalid;
+            for (uint32_t y = lo; y < hi; y++) {
+                const uint32_t q = y - b;
+                double v[7];
+#pragma unroll
+                for (int z = 0; z < 7; z++) v[z] = st.v[z][q];
+                const uint32_t kind = st.kind[q];
+                if (kind == kPairCoh) {
+                    pp.F = pp.F - mk3(v[0], v[1], v[2]);
+                    continue;
+                }
+                if (kind == kPairStale && last != kInvalid && A.stale_ft)
+                    Ft = mk3(T(st.v[7][last]), T(st.v[8][last]), T(st.v[9][last]));
+                sphere_pair_add<T>(v, kind == kPairSet, Ft, pp);
+                if (kind == kPairSet) last = q;
+            }
+            if (last != kInvalid && A.stale_ft && incl > b + 64u)   // more pairs in the next chunk
+                Ft = mk3(T(st.v[7][last]), T(st.v[8][last]), T(st.v[9][last]));
+            wave_lds_sync();
+            L = Ln; r = rn; k = kn;
+        }
+        if (i != kInvalid) {
+            const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+            uint32_t err = 0, n_wall = 0;
+            if (has_pp) {
+                const uint32_t n_new = min(c, A.cap);
+                A.pp_count_out[i] = n_new;
+                c0 += n_new;
+                if (c > A.cap) err |= XDEM_ERR_P2P_OVERFLOW;
+                if (nlist_all > A.list_cap) err |= XDEM_ERR_NBR_OVERFLOW;
+            }
+            OwnState o;
+            o.pos = {st.own[0][lane], st.own[1][lane], st.own[2][lane], st.own[3][lane]};
+            o.vel = mk3(st.own[4][lane], st.own[5][lane], st.own[6][lane]);
+            const V3<double> iom = mk3(st.own[7][lane], st.own[8][lane], st.own[9][lane]);
+            o.mass = st.own[10][lane];
+            o.ep = ld4(A.ep + 4 * (size_t)i);
+            o.ev = ld4(A.ev + 4 * (size_t)i);
+            o.t0 = A.tmax_persist ? ld3(A.tmax + 3 * (size_t)i) : mk3(0.0, 0.0, 0.0);
+            collide_tail<T, MULTI, FUSE, MODEL, GPU_LAW, CYL>(A, S, i, flags, wall_count0, o, iom, pp, n_wall, err, dmx);
+            c1 += n_wall;
+        }
     }
     add_contact_counts(A, c0, c1);
     add_disp_max(A, dmx);
@@ -1648,17 +1589,18 @@ __global__ __launch_bounds__(256) void k_finish(StepArgs A)
 }
 
 // Contact kernels of one precision (xdem_step_f64.hip / xdem_step_mixed.hip); pass 0 is the
-// lite pass, pass 1 the full pass, pass 2 the triangle pass. The other kernels are FP64 only.
+// lite pass, pass 1 the full pass, pass 2 the triangle pass before it. The other kernels are
+// FP64 only.
 using CollideLaunch = hipError_t (*)(const StepArgs&, bool multi, bool fuse, int model, bool gpu_law, int pass,
                                      hipStream_t);
 // which: 0 = k_lite_move then k_lite_turn, 1 = k_lite_move only, 2 = k_lite_turn only
 void launch_lite_fused(const StepArgs&, bool multi, hipStream_t, int which = 0);
-// Blocks of k_touch and k_pairs: as many as the device holds at once at three waves per SIMD
-// (both kernels fit three: k_pairs by its launch bounds, k_touch by its registers), one
-// round with no tail, a multiple of the queue segments.
-inline uint32_t resident_grid(int cus)
+// Blocks that the device holds at once at `waves` waves per SIMD, a multiple of the queue
+// segments: one round with no tail. k_touch fits three by its registers, k_collide two by its
+// launch bounds.
+inline uint32_t resident_grid(int cus, uint32_t waves)
 {
-    const uint32_t b = 3u * (uint32_t)(cus > 0 ? cus : 1) / kQueueSegs * kQueueSegs;
+    const uint32_t b = waves * (uint32_t)(cus > 0 ? cus : 1) / kQueueSegs * kQueueSegs;
     return b > kQueueSegs ? b : kQueueSegs;
 }
 CollideLaunch collide_launch_f64();

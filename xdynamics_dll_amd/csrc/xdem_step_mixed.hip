@@ -12,15 +12,15 @@ constexpr unsigned kBlock = 256;
 inline dim3 grid_for(unsigned n) { return dim3((n + kBlock - 1) / kBlock); }
 
 // pass 0: the lite pass over every sphere outside this step's full pass (two kernels in
-// fused mode); pass 2: the triangle pass (meshes) and pass 3: the sphere pairs, both before
-// pass 1, the rest of the full pass over the spheres k_touch queued. The full-pass kernels
-// stride over the queue segments (the queue lengths are on the device) with A.full_blocks
-// blocks, a multiple of kQueueSegs: a few blocks per CU keep several waves per SIMD for the
-// neighbour gathers. The two passes touch disjoint spheres and may run concurrently.
-inline dim3 full_grid(const StepArgs& A)
+// fused mode); pass 2: the triangle pass (meshes), before pass 1, the full pass over the
+// spheres k_touch queued. The full-pass kernels stride over the queue segments (the queue
+// lengths are on the device) with A.full_blocks blocks, a multiple of kQueueSegs. The two
+// passes touch disjoint spheres and may run concurrently.
+// per_block: the fewest spheres worth a block.
+inline dim3 full_grid(const StepArgs& A, unsigned per_block)
 {
-    const unsigned want = std::min(A.full_blocks, std::max(grid_for(A.np).x, kQueueSegs));
-    return dim3(std::max(1u, want / kQueueSegs) * kQueueSegs);
+    const unsigned blocks = (A.np + per_block - 1) / per_block;
+    return dim3((std::min(A.full_blocks, std::max(blocks, 1u)) + kQueueSegs - 1) / kQueueSegs * kQueueSegs);
 }
 
 template <bool MULTI, bool FUSE, int MODEL, bool GPU_LAW>
@@ -28,14 +28,11 @@ void collide_passes(const StepArgs& A, int pass, hipStream_t s)
 {
     const dim3 g = grid_for(A.np), b(kBlock);
     if (pass == 1) {
-        if (A.has_cyl) hipLaunchKernelGGL((k_collide<float, MULTI, FUSE, MODEL, GPU_LAW, true>), full_grid(A), b, 0, s, A);
-        else hipLaunchKernelGGL((k_collide<float, MULTI, FUSE, MODEL, GPU_LAW, false>), full_grid(A), b, 0, s, A);
-    } else if (pass == 3) {
-        // the pair pass: the resident grid (every block in one round)
-        hipLaunchKernelGGL((k_pairs<float, MULTI, MODEL, GPU_LAW>), dim3(A.resident_blocks), b, 0, s, A);
+        if (A.has_cyl) hipLaunchKernelGGL((k_collide<float, MULTI, FUSE, MODEL, GPU_LAW, true>), full_grid(A, 4 * kGroupMin), b, 0, s, A);
+        else hipLaunchKernelGGL((k_collide<float, MULTI, FUSE, MODEL, GPU_LAW, false>), full_grid(A, 4 * kGroupMin), b, 0, s, A);
     } else if (pass == 2) {
         // the triangle pass (grid-strided over the mesh queue, whose length is on the device)
-        hipLaunchKernelGGL((k_mesh_pass<float, MULTI, MODEL, GPU_LAW>), full_grid(A), b, 0, s, A);
+        hipLaunchKernelGGL((k_mesh_pass<float, MULTI, MODEL, GPU_LAW>), full_grid(A, kBlock), b, 0, s, A);
     } else if (FUSE) {
         launch_lite_fused(A, MULTI, s);
     } else {
