@@ -661,6 +661,7 @@ int xdem_ctx_add_scene(xdem_ctx* c, const xdem_scene* s, unsigned int* idx)
     D.grid.wo_x = wo[0]; D.grid.wo_y = wo[1]; D.grid.wo_z = wo[2];
     D.grid.cs = bucket_cs;
     D.ref_cs = s->cell_size;
+    D.ref_inv = 1.0 / s->cell_size;
     D.skin = skin;
     D.grid.mask_x = dims[0] - 1; D.grid.mask_y = dims[1] - 1; D.grid.mask_z = dims[2] - 1;
     D.grid.dim_x = dims[0];

@@ -407,7 +407,10 @@ __global__ __launch_bounds__(kBlock) void k_rebuild(StepArgs A, uint32_t ntile)
         if (blockIdx.x == 0 && threadIdx.x == 0) list_ctl_update(A, false);
         return;
     }
-    if (blockIdx.x == 0 && threadIdx.x < kQueueSegs) A.seg_count[threadIdx.x * kSegStride] = 0u;   // candidate queue
+    if (blockIdx.x == 0 && threadIdx.x < kQueueSegs) {   // candidate queue
+        A.seg_count[threadIdx.x * kSegStride] = 0u;
+        A.seg_count[threadIdx.x * kSegStride + 1u] = 0u;
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0 && A.has_mesh) *A.mesh_count = 0u;                      // mesh queue
     const uint32_t sp_units = (A.np + kUnit - 1) / kUnit;
     if (!run_phase(A, 0, sp_units, [&](uint32_t u) {
@@ -460,14 +463,17 @@ hipError_t launch_touch(const StepArgs& A, bool multi, hipStream_t s)
 {
     // the resident grid: a build step loops over the sorted slots, the other steps stride
     // over the candidate queue's segments
-    const dim3 g(A.resident_blocks);
+    const dim3 g(A.resident_blocks), b(kBlock);
+    const bool cyl = A.has_cyl != 0, mesh = A.has_mesh != 0;
+#define XDEM_TOUCH(M, C, T) hipLaunchKernelGGL((k_touch<M, C, T>), g, b, 0, s, A)
     if (multi) {
-        if (A.has_cyl) hipLaunchKernelGGL((k_touch<true, true>), g, dim3(kBlock), 0, s, A);
-        else hipLaunchKernelGGL((k_touch<true, false>), g, dim3(kBlock), 0, s, A);
+        if (cyl) { if (mesh) XDEM_TOUCH(true, true, true); else XDEM_TOUCH(true, true, false); }
+        else { if (mesh) XDEM_TOUCH(true, false, true); else XDEM_TOUCH(true, false, false); }
     } else {
-        if (A.has_cyl) hipLaunchKernelGGL((k_touch<false, true>), g, dim3(kBlock), 0, s, A);
-        else hipLaunchKernelGGL((k_touch<false, false>), g, dim3(kBlock), 0, s, A);
+        if (cyl) { if (mesh) XDEM_TOUCH(false, true, true); else XDEM_TOUCH(false, true, false); }
+        else { if (mesh) XDEM_TOUCH(false, false, true); else XDEM_TOUCH(false, false, false); }
     }
+#undef XDEM_TOUCH
     return hipGetLastError();
 }
 

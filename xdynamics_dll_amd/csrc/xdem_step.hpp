@@ -89,6 +89,7 @@ struct SceneDev {
                               // the lists use skin * ListCtl::scale
     double ref_cs;            // the reference's cell size (visiting order of the contacts);
                               // grid.cs, the bucket size, is larger by the skin and reach
+    double ref_inv;           // 1 / ref_cs
     int32_t mesh;             // the scene's mesh body (index into StepArgs::meshes), -1 for none
     uint32_t cyl_begin;       // the scene's cylinder bodies in StepArgs::cyls
     uint32_t ncyl;
@@ -193,7 +194,8 @@ struct StepArgs {
     uint32_t* err;
     unsigned long long* counters;  // kQueueSegs partial counts, kCounterStride apart: [0] stored sphere
                                    // contacts, [1] stored wall and cylinder contacts
-    uint32_t* seg_count;           // spheres per candidate queue segment (kSegStride apart)
+    uint32_t* seg_count;           // per candidate queue segment (kSegStride apart): its spheres, and
+                                   // the entries of their lists
     uint32_t* seg_count2;          // spheres per full-pass queue segment (kSegStride apart)
     uint32_t seg_cap;              // entries per queue segment in work and work2
     uint32_t* grid_bar;            // k_rebuild's phase cursors, done counters and release flags,
@@ -486,6 +488,15 @@ __device__ __forceinline__ OwnState load_own(const StepArgs& A, const SceneDev& 
     return o;
 }
 
+// LDS written by some lanes of a wave and then read by others: the wave's own accesses complete
+// in program order; the fences keep the compiler from moving them across this point.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------- reference visiting order
 // The reference visits the neighbours of sphere i cell by cell, z, y, x offsets -1..1 in
 // that nesting, spheres of a cell by id (impl:613-733 over the sorted cell table; the stable
@@ -505,123 +516,222 @@ __device__ __forceinline__ void ref_cell(const SceneDev& S, V4<double> p, int& c
     cz = (int)floor((p.z - S.grid.wo_z) / S.ref_cs);
 }
 
-__device__ __forceinline__ uint32_t visit_code(const SceneDev& S, int ix, int iy, int iz, V4<double> pj)
+// The same cells from products with the rounded reciprocal, which are within a few roundings of
+// the rounded quotients: away from an integer both have the same floor. False where a coordinate
+// is too near one (or not finite) to tell.
+__device__ __forceinline__ bool ref_cell_decided(const SceneDev& S, V4<double> p, int& cx, int& cy, int& cz)
 {
-    int jx, jy, jz;
-    ref_cell(S, pj, jx, jy, jz);
-    const int dx = jx - ix, dy = jy - iy, dz = jz - iz;
+    const double x = (p.x - S.grid.wo_x) * S.ref_inv, y = (p.y - S.grid.wo_y) * S.ref_inv, z = (p.z - S.grid.wo_z) * S.ref_inv;
+    const double fx = floor(x), fy = floor(y), fz = floor(z);
+    cx = (int)fx;
+    cy = (int)fy;
+    cz = (int)fz;
+    const double tol = 1e-12 * (1.0 + fmax(fmax(fabs(x), fabs(y)), fabs(z)));
+    const double lo = fmin(fmin(x - fx, y - fy), z - fz), hi = fmax(fmax(x - fx, y - fy), z - fz);
+    return lo > tol && hi < 1.0 - tol && tol < 1e-3;
+}
+
+__device__ __forceinline__ uint32_t offset_code(int dx, int dy, int dz)
+{
     if (dx < -1 || dx > 1 || dy < -1 || dy > 1 || dz < -1 || dz > 1) return kNotVisited;
     return (uint32_t)((dz + 1) * 9 + (dy + 1) * 3 + (dx + 1));
 }
 
-// Puts a neighbour list in the reference's visiting order at the current positions: codes
-// are packed above the caller's ids (the reference's ties within a cell), the list is
-// insertion-sorted in place (it is short and this thread's own), then each entry is turned
-// back into the stored sphere. k_touch does it when the pairs of a list that
-// pass are not in that order (after a build, the lists are in bucket order; later, a sphere
-// may have changed cells).
-__device__ __forceinline__ void order_list(const StepArgs& A, const SceneDev& S, uint32_t* lst, uint32_t n, int ix,
-                                           int iy, int iz)
+__device__ __forceinline__ uint32_t visit_code(const SceneDev& S, int ix, int iy, int iz, V4<double> pj)
 {
-    for (uint32_t t = 0; t < n; t++) {
-        const uint32_t k = lst[t];
-        lst[t] = (visit_code(S, ix, iy, iz, ld4(A.pos + 4 * (size_t)k)) << kIdBits) | A.ext_id[k];
-    }
-    for (uint32_t t = 1; t < n; t++) {
-        const uint32_t x = lst[t];
-        uint32_t u = t;
-        while (u > 0u && lst[u - 1u] > x) {
-            lst[u] = lst[u - 1u];
-            u--;
-        }
-        lst[u] = x;
-    }
-    for (uint32_t t = 0; t < n; t++) lst[t] = A.int_id[lst[t] & kIdMask];
+    int jx, jy, jz;
+    ref_cell(S, pj, jx, jy, jz);
+    return offset_code(jx - ix, jy - iy, jz - iz);
 }
 
 // The reference's pair predicate: overlap, or inside the JKR separation depth of a cohesive
-// pair (impl:671-718).
-__device__ __forceinline__ bool pair_passes(const ContactConst& cc, double ir, double jr, const PairGeom& g)
+// pair (impl:671-718). The depth is 3/4 pow(x, 1.0 / 3.0), x = cohesion_limit_depth's argument; its
+// cube decides but for distances within a billionth of it, and there cbrt(x) with the
+// difference of the rounded exponent to a third (-1.85e-17 ln x) is the same to an ulp, without
+// the registers of pow.
+__device__ __forceinline__ bool pair_passes(const ContactConst& cc, V4<double> pi, V4<double> pj)
 {
+    const PairGeom g = pair_geom(pi, pj);
     if (g.cdist > 0) return true;
     if (!(cc.coh_reach > 0.0 && -g.cdist < cc.coh_reach)) return false;
-    const double coh_s = cohesion_limit_depth(cc, jr ? (ir * jr) / (ir + jr) : ir);
-    return fabs(g.cdist) < fabs(coh_s);
+    const double ir = pi.w, jr = pj.w;
+    const double Req = jr ? (ir * jr) / (ir + jr) : ir;
+    const double x = (cc.pcc * Req) / cc.ee, d = fabs(g.cdist), v = d / 0.75, v3 = v * v * v;
+    if (v3 < x * (1.0 - 1e-9)) return true;
+    if (v3 > x * (1.0 + 1e-9)) return false;
+    const double t = cbrt(x);
+    return d < 0.75 * (t - t * (1.8503717077085941e-17 * (double)__logf(fmaxf((float)x, 1e-37f))));
 }
 
-// Exact test of candidate i with list flags fl: walls in reach, the listed pairs that pass
-// (in the reference's visiting order, the list re-sorted when broken), their mask. built: the
-// lists were made this step (no displacement since); dm: the largest displacement since the
-// build.
-template <bool MULTI, bool CYL>
-__device__ __forceinline__ bool touch_sphere(const StepArgs& A, uint32_t i, uint32_t fl, bool built, float dm)
+// The predicate where the squared distance decides it without a root: 1 passes, 0 does not, 2
+// undecided. cdist = (ri + rj) - |rp| > 0 exactly when ri + rj exceeds the rounded root, and the
+// root is correctly rounded, so a squared distance off (ri + rj)^2 (or off the square of the
+// largest reach) by more than a few roundings decides; anything not finite is undecided.
+__device__ __forceinline__ uint32_t pair_decided(const ContactConst& cc, V4<double> pi, V4<double> pj)
 {
-    // a sphere with listed triangles goes to the full pass every step (the triangle pass
-    // evaluates its list exactly)
-    const bool mesh_near = (fl & kMeshNear) != 0u;
-    bool touch = mesh_near;
-    // a pair can pass only once the two spheres have moved its gap together, a wall come
-    // into reach only once the sphere has moved its gap
-    const float di = built ? 0.0f : A.disp[i];
-    const bool may = mesh_near || !(A.gap[i] > (di + dm) * 1.0001f + 1e-9f);
-    const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
-    const V4<double> p = ld4(A.pos + 4 * i);
-    if (may && (fl & kWallNear)) {
-        for (uint32_t w = 0; w < S.nwall; w++) {
-            const WallDev& W = A.walls[S.wall_begin + w];
-            touch = touch || !wall_out_of_reach(W.cc, W.info, p);
-        }
-        if (CYL)
-            for (uint32_t c = 0; c < S.ncyl; c++) {
-                const CylDev& C = A.cyls[S.cyl_begin + c];
-                touch = touch || !cylinder_out_of_reach(C.cc, C.info, C.dbi, C.margin, p, 0.0);
+    const V3<double> rp = mk3(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
+    const double d2 = rp.x * rp.x + rp.y * rp.y + rp.z * rp.z;
+    const double s = pi.w + pj.w, far = s + cc.coh_reach;
+    if (!(s > 0.0)) return 2u;
+    if (d2 > far * far * (1.0 + 1e-12)) return 0u;
+    return d2 < s * s * (1.0 - 1e-12) ? 1u : 2u;
+}
+
+// A group of W lanes (1 to 16, a power of two, aligned in its wave) that tests one sphere: the lane's place in
+// it, the group's first lane, and its keys in LDS (as many as its list has).
+struct TouchGroup {
+    uint32_t W, l, g0;
+    uint32_t* keys;
+};
+
+__device__ __forceinline__ uint32_t group_bits(const TouchGroup& T, unsigned long long ballot)
+{
+    return (uint32_t)(ballot >> T.g0) & ((1u << T.W) - 1u);
+}
+
+// Exact test of sphere i (kInvalid: none) with list flags fl by the group's lanes: walls in reach,
+// the listed pairs that pass, in the reference's visiting order (the list re-sorted when
+// broken), their mask. Lane l tests entries l, l + W, ...: the group reads consecutive list
+// entries. Every lane of the wave calls it. SOLO: groups of one lane.
+template <bool MULTI, bool CYL, bool SOLO>
+__device__ __forceinline__ bool touch_sphere(const StepArgs& A, const TouchGroup& T, uint32_t i, uint32_t fl)
+{
+    bool touch = false;
+    uint32_t n = 0;
+    V4<double> p = {0.0, 0.0, 0.0, 0.0};
+    const SceneDev& S = A.scenes[i != kInvalid ? scene_index(A, i, MULTI) : 0u];
+    if (i != kInvalid) {
+        p = ld4(A.pos + 4 * (size_t)i);
+        touch = (fl & kMeshNear) != 0u;
+        if (fl & kWallNear) {
+            for (uint32_t w = 0; w < S.nwall; w++) {
+                const WallDev& W = A.walls[S.wall_begin + w];
+                touch = touch || !wall_out_of_reach(W.cc, W.info, p);
             }
+            if (CYL)
+                for (uint32_t c = 0; c < S.ncyl; c++) {
+                    const CylDev& C = A.cyls[S.cyl_begin + c];
+                    touch = touch || !cylinder_out_of_reach(C.cc, C.info, C.dbi, C.margin, p, 0.0);
+                }
+        }
+        n = min(fl & kCountMask, A.list_cap);
     }
-    const uint32_t n = may ? min(fl & kCountMask, A.list_cap) : 0u;
-    if (n) {
-        int ix, iy, iz;
-        ref_cell(S, p, ix, iy, iz);
-        uint32_t* lst = A.nbr + (size_t)i * A.list_cap;
-        uint32_t prev = 0;
-        bool have = false, ordered = true;
-        unsigned long long m = 0;
-        // four list entries at a time: their ids, then their positions, are loaded together
-        for (uint32_t t0 = 0; t0 < n; t0 += 4u) {
-            uint32_t kk[4];
-            V4<double> pp[4];
+    uint32_t* lst = A.nbr + (size_t)(n ? i : 0u) * A.list_cap;
+    int ix = 0, iy = 0, iz = 0;
+    if (n && !ref_cell_decided(S, p, ix, iy, iz)) ref_cell(S, p, ix, iy, iz);
+    unsigned long long m = 0;
+    uint32_t prev = 0;
+    bool have = false, ordered = true;
+    // four entries a lane at a time: their ids, then their positions, are loaded together
+    for (uint32_t t0 = 0; __any(t0 < n); t0 += 4u * T.W) {
+        uint32_t kk[4];
+        V4<double> pp[4];
 #pragma unroll
-            for (uint32_t u = 0; u < 4u; u++) kk[u] = t0 + u < n ? lst[t0 + u] : i;
+        for (uint32_t u = 0; u < 4u; u++) {
+            const uint32_t t = t0 + u * T.W + T.l;
+            kk[u] = t < n ? lst[t] : kInvalid;
+        }
 #pragma unroll
-            for (uint32_t u = 0; u < 4u; u++) pp[u] = ld4(A.pos + 4 * (size_t)kk[u]);
+        for (uint32_t u = 0; u < 4u; u++)
+            if (kk[u] != kInvalid) pp[u] = ld4(A.pos + 4 * (size_t)kk[u]);
+        // decided from the squared distance and the reciprocal; what is not, below
+        uint32_t pass = 0, open = 0, code[4];
 #pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            code[u] = kNotVisited;
+            if (kk[u] == kInvalid) continue;
+            const uint32_t d = pair_decided(S.cc, p, pp[u]);
+            if (d == 0u) continue;
+            int jx, jy, jz;
+            const bool cells = ref_cell_decided(S, pp[u], jx, jy, jz);
+            code[u] = offset_code(jx - ix, jy - iy, jz - iz);
+            if (d == 2u || !cells) open |= 1u << u;
+            else if (code[u] != kNotVisited) pass |= 1u << u;
+        }
+        if (__any(open != 0u)) {
+#pragma unroll 1
             for (uint32_t u = 0; u < 4u; u++) {
-                const uint32_t t = t0 + u;
-                if (t >= n) break;
-                const V4<double> pj = pp[u];
-                if (!pair_passes(S.cc, p.w, pj.w, pair_geom(p, pj))) continue;
-                const uint32_t code = visit_code(S, ix, iy, iz, pj);
-                if (code == kNotVisited) continue;
-                m |= 1ull << t;
-                const uint32_t key = (code << kIdBits) | A.ext_id[kk[u]];
+                if (!(open & (1u << u))) continue;
+                const V4<double> pj = ld4(A.pos + 4 * (size_t)lst[t0 + u * T.W + T.l]);
+                const uint32_t c = visit_code(S, ix, iy, iz, pj);
+                if (u == 0u) code[0] = c;
+                else if (u == 1u) code[1] = c;
+                else if (u == 2u) code[2] = c;
+                else code[3] = c;
+                if (c != kNotVisited && pair_passes(S.cc, p, pj)) pass |= 1u << u;
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            const uint32_t tu = t0 + u * T.W;
+            if (!__any(tu < n)) break;
+            const bool on = (pass & (1u << u)) != 0u;
+            const uint32_t key = on ? (code[u] << kIdBits) | A.ext_id[kk[u]] : 0u;
+            // the keys of the passing entries have to rise
+            if (SOLO) {
+                if (!on) continue;
+                m |= 1ull << tu;
                 if (have && key <= prev) ordered = false;
                 prev = key;
                 have = true;
+                continue;
+            }
+            const uint32_t bits = group_bits(T, __ballot(on));
+            m |= tu < n ? (unsigned long long)bits << tu : 0ull;
+            const uint32_t below = bits & ((1u << T.l) - 1u);
+            const uint32_t before = __shfl(key, (int)(T.g0 + (below ? 31u - __clz((int)below) : 0u)), 64);
+            const bool bad = on && (below ? key <= before : (have && key <= prev));
+            if (group_bits(T, __ballot(bad))) ordered = false;
+            const uint32_t top = __shfl(key, (int)(T.g0 + (bits ? 31u - __clz((int)bits) : 0u)), 64);
+            if (bits) {
+                prev = top;
+                have = true;
             }
         }
-        if (!ordered) {
-            // sort, then find the passing entries at their new places
-            order_list(A, S, lst, n, ix, iy, iz);
-            m = 0;
-            for (uint32_t t = 0; t < n; t++) {
-                const V4<double> pj = ld4(A.pos + 4 * (size_t)lst[t]);
-                if (pair_passes(S.cc, p.w, pj.w, pair_geom(p, pj)) && visit_code(S, ix, iy, iz, pj) != kNotVisited)
-                    m |= 1ull << t;
-            }
-        }
-        touch = touch || m != 0ull;
-        A.pass_mask[i] = m;
     }
-    return touch;
+    if (__any(!ordered)) {
+        // sort by rank: every entry's key to LDS, its rank the number of smaller keys (they differ:
+        // each holds another sphere's id), its sphere to that place of the list and its bit of
+        // the mask to that place of the mask
+        const uint32_t ns = ordered ? 0u : n;
+#pragma unroll 1
+        for (uint32_t t = T.l; t < ns; t += T.W) {
+            const uint32_t k = lst[t];
+            const V4<double> pj = ld4(A.pos + 4 * (size_t)k);
+            int jx, jy, jz;
+            if (!ref_cell_decided(S, pj, jx, jy, jz)) ref_cell(S, pj, jx, jy, jz);
+            T.keys[t] = (offset_code(jx - ix, jy - iy, jz - iz) << kIdBits) | A.ext_id[k];
+        }
+        wave_lds_sync();
+        unsigned long long ms = 0;
+#pragma unroll 1
+        for (uint32_t t = T.l; t < ns; t += T.W) {
+            const uint32_t key = T.keys[t];
+            uint32_t rank = 0;
+            for (uint32_t v = 0; v < ns; v++) rank += T.keys[v] < key ? 1u : 0u;
+            lst[rank] = A.int_id[key & kIdMask];
+            ms |= ((m >> t) & 1ull) << rank;
+        }
+#pragma unroll 1
+        for (uint32_t off = 1; off < T.W; off <<= 1) {
+            const uint32_t lo = __shfl_xor((uint32_t)ms, (int)off, 64), hi = __shfl_xor((uint32_t)(ms >> 32), (int)off, 64);
+            ms |= ((unsigned long long)hi << 32) | lo;
+        }
+        if (!ordered) m = ms;
+        wave_lds_sync();
+    }
+    if (n && T.l == 0u) A.pass_mask[i] = m;
+    return touch || m != 0ull;
+}
+
+// The entries of all segments of a queue: one counter per lane of a wave.
+__device__ __forceinline__ uint32_t queue_total(const uint32_t* seg_count)
+{
+    static_assert(kQueueSegs == 64, "one segment counter per lane");
+    uint32_t c = seg_count[(threadIdx.x & 63u) * kSegStride];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+    return c;
 }
 
 // Appends the lanes with `on` set to queue segment seg (one atomic per wave, by its first
@@ -640,18 +750,26 @@ __device__ __forceinline__ void queue_append(uint32_t* q, uint32_t* count, uint3
 }
 
 // Every step, the spheres of this step's full pass. On a build step (the rebuild kernel's
-// phases completed), one thread per sorted slot: the pair search for the slot's sphere
-// (pairs_slot: its list, list gap and candidate flags, the candidate queue work), then the
-// exact test of a candidate on the list it has just written. On the other steps, the
-// candidates of the last build from their queue (block b walks segment b mod kQueueSegs):
-// candidates whose gap exceeds their displacement plus the largest displacement since the
-// build cannot touch and are not tested. Touched spheres get kTouch, the pass mask, and a
-// place in the full-pass queue work2 (the segment of their candidate queue entry, so a
-// segment never holds more than seg_cap); the others are completed by the lite pass, as the
-// full pass would add only zero sums for them. The grid has a multiple of kQueueSegs
-// blocks.
-template <bool MULTI, bool CYL>
-__global__ __launch_bounds__(256) void k_touch(StepArgs A)
+// phases completed), one thread per sorted slot does the pair search for the slot's sphere
+// (pairs_slot: its list, list gap and candidate flags, the candidate queue work), then the wave
+// the exact test of its candidates on the lists it has just written. On the other steps, the
+// candidates of the last build: those of at least half the sorted slots by sweeping the slots,
+// each XCD one contiguous eighth of them (its L2 then holds the positions that its spheres'
+// lists name), fewer from their queue (block b walks segment b mod kQueueSegs); candidates whose
+// gap exceeds their displacement plus the largest displacement since the build cannot touch and
+// are not tested. Touched spheres get kTouch, the pass mask, and a place in the full-pass queue
+// work2 (the segment of their sorted slot, so a segment never holds more than seg_cap); the
+// others are completed by the lite pass, as the full pass would add only zero sums for them. The
+// grid has a multiple of kQueueSegs blocks.
+//
+// One lane per sphere sorts out by the gap; each of the rest is tested by a group of lanes. The
+// kernel waits for dependent loads (the list entries, then the positions they name), so a small
+// set of candidates takes 4 to 16 lanes a sphere, one such round trip on more waves; a large one
+// a lane a sphere. Per launch, against a lane a sphere for every set and a root for every pair:
+// 10,000 candidates with lists of 14: 27 -> 12 us, 61,000: 35 -> 23, 500,000: 109 -> 102 (the
+// build steps among them, with lists sorted by rank in LDS: 440 -> 314).
+template <bool MULTI, bool CYL, bool MESH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_touch(StepArgs A)
 {
     const bool built = *A.rebuild_cur != 0u;
     // A build always completes: a rebuild block that stops waiting (XDEM_ERR_GRID_SYNC, a
@@ -666,66 +784,122 @@ __global__ __launch_bounds__(256) void k_touch(StepArgs A)
             A.nbr_count[i] &= ~kTouch;
         return;
     }
-    if (built) {
-        // virtual blocks of 256 sorted slots, block vb on the XCD of physical block vb mod
-        // gridDim (gridDim is a multiple of 8)
-        const uint32_t nvb = (A.nsorted + blockDim.x - 1) / blockDim.x;
-        for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
-            const uint32_t j = xcd_block(vb, nvb) * blockDim.x + threadIdx.x;
-            const uint32_t i = j < A.nsorted ? A.svals[j] : kInvalid;
-            bool full = false, touch = false, mesh = false;
-            if (i < A.np) {
-                uint32_t fl = pairs_slot<MULTI>(A, j, i);
-                if (A.has_mesh) {
+    __shared__ uint32_t keys_all[4][1024];   // per wave: its groups' lists' keys, 16 a lane
+    __shared__ uint32_t test_lane[4][64];                    // per wave: the lanes of the spheres to test
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const QueueBlock qb = queue_block(blockIdx.x, gridDim.x);
+    const uint32_t* wq = A.work + (size_t)qb.seg * A.seg_cap;
+    // on a build step the candidates are not known yet: every slot
+    const uint32_t mine = built ? 0u : A.seg_count[qb.seg * kSegStride];
+    const uint32_t ncand = queue_total(A.seg_count), nlisted = queue_total(A.seg_count + 1);
+    const bool sweep = built || 2ull * ncand >= (unsigned long long)A.nsorted;
+    if (!sweep && mine == 0u) return;
+    const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;
+    const uint32_t todo = sweep ? A.nsorted : mine;
+    // lanes to a sphere: the most, 16 to 4, that put all on the waves in one round and that a list
+    // of mean length (counted by the build) keeps busy; one, and 64 spheres to a wave, where four
+    // take more than three rounds or lists are shorter than four. The same in every block that
+    // shares the division: all of them in a sweep, those of a segment otherwise.
+    const uint32_t listed = built || ncand == 0u ? 0u : nlisted / ncand;
+    uint32_t lanes_log2 = listed >= 12u ? 4u : (listed >= 6u ? 3u : 2u);
+    while (lanes_log2 > 2u && ((unsigned long long)todo << lanes_log2) > 64ull * waves) lanes_log2--;
+    const bool many = built || listed < 4u || ((unsigned long long)todo << lanes_log2) > 3ull * 64ull * waves;
+    // no sphere has moved more than dm since the build (0 on a build step); moving walls and
+    // meshes: their displacement since the build bounds the wall part of the gap the same way
+    // (taking the larger of the two keeps both bounds)
+    float dm = 0.0f;
+    if (!built) {
+        dm = __uint_as_float(A.dmax_cur[lane * kSegStride]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) dm = fmaxf(dm, __shfl_xor(dm, off, 64));
+        dm = fmaxf(dm, __double2float_ru(A.lctl->body_path - A.lctl->body_path_build));
+    }
+    // a wave takes `per` spheres: consecutive sorted slots (it = virtual block of 4 per slots, on
+    // the XCD of physical block it mod gridDim, a multiple of 8) or queue entries (it = the
+    // wave's first entry)
+    const uint32_t per = many ? 64u : 64u >> lanes_log2;
+    const uint32_t nvb = (A.nsorted + 4u * per - 1u) / (4u * per);
+    const uint32_t it0 = sweep ? blockIdx.x : (qb.chunk * 4u + wave) * per;
+    const uint32_t it_end = sweep ? nvb : mine;
+    const uint32_t it_step = sweep ? gridDim.x : waves * per;
+    for (uint32_t it = it0; it < it_end; it += it_step) {
+        uint32_t i = kInvalid, seg = qb.seg, fl = 0;
+        if (sweep) {
+            const uint32_t j0 = (xcd_block(it, nvb) * 4u + wave) * per, j = j0 + lane;
+            seg = (j0 >> 6) & (kQueueSegs - 1u);
+            if (lane < per && j < A.nsorted) i = A.svals[j];
+            if (i >= A.np) i = kInvalid;
+            if (built && i != kInvalid) {
+                fl = pairs_slot<MULTI>(A, j, i);
+                if (MESH) {
                     const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
                     if (S.mesh >= 0 && mesh_slot(A, S, i)) fl |= kMeshNear | kCandidate;
-                    mesh = (fl & kMeshNear) != 0u;
                 }
-                full = (fl & kCandidate) != 0u;
-                if (full) touch = touch_sphere<MULTI, CYL>(A, i, fl, true, 0.0f);
-                A.nbr_count[i] = touch ? (fl | kTouch) : fl;
             }
-            const uint32_t seg = (j >> 6) & (kQueueSegs - 1u);
-            queue_append(A.work, A.seg_count, seg, A.seg_cap, full, i);
-            queue_append(A.work2, A.seg_count2, seg, A.seg_cap, touch, i);
-            if (A.has_mesh) queue_append(A.mesh_work, A.mesh_count, 0u, 0u, mesh, i);
+        } else if (lane < per && it + lane < mine) {
+            i = wq[it + lane];
         }
-        return;
-    }
-    const QueueBlock qb = queue_block(blockIdx.x, gridDim.x);
-    const uint32_t seg = qb.seg;
-    const uint32_t nchunk = qb.nchunk;
-    const uint32_t* wq = A.work + (size_t)seg * A.seg_cap;
-    uint32_t base = qb.chunk * blockDim.x;
-    // the first entry is read together with the segment's count
-    uint32_t i_next = base + threadIdx.x < A.seg_cap ? wq[base + threadIdx.x] : 0u;
-    const uint32_t cnt = A.seg_count[seg * kSegStride];
-    if (base >= cnt) return;
-    // no sphere has moved more than dm since the build (0 on a build step)
-    __shared__ float dm_sh;
-    if (threadIdx.x < 64) {
-        float d = built ? 0.0f : __uint_as_float(A.dmax_cur[threadIdx.x * kSegStride]);
+        if (built) {
+            queue_append(A.work, A.seg_count, seg, A.seg_cap, (fl & kCandidate) != 0u, i);
+            uint32_t listed_sum = min(fl & kCountMask, A.list_cap);
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) d = fmaxf(d, __shfl_xor(d, off, 64));
-        if (threadIdx.x == 0) dm_sh = d;
-    }
-    __syncthreads();
-    // moving walls and meshes: their displacement since the build bounds the wall part of
-    // the gap the same way (taking the larger of the two keeps both bounds)
-    const float dm = fmaxf(dm_sh, __double2float_ru(A.lctl->body_path - A.lctl->body_path_build));
-    for (; base < cnt; base += nchunk * blockDim.x) {
-        const uint32_t e = base + threadIdx.x;
-        bool touch = false;
-        const uint32_t i = i_next;
-        if (e + nchunk * blockDim.x < cnt) i_next = wq[e + nchunk * blockDim.x];
-        if (e < cnt) {
-            const uint32_t fl = A.nbr_count[i];
-            touch = touch_sphere<MULTI, CYL>(A, i, fl, built, dm);
-            // a touched sphere's rotation, acceleration and contact counts are written by the
-            // full pass: no longer known stable
-            A.nbr_count[i] = touch ? ((fl & ~kLiteStable) | kTouch) : (fl & ~kTouch);
+            for (int off = 32; off > 0; off >>= 1) listed_sum += __shfl_xor(listed_sum, off, 64);
+            if (lane == 0u && listed_sum) atomicAdd(&A.seg_count[seg * kSegStride + 1u], listed_sum);
+            if (MESH) queue_append(A.mesh_work, A.mesh_count, 0u, 0u, (fl & kMeshNear) != 0u, i);
+            // the lanes' list and gap stores are read back by other lanes of the wave
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         }
+        // whether the sphere has to be tested: one with listed triangles goes to the full pass every
+        // step (the triangle pass evaluates its list exactly); a pair can pass only once the two
+        // spheres have moved its gap together, a wall come into reach only once the sphere has
+        // moved its gap (no displacement yet on a build step)
+        float gap = 3.0e38f, moved = 0.0f;
+        if (i < A.np) {
+            if (!built) {
+                fl = A.nbr_count[i];
+                moved = A.disp[i];
+            }
+            gap = A.gap[i];
+        }
+        const bool test = (fl & kCandidate) && ((fl & kMeshNear) || !(gap > (moved + dm) * 1.0001f + 1e-9f));
+        const unsigned long long tests = __ballot(test);
+        const uint32_t ntest = (uint32_t)__popcll(tests);
+        if (test) test_lane[wave][__popcll(tests & ((1ull << lane) - 1ull))] = lane;
+        wave_lds_sync();
+        uint32_t ws = lanes_log2;
+        if (per == 64u) {
+            // a wave of 64 spheres: a lane each, more only where the keys of its longest list need
+            // the room (1,024 keys a wave)
+            uint32_t nmax = test ? min(fl & kCountMask, A.list_cap) : 0u;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor(nmax, off, 64));
+            nmax = __builtin_amdgcn_readfirstlane(nmax);
+            ws = nmax > 32u ? 2u : (nmax > 16u ? 1u : 0u);
+        }
+        TouchGroup T;
+        T.W = 1u << ws;
+        T.l = lane & (T.W - 1u);
+        T.g0 = lane - T.l;
+        const uint32_t g = lane >> ws, groups = 64u >> ws;
+        T.keys = keys_all[wave] + 16u * T.W * g;
+        for (uint32_t r = 0; r < ntest; r += groups) {
+            const uint32_t q = r + g;
+            const int src = q < ntest ? (int)test_lane[wave][q] : 0;
+            const uint32_t fs = __shfl(fl, src, 64), is = __shfl(i, src, 64);
+            const uint32_t it_ = q < ntest ? is : kInvalid;
+            const bool t = T.W == 1u ? touch_sphere<MULTI, CYL, true>(A, T, it_, fs)
+                                     : touch_sphere<MULTI, CYL, false>(A, T, it_, fs);
+            if (T.l == 0u && q < ntest) test_lane[wave][q] = t ? 64u + (uint32_t)src : (uint32_t)src;
+        }
+        wave_lds_sync();
+        const bool touch = test && test_lane[wave][__popcll(tests & ((1ull << lane) - 1ull))] >= 64u;
+        // a touched sphere's rotation, acceleration and contact counts are written by the full
+        // pass: no longer known stable
+        const uint32_t nf = touch ? ((fl & ~kLiteStable) | kTouch) : (fl & ~kTouch);
+        if (i < A.np && (built || nf != fl)) A.nbr_count[i] = nf;
         queue_append(A.work2, A.seg_count2, seg, A.seg_cap, touch, i);
+        wave_lds_sync();   // test_lane is written again
     }
 }
 
@@ -824,16 +998,6 @@ __device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S
         A.pp_tsd_out[hb + rank] = make_double2(sd0, sd1);
     }
     return kind;
-}
-
-// The full-pass spheres of this step (all queue segments): one counter per lane of a wave.
-__device__ __forceinline__ uint32_t full_queue_total(const StepArgs& A)
-{
-    static_assert(kQueueSegs == 64, "one segment counter per lane");
-    uint32_t c = A.seg_count2[(threadIdx.x & 63u) * kSegStride];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
-    return c;
 }
 
 // Sphere i against the cylinders of its scene, in order: each looks up the slots as the previous
@@ -1106,15 +1270,6 @@ struct PairStage {
     uint32_t ids[64][kPairIds];   // each owner lane's sphere: its first slot ids of the previous step
 };
 
-// LDS written by some lanes of a wave and then read by others: the wave's own accesses complete
-// in program order; the fences keep the compiler from moving them across this point.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Wave-wide sums of the stored-contact counts, at most one atomic each per wave, on the wave's line
 // of the counters (adds to one address queue up at about 2 ns each).
 __device__ __forceinline__ void add_contact_counts(const StepArgs& A, unsigned long long c0, unsigned long long c1)
@@ -1365,7 +1520,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     PairStage& st = stage_all[threadIdx.x >> 6];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t nfull = full_queue_total(A);
+    const uint32_t nfull = queue_total(A.seg_count2);
     const bool sweep = 2ull * nfull >= (unsigned long long)A.nsorted;
     // the wave's spheres: sorted slots (it = virtual block of 4 G slots) or queue entries (it =
     // the wave's first entry); either way the loop bounds are the same for the whole wave
