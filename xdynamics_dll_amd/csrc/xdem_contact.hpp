@@ -74,39 +74,49 @@ __device__ __forceinline__ PairGeom pair_geom(V4<double> pi_, V4<double> pj)
     return g;
 }
 
-// Contact of sphere i with sphere j (cdist > 0), impl:679-706. Updates the i-side sums
-// and the pair's history (sd0, sd1). Ft carries over between calls (quirk Q4) unless
-// the caller resets it.
-template <class T, int MODEL, bool GPU_LAW>
-__device__ __forceinline__ void sphere_contact(const ContactConst& cc, double dt, V4<double> ipos, V3<double> ivel,
-                                               V3<double> iom, double im, V4<double> jpos, V3<double> jvel,
-                                               V3<double> jom, double jm, const PairGeom& g, double& sd0, double& sd1,
-                                               V3<T>& Ft, Accum& acc)
+// The reference's pair predicate: overlap, or inside the JKR separation depth of a cohesive
+// pair (impl:671-718). The depth is 3/4 pow(x, 1.0 / 3.0), x = cohesion_limit_depth's argument; its
+// cube decides but for distances within a billionth of it, and there cbrt(x) with the
+// difference of the rounded exponent to a third (-1.85e-17 ln x) is the same to an ulp, without
+// the registers of pow.
+__device__ __forceinline__ bool pair_passes(const ContactConst& cc, V4<double> pi, V4<double> pj)
 {
-    const double ir = ipos.w, jr = jpos.w;
-    const PairConst<T> c = pair_const<T, MODEL>(cc, ir, jr, im, jm);
-    const V3<double> unit = g.rp / g.dist;
-    const V3<double> ip3 = mk3(ipos.x, ipos.y, ipos.z);
-    const V3<double> cpt = ip3 + ir * unit;
-    const V3<double> dcpr = cpt - ip3;
-    const V3<double> dcpr_j = cpt - mk3(jpos.x, jpos.y, jpos.z);
-    const V3<double> rv = (jvel + cross(jom, dcpr_j)) - (ivel + cross(iom, dcpr));
-    V3<T> Fn;
-    force_law<T, MODEL, GPU_LAW>(cc, c, g.cdist, dt, sd0, sd1, rv, unit, Ft, Fn);
-    const V3<T> fnt = Fn + Ft;
-    const V3<T> dc = cvt3<T>(dcpr);
-    acc.T = acc.T + cvt3<double>(cross(dc, fnt));
-    acc.R += (double)(c.eq_r * T(cc.rfric) * length(Fn));
-    acc.F = acc.F + cvt3<double>(fnt);
-    acc.M = acc.M + cvt3<double>(cross(dc, fnt));
+    const PairGeom g = pair_geom(pi, pj);
+    if (g.cdist > 0) return true;
+    if (!(cc.coh_reach > 0.0 && -g.cdist < cc.coh_reach)) return false;
+    const double ir = pi.w, jr = pj.w;
+    const double Req = jr ? (ir * jr) / (ir + jr) : ir;
+    const double x = (cc.pcc * Req) / cc.ee, d = fabs(g.cdist), v = d / 0.75, v3 = v * v * v;
+    if (v3 < x * (1.0 - 1e-9)) return true;
+    if (v3 > x * (1.0 + 1e-9)) return false;
+    const double t = cbrt(x);
+    return d < 0.75 * (t - t * (1.8503717077085941e-17 * (double)__logf(fmaxf((float)x, 1e-37f))));
 }
 
-// One contact of sphere i with sphere j evaluated on its own: the parts of sphere_contact that do
-// not depend on the earlier pairs of the sphere. Returns whether Ft was set (|e| != 0). Set: out =
+// The predicate where the squared distance decides it without a root: 1 passes, 0 does not, 2
+// undecided. cdist = (ri + rj) - |rp| > 0 exactly when ri + rj exceeds the rounded root, and the
+// root is correctly rounded, so a squared distance off (ri + rj)^2 (or off the square of the
+// largest reach) by more than a few roundings decides; anything not finite is undecided.
+__device__ __forceinline__ uint32_t pair_decided(const ContactConst& cc, V4<double> pi, V4<double> pj)
+{
+    const V3<double> rp = mk3(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
+    const double d2 = rp.x * rp.x + rp.y * rp.y + rp.z * rp.z;
+    const double s = pi.w + pj.w, far = s + cc.coh_reach;
+    if (!(s > 0.0)) return 2u;
+    if (d2 > far * far * (1.0 + 1e-12)) return 0u;
+    return d2 < s * s * (1.0 - 1e-12) ? 1u : 2u;
+}
+
+// Kinds of an evaluated pair: Ft set, not set, cohesion only.
+constexpr uint32_t kPairSet = 0, kPairStale = 1, kPairCoh = 2;
+
+// One contact of sphere i with sphere j (cdist > 0), impl:679-706, evaluated on its own: what does
+// not depend on the earlier pairs of the sphere. Updates the pair's history (sd0, sd1). Returns
+// whether Ft was set (|e| != 0). Set: out =
 // Fn + Ft (3), its moment about the centre (3), the rolling-resistance term, Ft (3). Not set (the
 // force needs the previous pair's Ft, quirk Q4): out = Fn (3), the lever arm (3), the
 // rolling-resistance term. All in T, stored as double. sphere_pair_add then adds the pairs in
-// visiting order with sphere_contact's operations.
+// visiting order.
 template <class T, int MODEL, bool GPU_LAW>
 __device__ __forceinline__ bool sphere_pair_eval(const ContactConst& cc, double dt, V4<double> ipos, V3<double> ivel,
                                                  V3<double> iom, double im, V4<double> jpos, V3<double> jvel,
@@ -139,9 +149,9 @@ struct PairSums {
     double R;
 };
 
-// Adds one evaluated contact (out[0..6] of sphere_pair_eval) to the sphere's sums:
-// sphere_contact's accumulation, in its order. Ft: the tangential force a pair without one of
-// its own takes over.
+// Adds one evaluated contact (out[0..6] of sphere_pair_eval) to the sphere's sums, as the
+// reference's kernel accumulates. Ft: the tangential force a pair without one of its own takes
+// over.
 template <class T>
 __device__ __forceinline__ void sphere_pair_add(const double v[7], bool set, V3<T> Ft, PairSums& acc)
 {
@@ -156,14 +166,15 @@ __device__ __forceinline__ void sphere_pair_add(const double v[7], bool set, V3<
     acc.M = acc.M + m;
 }
 
-// Cohesion-only attraction of a separated pair (impl:708-718), FP64 for every precision.
-__device__ __forceinline__ void sphere_cohesion(const ContactConst& cc, double ir, double jr, const PairGeom& g, Accum& acc)
+// Cohesion-only attraction of a separated pair (impl:708-718), FP64 for every precision: the force
+// that the pair's sphere loses.
+__device__ __forceinline__ V3<double> sphere_attraction(const ContactConst& cc, double ir, double jr, const PairGeom& g)
 {
     const double Req = jr ? (ir * jr) / (ir + jr) : ir;
     const double f = cc.jk * Req;
     const double cf = cohesion_force<double>(cc, Req, f);
     const V3<double> unit = g.rp / g.dist;
-    acc.F = acc.F - cf * unit;
+    return cf * unit;
 }
 
 // -------------------------------------------------------------------------- walls

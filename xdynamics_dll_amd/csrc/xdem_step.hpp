@@ -544,39 +544,6 @@ __device__ __forceinline__ uint32_t visit_code(const SceneDev& S, int ix, int iy
     return offset_code(jx - ix, jy - iy, jz - iz);
 }
 
-// The reference's pair predicate: overlap, or inside the JKR separation depth of a cohesive
-// pair (impl:671-718). The depth is 3/4 pow(x, 1.0 / 3.0), x = cohesion_limit_depth's argument; its
-// cube decides but for distances within a billionth of it, and there cbrt(x) with the
-// difference of the rounded exponent to a third (-1.85e-17 ln x) is the same to an ulp, without
-// the registers of pow.
-__device__ __forceinline__ bool pair_passes(const ContactConst& cc, V4<double> pi, V4<double> pj)
-{
-    const PairGeom g = pair_geom(pi, pj);
-    if (g.cdist > 0) return true;
-    if (!(cc.coh_reach > 0.0 && -g.cdist < cc.coh_reach)) return false;
-    const double ir = pi.w, jr = pj.w;
-    const double Req = jr ? (ir * jr) / (ir + jr) : ir;
-    const double x = (cc.pcc * Req) / cc.ee, d = fabs(g.cdist), v = d / 0.75, v3 = v * v * v;
-    if (v3 < x * (1.0 - 1e-9)) return true;
-    if (v3 > x * (1.0 + 1e-9)) return false;
-    const double t = cbrt(x);
-    return d < 0.75 * (t - t * (1.8503717077085941e-17 * (double)__logf(fmaxf((float)x, 1e-37f))));
-}
-
-// The predicate where the squared distance decides it without a root: 1 passes, 0 does not, 2
-// undecided. cdist = (ri + rj) - |rp| > 0 exactly when ri + rj exceeds the rounded root, and the
-// root is correctly rounded, so a squared distance off (ri + rj)^2 (or off the square of the
-// largest reach) by more than a few roundings decides; anything not finite is undecided.
-__device__ __forceinline__ uint32_t pair_decided(const ContactConst& cc, V4<double> pi, V4<double> pj)
-{
-    const V3<double> rp = mk3(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
-    const double d2 = rp.x * rp.x + rp.y * rp.y + rp.z * rp.z;
-    const double s = pi.w + pj.w, far = s + cc.coh_reach;
-    if (!(s > 0.0)) return 2u;
-    if (d2 > far * far * (1.0 + 1e-12)) return 0u;
-    return d2 < s * s * (1.0 - 1e-12) ? 1u : 2u;
-}
-
 // A group of W lanes (1 to 16, a power of two, aligned in its wave) that tests one sphere: the lane's place in
 // it, the group's first lane, and its keys in LDS (as many as its list has).
 struct TouchGroup {
@@ -954,12 +921,11 @@ __device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S
 // A pair's place among the passing list entries of its sphere, its rank, is the reference's
 // visiting order. Each pair is looked up in the previous step's slots, evaluated
 // (sphere_pair_eval), written to its new slot (= rank, up to the capacity) and added in rank
-// order with sphere_contact's operations, so the sums are those of the reference's walk.
+// order, so the sums are those of the reference's walk.
 // Cohesion-only pairs add their attraction. The first kPairIds slot ids of the previous step
 // are staged in LDS.
 constexpr uint32_t kPairIds = 16;
 constexpr uint32_t kGroupMin = 4;      // k_collide: the fewest spheres to a wave
-constexpr uint32_t kPairSet = 0, kPairStale = 1, kPairCoh = 2;   // kinds of an evaluated pair
 
 // Sphere i's pair with neighbour k: the neighbour's state, the history entry of `slot`, the
 // force law; writes the new slot `rank` and returns the kind.
@@ -984,12 +950,7 @@ __device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S
                                                              omega_of(jep, jev), jmass, g, sd0, sd1, v);
         kind = set ? kPairSet : kPairStale;
     } else {
-        // cohesion only: the attraction cf * unit that sphere_cohesion subtracts
-        const double ir = ipos.w, jr = jpos.w;
-        const double Req = jr ? (ir * jr) / (ir + jr) : ir;
-        const double cf = cohesion_force<double>(S.cc, Req, S.cc.jk * Req);
-        const V3<double> u = g.rp / g.dist;
-        const V3<double> a = cf * u;
+        const V3<double> a = sphere_attraction(S.cc, ipos.w, jpos.w, g);   // cohesion only
         v[0] = a.x; v[1] = a.y; v[2] = a.z;
         kind = kPairCoh;
     }
