@@ -41,32 +41,6 @@ int scratch_address(uint32_t** out)
     return XDEM_OK;
 }
 
-constexpr unsigned kThreads = 256;
-
-__global__ __launch_bounds__(kThreads) void k_clear_cells(unsigned* cstart, unsigned* cend, size_t ncell)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < ncell) {
-        cstart[i] = 0xffffffffu;
-        cend[i] = 0u;
-    }
-}
-
-// First and one-past-last sorted position of every occupied cell (impl:317-360).
-__global__ __launch_bounds__(kThreads) void k_bounds(const unsigned* hash, const unsigned* index, unsigned* cstart,
-                                                     unsigned* cend, unsigned* sorted_index, unsigned n)
-{
-    const unsigned id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n) return;
-    const unsigned h = hash[id];
-    if (id == 0 || h != hash[id - 1]) {
-        cstart[h] = id;
-        if (id > 0) cend[hash[id - 1]] = id;
-    }
-    if (id == n - 1) cend[h] = id + 1;
-    sorted_index[id] = index[id];
-}
-
 }  // namespace
 }  // namespace xdem
 
@@ -82,24 +56,8 @@ extern "C" int xdem_cu_reorderDataAndFindCellStart_noalloc(unsigned int* hash, u
     uint32_t* s = nullptr;
     const int rc = scratch_address(&s);
     if (rc) return rc;
-    hipStream_t st = runtime().stream;
-    if (np > 0) {
-        int bits = 1;
-        while (bits < 32 && (1ull << bits) < (unsigned long long)ncell) bits++;
-        uint32_t* kout = s;
-        uint32_t* vout = s + kNoAllocMaxN;
-        uint32_t* ktmp = s + 2 * (size_t)kNoAllocMaxN;
-        uint32_t* vtmp = s + 3 * (size_t)kNoAllocMaxN;
-        uint32_t* hist = s + kSortWords;   // fully rewritten by every pass: no clearing needed
-        XDEM_HIP_CHECK(radix_sort_pairs(hash, index, kout, vout, ktmp, vtmp, np, bits, hist, st));
-        XDEM_HIP_CHECK(hipMemcpyAsync(hash, kout, sizeof(unsigned) * np, hipMemcpyDeviceToDevice, st));
-        XDEM_HIP_CHECK(hipMemcpyAsync(index, vout, sizeof(unsigned) * np, hipMemcpyDeviceToDevice, st));
-    }
-    hipLaunchKernelGGL(k_clear_cells, dim3((unsigned)((ncell + kThreads - 1) / kThreads)), dim3(kThreads), 0, st,
-                       cstart, cend, (size_t)ncell);
-    if (np > 0)
-        hipLaunchKernelGGL(k_bounds, dim3((np + kThreads - 1) / kThreads), dim3(kThreads), 0, st, hash, index, cstart,
-                           cend, sorted_index, np);
-    if (hipGetLastError() != hipSuccess) return XDEM_E_HIP;
+    uint32_t* const buf[4] = {s, s + kNoAllocMaxN, s + 2 * (size_t)kNoAllocMaxN, s + 3 * (size_t)kNoAllocMaxN};
+    // the digit counts are fully rewritten by every digit: no clearing needed
+    XDEM_HIP_CHECK(cell_sort(hash, index, sorted_index, cstart, cend, np, ncell, buf, s + kSortWords, runtime().stream));
     return XDEM_OK;
 }

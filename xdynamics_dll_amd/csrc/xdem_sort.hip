@@ -1,218 +1,321 @@
-// xdem_sort.hip -- stable LSD radix sort of (uint32 key, uint32 value) pairs for gfx950.
+// xdem_sort.hip -- stable LSD radix sort of (cell hash, index) pairs and the cell table, for gfx950.
 //
-// 8-bit digits, three kernels per digit:
-//   k_rs_hist    per-tile digit counts (LDS atomics) -> hist[digit][tile]
-//   k_rs_scan    one work-group exclusive scan of hist (digit-major, so the result is the
-//                global output offset of each (digit, tile))
-//   k_rs_scatter ranks every key of a tile among equal digits with wave64 ballots (the
-//                rank respects input order, which makes the sort stable), reorders the
-//                tile in LDS by digit, and writes runs of equal digits to global memory.
-// A tile is 256 threads x 16 keys = 4096 keys.
+// 8-bit digits over tiles of 4,096 pairs, blocks of 1,024 threads. Up to kSmall pairs one block does
+// everything in LDS (after a kernel that clears the cell table). Beyond, two kernels a digit:
+//   k_hist      per-tile digit counts (LDS atomics) -> hist[tile][digit]; the first digit's launch
+//               has further blocks that clear the cell table meanwhile
+//   k_scatter   adds up the counts of the earlier tiles and of all tiles itself (no scan kernel
+//               between: a block reads the whole table, 1 KB a tile, coalesced and from L2), ranks
+//               its pairs among equal digits, reorders the tile in LDS by digit and writes runs of
+//               equal digits
+// and k_bounds, the first and one-past-last position of every occupied cell. A wave ranks its own 64
+// pairs at a time with wave64 ballots against counters of its own, so the block synchronises only
+// once for all of them; ranks respect input order, which makes the sort stable.
+//
+// Bound by latency: the kernels of a call take 84 -> 48 us for 120,000 pairs and 21 key bits and 131 ->
+// 64 us for 1,048,575
+// (three kernels a digit, one of them a scan by one work-group, and separate copies and fills).
 #include "xdem_sort.hpp"
 
 namespace xdem {
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kItems = 16;
-constexpr int kTile = kBlock * kItems;
-constexpr int kWaves = kBlock / 64;
+constexpr uint32_t kThreads = 1024;
+constexpr uint32_t kWaves = kThreads / 64;
+constexpr uint32_t kItems = 4;
+constexpr uint32_t kTile = kThreads * kItems;
+constexpr uint32_t kSmall = kThreads * 8;   // pairs that one block sorts, 2, 4 or 8 a thread
+constexpr uint32_t kNone = 0xffffffffu;
 
-__global__ __launch_bounds__(kBlock) void k_rs_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
-                                                   uint32_t* __restrict__ hist, uint32_t ntiles)
+// Both cell tables from entry b * kThreads on, four entries a thread and step, by nb blocks.
+__device__ __forceinline__ void clear_cells(uint32_t* cstart, uint32_t* cend, uint32_t ncell, uint32_t b, uint32_t nb)
 {
+    for (size_t i = (size_t)b * kThreads + threadIdx.x; i < ncell; i += (size_t)nb * kThreads) {
+        cstart[i] = kNone;
+        cend[i] = 0u;
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void k_clear(uint32_t* cstart, uint32_t* cend, uint32_t ncell)
+{
+    clear_cells(cstart, cend, ncell, blockIdx.x, gridDim.x);
+}
+
+__global__ __launch_bounds__(kThreads) void k_hist(const uint32_t* __restrict__ keys, uint32_t n, uint32_t shift,
+                                                   uint32_t* __restrict__ hist, uint32_t ntiles, uint32_t* cstart,
+                                                   uint32_t* cend, uint32_t ncell)
+{
+    if (blockIdx.x >= ntiles) {
+        clear_cells(cstart, cend, ncell, blockIdx.x - ntiles, gridDim.x - ntiles);
+        return;
+    }
     __shared__ uint32_t cnt[256];
-    const uint32_t tid = threadIdx.x;
-    cnt[tid] = 0;
+    if (threadIdx.x < 256u) cnt[threadIdx.x] = 0u;
     __syncthreads();
-    const uint32_t base = blockIdx.x * kTile;
+    const uint32_t base = blockIdx.x * kTile + threadIdx.x;
 #pragma unroll
-    for (int s = 0; s < kItems; s++) {
-        const uint32_t idx = base + s * kBlock + tid;
+    for (uint32_t s = 0; s < kItems; s++) {
+        const uint32_t idx = base + s * kThreads;
         if (idx < n) atomicAdd(&cnt[(keys[idx] >> shift) & 255u], 1u);
     }
     __syncthreads();
-    hist[tid * ntiles + blockIdx.x] = cnt[tid];
+    if (threadIdx.x < 256u) hist[blockIdx.x * 256u + threadIdx.x] = cnt[threadIdx.x];
 }
 
-// Exclusive scan of `total` entries (a multiple of 4) by one work-group of 1024 threads.
-__global__ __launch_bounds__(1024) void k_rs_scan(uint32_t* __restrict__ data, uint32_t total)
+// Exclusive scan of one value per thread over threads 0..255 (4 waves); every thread of the block
+// calls it, threads past 255 get nothing of use.
+__device__ __forceinline__ uint32_t scan256(uint32_t v, uint32_t* wsum)
 {
-    __shared__ uint32_t s_wsum[16];
-    __shared__ uint32_t s_carry;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    if (tid == 0) s_carry = 0;
-    __syncthreads();
-    for (uint32_t base = 0; base < total; base += 4096u) {
-        const uint32_t idx = base + tid * 4u;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (idx < total) v = *reinterpret_cast<const uint4*>(data + idx);
-        const uint32_t t0 = v.x, t1 = t0 + v.y, t2 = t1 + v.z, t3 = t2 + v.w;
-        uint32_t x = t3;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    uint32_t x = v;
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(x, off, 64);
-            if (lane >= (uint32_t)off) x += y;
-        }
-        if (lane == 63) s_wsum[w] = x;
-        __syncthreads();
-        if (w == 0) {
-            uint32_t s = lane < 16 ? s_wsum[lane] : 0u;
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) {
-                const uint32_t y = __shfl_up(s, off, 64);
-                if (lane >= (uint32_t)off) s += y;
-            }
-            if (lane < 16) s_wsum[lane] = s;
-        }
-        __syncthreads();
-        const uint32_t pre = s_carry + (w > 0 ? s_wsum[w - 1] : 0u) + (x - t3);
-        if (idx < total) *reinterpret_cast<uint4*>(data + idx) = make_uint4(pre, pre + t0, pre + t1, pre + t2);
-        __syncthreads();
-        if (tid == 0) s_carry += s_wsum[15];
-        __syncthreads();
+    for (uint32_t off = 1; off < 64u; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
     }
+    if (lane == 63u && w < 4u) wsum[w] = x;
+    __syncthreads();
+    uint32_t pre = 0;
+    for (uint32_t q = 0; q < 4u && q < w; q++) pre += wsum[q];
+    __syncthreads();
+    return pre + x - v;
 }
 
-__global__ __launch_bounds__(kBlock) void k_rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                      uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                      uint32_t n, int shift, const uint32_t* __restrict__ offsets,
-                                                      uint32_t ntiles)
+// The tile's ranking. Item s of a thread is pair wave * 64 ITEMS + s * 64 + lane of the tile; items
+// past the tile's end come last and count as digit 255, after every pair. place[s]: the item's
+// position in the tile sorted by digit; start[d]: the first position of digit d.
+template <uint32_t ITEMS>
+__device__ __forceinline__ void rank_tile(const uint32_t (&digit)[ITEMS], uint32_t (&place)[ITEMS], uint32_t (*cnt)[256],
+                                          uint32_t* start, uint32_t* wsum)
 {
-    __shared__ uint32_t s_keys[kTile];
-    __shared__ uint32_t s_vals[kTile];
-    __shared__ uint32_t s_cnt[2][kWaves][256];
-    __shared__ uint32_t s_run[256];
-    __shared__ uint32_t s_start[256];
-    __shared__ uint32_t s_gbase[256];
-
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
-    const uint32_t base = blockIdx.x * kTile;
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
-
-    s_run[tid] = 0;
-    for (int b = 0; b < 2; b++)
-        for (int q = 0; q < kWaves; q++) s_cnt[b][q][tid] = 0;
-    s_gbase[tid] = offsets[tid * ntiles + blockIdx.x];
-
-    uint32_t key[kItems], val[kItems], rank[kItems];
+    const uint64_t lt = lane == 0u ? 0ull : (~0ull >> (64u - lane));
+    for (uint32_t q = lane; q < 256u; q += 64u) cnt[w][q] = 0u;
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int s = 0; s < kItems; s++) {
-        const uint32_t idx = base + s * kBlock + tid;
-        key[s] = idx < n ? kin[idx] : 0xffffffffu;
-        val[s] = idx < n ? vin[idx] : 0u;
-    }
-    __syncthreads();
-
+    for (uint32_t s = 0; s < ITEMS; s++) {
+        const uint32_t d = digit[s];
+        uint64_t peers = ~0ull;   // lanes of this wave holding the same digit
 #pragma unroll
-    for (int s = 0; s < kItems; s++) {
-        const uint32_t buf = s & 1;
-        const uint32_t idx = base + s * kBlock + tid;
-        const uint32_t d = idx < n ? ((key[s] >> shift) & 255u) : 255u;
-        // lanes of this wave holding the same digit
-        uint64_t peers = ~0ull;
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
+        for (uint32_t b = 0; b < 8u; b++) {
             const bool bit = (d >> b) & 1u;
             const uint64_t m = __ballot(bit);
             peers &= bit ? m : ~m;
         }
-        const uint32_t before = (uint32_t)__popcll(peers & lt_mask);
-        if (before == 0) s_cnt[buf][w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        {
-            // thread `tid` owns digit `tid`: wave counts -> exclusive bases; clear the other buffer
-            uint32_t run = s_run[tid];
-#pragma unroll
-            for (int q = 0; q < kWaves; q++) {
-                const uint32_t c = s_cnt[buf][q][tid];
-                s_cnt[buf][q][tid] = run;
-                run += c;
-            }
-            s_run[tid] = run;
-#pragma unroll
-            for (int q = 0; q < kWaves; q++) s_cnt[buf ^ 1u][q][tid] = 0;
-        }
-        __syncthreads();
-        rank[s] = s_cnt[buf][w][d] + before;
+        const uint32_t before = (uint32_t)__popcll(peers & lt);
+        const uint32_t c = cnt[w][d];
+        place[s] = c + before;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (before == 0u) cnt[w][d] = c + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
+    uint32_t total = 0;
+    if (tid < 256u) {
+#pragma unroll
+        for (uint32_t q = 0; q < kWaves; q++) {
+            const uint32_t c = cnt[q][tid];
+            cnt[q][tid] = total;
+            total += c;
+        }
+    }
+    const uint32_t first = scan256(total, wsum);
+    if (tid < 256u) start[tid] = first;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t s = 0; s < ITEMS; s++) place[s] += start[digit[s]] + cnt[w][digit[s]];
+}
 
-    // exclusive scan of the tile's digit counts (s_run) -> s_start
+__global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                      uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
+                                                      uint32_t* __restrict__ vout2, uint32_t n, uint32_t shift,
+                                                      const uint32_t* __restrict__ hist, uint32_t ntiles)
+{
+    __shared__ uint32_t s_keys[kTile], s_vals[kTile];
+    __shared__ uint32_t s_cnt[kWaves][256];
+    __shared__ uint32_t s_start[256], s_gbase[256], s_wsum[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const uint32_t base = blockIdx.x * kTile;
+    uint32_t key[kItems], val[kItems], digit[kItems], place[kItems];
+#pragma unroll
+    for (uint32_t s = 0; s < kItems; s++) {
+        const uint32_t idx = base + (w * kItems + s) * 64u + lane;
+        key[s] = idx < n ? kin[idx] : 0u;
+        val[s] = idx < n ? vin[idx] : 0u;
+        digit[s] = idx < n ? (key[s] >> shift) & 255u : 255u;
+    }
+    // digit d of this tile goes after all smaller digits and after digit d of the earlier tiles:
+    // a quarter of the block adds up a quarter of the tiles' counts
     {
-        const uint32_t c = s_run[tid];
-        uint32_t x = c;
+        const uint32_t d = tid & 255u, g = tid >> 8, per = (ntiles + 3u) / 4u;
+        const uint32_t lo = min(ntiles, g * per), hi = min(ntiles, lo + per);
+        uint32_t pre = 0, all = 0, t = lo;
+        for (; t + 8u <= hi; t += 8u) {
+            uint32_t c[8];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = __shfl_up(x, off, 64);
-            if (lane >= (uint32_t)off) x += y;
+            for (uint32_t u = 0; u < 8u; u++) c[u] = hist[(t + u) * 256u + d];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; u++) {
+                all += c[u];
+                pre += t + u < blockIdx.x ? c[u] : 0u;
+            }
         }
-        __shared__ uint32_t s_wtot[kWaves];
-        if (lane == 63) s_wtot[w] = x;
+        for (; t < hi; t++) {
+            const uint32_t c = hist[t * 256u + d];
+            all += c;
+            pre += t < blockIdx.x ? c : 0u;
+        }
+        s_keys[tid] = pre;
+        s_vals[tid] = all;
         __syncthreads();
-        uint32_t pre = 0;
-        for (uint32_t q = 0; q < w; q++) pre += s_wtot[q];
-        s_start[tid] = pre + x - c;
+        pre = all = 0;
+        if (tid < 256u)
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; q++) {
+                pre += s_keys[q * 256u + tid];
+                all += s_vals[q * 256u + tid];
+            }
+        const uint32_t first = scan256(all, s_wsum);
+        if (tid < 256u) s_gbase[tid] = first + pre;
+    }
+    rank_tile<kItems>(digit, place, s_cnt, s_start, s_wsum);
+#pragma unroll
+    for (uint32_t s = 0; s < kItems; s++) {
+        s_keys[place[s]] = key[s];
+        s_vals[place[s]] = val[s];
     }
     __syncthreads();
-
+    const uint32_t valid = min(n - base, kTile);
 #pragma unroll
-    for (int s = 0; s < kItems; s++) {
-        const uint32_t idx = base + s * kBlock + tid;
-        const uint32_t d = idx < n ? ((key[s] >> shift) & 255u) : 255u;
-        const uint32_t p = s_start[d] + rank[s];
-        s_keys[p] = key[s];
-        s_vals[p] = val[s];
-    }
-    __syncthreads();
-
-    const uint32_t valid = n - base < (uint32_t)kTile ? n - base : (uint32_t)kTile;
-#pragma unroll
-    for (int s = 0; s < kItems; s++) {
-        const uint32_t p = s * kBlock + tid;
+    for (uint32_t s = 0; s < kItems; s++) {
+        const uint32_t p = s * kThreads + tid;
         if (p < valid) {
-            const uint32_t k = s_keys[p];
-            const uint32_t d = (k >> shift) & 255u;
+            const uint32_t k = s_keys[p], v = s_vals[p], d = (k >> shift) & 255u;
             const uint32_t o = s_gbase[d] + (p - s_start[d]);
             kout[o] = k;
-            vout[o] = s_vals[p];
+            vout[o] = v;
+            if (vout2) vout2[o] = v;
         }
+    }
+}
+
+// Cell bounds (impl:317-360) of n sorted hashes; with kcopy, also the copies of a single digit's sort
+// (whose source is the caller's arrays).
+__global__ __launch_bounds__(256) void k_bounds(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
+                                                uint32_t* kcopy, uint32_t* vcopy, uint32_t* sorted_index,
+                                                uint32_t* cstart, uint32_t* cend, uint32_t n)
+{
+    const uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= n) return;
+    const uint32_t h = keys[id], prev = id ? keys[id - 1u] : 0u;
+    if (kcopy) {
+        const uint32_t v = vals[id];
+        kcopy[id] = h;
+        vcopy[id] = v;
+        sorted_index[id] = v;
+    }
+    if (id == 0u || h != prev) {
+        cstart[h] = id;
+        if (id) cend[prev] = id;
+    }
+    if (id == n - 1u) cend[h] = id + 1u;
+}
+
+// All digits of up to kThreads * ITEMS pairs, the copies and the cell bounds, by one block.
+template <uint32_t ITEMS>
+__global__ __launch_bounds__(kThreads) void k_sort_small(uint32_t* hash, uint32_t* index, uint32_t* sorted_index,
+                                                         uint32_t* cstart, uint32_t* cend, uint32_t n, uint32_t npass)
+{
+    __shared__ uint32_t s_keys[kThreads * ITEMS], s_vals[kThreads * ITEMS];
+    __shared__ uint32_t s_cnt[kWaves][256];
+    __shared__ uint32_t s_start[256], s_wsum[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    uint32_t key[ITEMS], val[ITEMS], digit[ITEMS], place[ITEMS];
+#pragma unroll
+    for (uint32_t s = 0; s < ITEMS; s++) {
+        const uint32_t idx = (w * ITEMS + s) * 64u + lane;
+        key[s] = idx < n ? hash[idx] : 0u;
+        val[s] = idx < n ? index[idx] : 0u;
+    }
+    for (uint32_t p = 0; p < npass; p++) {
+#pragma unroll
+        for (uint32_t s = 0; s < ITEMS; s++) {
+            const uint32_t idx = (w * ITEMS + s) * 64u + lane;
+            if (p) {
+                key[s] = s_keys[idx];
+                val[s] = s_vals[idx];
+            }
+            digit[s] = idx < n ? (key[s] >> (8u * p)) & 255u : 255u;
+        }
+        __syncthreads();
+        rank_tile<ITEMS>(digit, place, s_cnt, s_start, s_wsum);
+#pragma unroll
+        for (uint32_t s = 0; s < ITEMS; s++) {
+            s_keys[place[s]] = key[s];
+            s_vals[place[s]] = val[s];
+        }
+        __syncthreads();
+    }
+    for (uint32_t p = tid; p < n; p += kThreads) {
+        const uint32_t h = s_keys[p], v = s_vals[p];
+        hash[p] = h;
+        index[p] = v;
+        sorted_index[p] = v;
+        const uint32_t prev = p ? s_keys[p - 1u] : 0u;
+        if (p == 0u || h != prev) {
+            cstart[h] = p;
+            if (p) cend[prev] = p;
+        }
+        if (p == n - 1u) cend[h] = p + 1u;
     }
 }
 
 }  // namespace
 
-size_t radix_sort_scratch_bytes(uint32_t n)
+size_t cell_sort_scratch_bytes(uint32_t n)
 {
     const size_t ntiles = (n + kTile - 1) / kTile;
     return sizeof(uint32_t) * 256 * (ntiles ? ntiles : 1);
 }
 
-hipError_t radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
-                            uint32_t* vals_out, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t n,
-                            int bits, void* scratch, hipStream_t stream)
+hipError_t cell_sort(uint32_t* hash, uint32_t* index, uint32_t* sorted_index, uint32_t* cstart, uint32_t* cend, uint32_t n,
+                     uint32_t ncell, uint32_t* const buf[4], void* scratch, hipStream_t stream)
 {
-    if (n == 0) return hipSuccess;
-    if (bits < 1) bits = 1;
-    if (bits > 32) bits = 32;
-    const int npass = (bits + 7) / 8;
-    const uint32_t ntiles = (n + kTile - 1) / kTile;
+    uint32_t bits = 1;
+    while (bits < 32u && (1ull << bits) < (unsigned long long)ncell) bits++;
+    const uint32_t npass = (bits + 7u) / 8u;
+    const uint32_t clear_blocks = std::min(512u, (ncell + kThreads - 1u) / kThreads);
+    if (n <= kSmall) {
+        hipLaunchKernelGGL(k_clear, dim3(clear_blocks), dim3(kThreads), 0, stream, cstart, cend, ncell);
+        if (n > 4u * kThreads)
+            hipLaunchKernelGGL(k_sort_small<8>, dim3(1), dim3(kThreads), 0, stream, hash, index, sorted_index, cstart, cend, n, npass);
+        else if (n > 2u * kThreads)
+            hipLaunchKernelGGL(k_sort_small<4>, dim3(1), dim3(kThreads), 0, stream, hash, index, sorted_index, cstart, cend, n, npass);
+        else if (n)
+            hipLaunchKernelGGL(k_sort_small<2>, dim3(1), dim3(kThreads), 0, stream, hash, index, sorted_index, cstart, cend, n, npass);
+        return hipGetLastError();
+    }
+    const uint32_t ntiles = (n + kTile - 1u) / kTile;
     uint32_t* hist = static_cast<uint32_t*>(scratch);
-    const uint32_t* ksrc = keys_in;
-    const uint32_t* vsrc = vals_in;
-    for (int p = 0; p < npass; p++) {
-        // the last pass must land in *_out
-        const bool to_out = ((npass - 1 - p) % 2) == 0;
-        uint32_t* kdst = to_out ? keys_out : keys_tmp;
-        uint32_t* vdst = to_out ? vals_out : vals_tmp;
-        const int shift = 8 * p;
-        hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kBlock), 0, stream, ksrc, n, shift, hist, ntiles);
-        hipLaunchKernelGGL(k_rs_scan, dim3(1), dim3(1024), 0, stream, hist, 256u * ntiles);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kBlock), 0, stream, ksrc, vsrc, kdst, vdst, n, shift,
-                           hist, ntiles);
+    const uint32_t *ksrc = hash, *vsrc = index;
+    for (uint32_t p = 0; p < npass; p++) {
+        // the last digit goes to the caller's arrays, unless they are its source
+        const bool out = p + 1u == npass && npass > 1u;
+        uint32_t* kdst = out ? hash : buf[2u * (p & 1u)];
+        uint32_t* vdst = out ? index : buf[2u * (p & 1u) + 1u];
+        const uint32_t extra = p == 0u ? clear_blocks : 0u;
+        hipLaunchKernelGGL(k_hist, dim3(ntiles + extra), dim3(kThreads), 0, stream, ksrc, n, 8u * p, hist, ntiles, cstart,
+                           cend, ncell);
+        hipLaunchKernelGGL(k_scatter, dim3(ntiles), dim3(kThreads), 0, stream, ksrc, vsrc, kdst, vdst,
+                           out ? sorted_index : nullptr, n, 8u * p, hist, ntiles);
         ksrc = kdst;
         vsrc = vdst;
     }
+    const bool copy = npass == 1u;
+    hipLaunchKernelGGL(k_bounds, dim3((n + 255u) / 256u), dim3(256), 0, stream, ksrc, vsrc, copy ? hash : nullptr,
+                       copy ? index : nullptr, sorted_index, cstart, cend, n);
     return hipGetLastError();
 }
 
