@@ -276,11 +276,11 @@ struct P2pStage {
 // A wave takes G particles, one per owner lane, and walks the cells of two at a time, a candidate a
 // lane in the reference's visiting order. What passes the predicate goes to a queue, which is
 // evaluated 64 pairs at a time (sphere_pair_eval); the owners add their pairs' results in visiting
-// order, so sums, slots and counts are those of one thread walking
-// the cells. Bound by dependent loads (cell, sorted index, position, then the pair's state) on few
-// waves for small sets and by instructions for large ones: 120,000 particles in a close packing
-// 260 -> XX us, 20,000 in cells of 3.3 mm (160 candidates each) 587 -> XX us against a thread per
-// particle with its slots in scratch.
+// order, so sums, slots and counts are those of one thread walking the cells. Bound by dependent
+// loads (cell, sorted index, position, then the pair's state) on few waves for small sets, by
+// gathers that miss L2 for large ones listed in random order: 120,000 particles in a close
+// packing 260 -> 154 us, 20,000 in cells of 3.3 mm (160 candidates each) 587 -> 87 us against a
+// thread per particle with its slots in scratch.
 template <int MODEL, bool GPU_LAW, bool STALE>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_p2p(LaunchPrm P, const double* __restrict__ pos, const double* __restrict__ ep,
                                                      const double* __restrict__ vel, const double* __restrict__ ev,
