@@ -69,6 +69,7 @@ struct CalArgs {
     uint32_t* tape_code;             // [n * kTape] or null
     uint16_t* tape_slot;
     uint8_t* tape_n;
+    double* sums;                    // [10n] recorded contact sums F, M, T, R, or null
     uint32_t* err;
 };
 
@@ -100,7 +101,6 @@ template <int N> __host__ __device__ inline V4<Dual<N>> seed4(V4<double> v, int 
     return {Dual<N>::input(v.x, k0), Dual<N>::input(v.y, k0 + 1), Dual<N>::input(v.z, k0 + 2),
             Dual<N>::input(v.w, k0 + 3)};
 }
-template <int N> __host__ __device__ inline V3<Dual<N>> const3(V3<double> v) { return {Dual<N>(v.x), Dual<N>(v.y), Dual<N>(v.z)}; }
 
 // cotangent accumulation: out[k] += bar * d/dk of the dual y
 template <int N> __host__ __device__ inline void vjp_add(double (&out)[N], const Dual<N>& y, double bar)
@@ -113,13 +113,6 @@ template <int N> __host__ __device__ inline void vjp_add3(double (&out)[N], cons
     vjp_add(out, y.x, bar.x);
     vjp_add(out, y.y, bar.y);
     vjp_add(out, y.z, bar.z);
-}
-
-__device__ inline void atomic_add3(double* p, double a, double b, double c)
-{
-    if (a != 0.0) atomicAdd(p, a);
-    if (b != 0.0) atomicAdd(p + 1, b);
-    if (c != 0.0) atomicAdd(p + 2, c);
 }
 
 // ----------------------------------------------------------------------------- forward
@@ -287,7 +280,11 @@ __global__ __launch_bounds__(kThreads) void k_cal_contacts(CalArgs A)
         Tm = Tm + ps.T;
         R = R + ps.R;
     }
-    if (A.tape_n) A.tape_n[i] = (uint8_t)nt;
+    if (A.tape_n) {
+        A.tape_n[i] = (uint8_t)nt;
+        const double o[10] = {F.x, F.y, F.z, M.x, M.y, M.z, Tm.x, Tm.y, Tm.z, R};
+        for (int q = 0; q < 10; q++) A.sums[10 * (size_t)i + q] = o[q];
+    }
 
     // ---- rolling resistance (impl:2420-2454), then the velocity update
     if (R != 0.0) {
@@ -335,6 +332,7 @@ struct StepRec {
     const uint32_t* tape_code;
     const uint16_t* tape_slot;
     const uint8_t* tape_n;
+    const double* sums;
 };
 
 // Cotangents of a state (the reverse sweep's lambda): positions 3 per sphere.
@@ -354,284 +352,190 @@ struct RevArgs {
     double* gtheta;     // [3]
 };
 
-// The contact sums of sphere i at step r (the forward's order and values).
-struct TailIn {
-    V3<double> F, Mc, Tm;
-    double R;
-};
+// A reverse kernel gives each lane one input direction of a sphere's Jacobian: Dual<1> values
+// whose derivative is taken with respect to input `dir` (every lane of the sphere repeats the
+// values). A thread per sphere on Dual<15> and Dual<23> kept hundreds of registers' worth of
+// derivatives in scratch memory on a few waves: for 5,000 spheres k_cal_rev_tail 292 -> 11.7 us,
+// k_cal_rev_contacts 91 -> 12.4 us.
+typedef Dual<1> D1;
 
-__device__ inline TailIn recompute_sums(const RevArgs& R, uint32_t i)
+__device__ inline D1 in1(double x, int k, int dir)
 {
-    const CalArgs& A = R.A;
-    const StepRec& r = R.r;
-    const Theta<double> th = {A.mu, A.rest, A.s};
-    const V4<double> ip = ld4d(r.pos1 + 4 * (size_t)i);
-    const V3<double> xi = {ip.x, ip.y, ip.z};
-    const double ir = ip.w, im = A.mass[i];
-    const V3<double> vi = ld3d(r.vel + 3 * (size_t)i);
-    const V3<double> wi = ang_vel(ld4d(r.ep1 + 4 * (size_t)i), ld4d(r.ev + 4 * (size_t)i));
-    Sums<double> pp = zero_sums<double>();
-    V3<double> Ft = {0.0, 0.0, 0.0};
-    const uint32_t nt = r.tape_n[i];
-    const size_t sb = (size_t)i * A.cap;
-    // sphere entries come first, in the forward's order
-    uint32_t m = 0;
-    for (; m < nt; m++) {
-        const uint32_t code = r.tape_code[(size_t)i * kTape + m];
-        if (code & kPlaneTag) break;
-        const int slot_in = (int)(r.tape_slot[(size_t)i * kTape + m] & 0xffu) - 1;
-        double sd0 = 0.0, sd1 = 0.0;
-        if (slot_in >= 0) {
-            sd0 = r.pp_tsd[2 * (sb + slot_in)];
-            sd1 = r.pp_tsd[2 * (sb + slot_in) + 1];
-        }
-        const V4<double> jp = ld4d(r.pos1 + 4 * (size_t)code);
-        const PairK<double> c = pair_k<double>(A.law.model, A.mat_pp, th, ir, jp.w, im, A.mass[code]);
-        pair_side<double>(A.law, c, A.mat_pp.rfric, xi, ir, V3<double>{jp.x, jp.y, jp.z}, jp.w, vi,
-                          ld3d(r.vel + 3 * (size_t)code), wi,
-                          ang_vel(ld4d(r.ep1 + 4 * (size_t)code), ld4d(r.ev + 4 * (size_t)code)), sd0, sd1, Ft, pp);
-    }
-    TailIn t;
-    t.F = V3<double>{0.0, 0.0, 0.0} + pp.F;
-    t.Mc = V3<double>{0.0, 0.0, 0.0} + pp.M;
-    t.Tm = ld3d(r.tmax + 3 * (size_t)i) + pp.T;
-    t.R = r.rres[i] + pp.R;
-    // walls: every wall adds its sums (zero without a contact), in id order
-    const size_t lb = (size_t)i * kPlSlots;
-    for (uint32_t w = 0; w < A.nplane; w++) {
-        Sums<double> ps = zero_sums<double>();
-        if (m < nt && r.tape_code[(size_t)i * kTape + m] == (kPlaneTag | w)) {
-            const int slot_in = (int)(r.tape_slot[(size_t)i * kTape + m] & 0xffu) - 1;
-            double sd0 = 0.0, sd1 = 0.0;
-            if (slot_in >= 0) {
-                sd0 = r.pl_tsd[2 * (lb + slot_in)];
-                sd1 = r.pl_tsd[2 * (lb + slot_in) + 1];
-            }
-            const PairK<double> c = pair_k<double>(A.law.model, A.mat_pl[w], th, ir, 0.0, im, 0.0);
-            plane_side<double>(A.law, c, A.mat_pl[w].rfric, A.planes[w], A.plane_dbi + 15 * (size_t)w, xi, ir, vi, wi,
-                               sd0, sd1, ps);
-            m++;
-        }
-        t.F = t.F + ps.F;
-        t.Mc = t.Mc + ps.M;
-        t.Tm = t.Tm + ps.T;
-        t.R = t.R + ps.R;
-    }
-    return t;
+    D1 r(x);
+    r.d[0] = k == dir ? 1.0 : 0.0;
+    return r;
+}
+__device__ inline V3<D1> in3(V3<double> v, int k0, int dir) { return {in1(v.x, k0, dir), in1(v.y, k0 + 1, dir), in1(v.z, k0 + 2, dir)}; }
+__device__ inline V4<D1> in4(V4<double> v, int k0, int dir)
+{
+    return {in1(v.x, k0, dir), in1(v.y, k0 + 1, dir), in1(v.z, k0 + 2, dir), in1(v.w, k0 + 3, dir)};
 }
 
 // Rolling resistance and the velocity update of sphere i. The translational part and the
 // rate update are linear and taken by hand; the Euler parameter accelerations (rolling
 // resistance, A(e)^T M, calculate_uceom) are differentiated with respect to e' (0-3), e_dot
-// (4-7), the contact moment (8-10), Tm (11-13) and Tr (14).
-constexpr int kTailN = 15;
+// (4-7), the contact moment (8-10), Tm (11-13) and Tr (14), one direction a lane, 16 lanes a
+// sphere. The contact sums are the recorded ones.
+constexpr uint32_t kTailLanes = 16;
 
-__global__ __launch_bounds__(64) void k_cal_rev_tail(RevArgs R)
+__global__ __launch_bounds__(256) void k_cal_rev_tail(RevArgs R)
 {
     const CalArgs& A = R.A;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = t / kTailLanes;
+    const int dir = (int)(t % kTailLanes);
     if (i >= A.n) return;
     const StepRec& r = R.r;
     const Lam &la = R.la, &lb = R.lb;
-    const TailIn t = recompute_sums(R, i);
+    const double* sum = r.sums + 10 * (size_t)i;
     const double hdt = 0.5 * A.dt, inv_m = 1.0 / A.mass[i];
     // v' = (v + hdt acc) + hdt a, acc' = a = (F + m g) / m; ev' = (ev + hdt ea) + hdt mea, ea' = mea
-    const V3<double> lv = ld3d(la.vel + 3 * (size_t)i), lacc = ld3d(la.acc + 3 * (size_t)i);
     const V4<double> lev = ld4d(la.ev + 4 * (size_t)i), lea = ld4d(la.ea + 4 * (size_t)i);
-    const double lmea[4] = {hdt * lev.x + lea.x, hdt * lev.y + lea.y, hdt * lev.z + lea.z, hdt * lev.w + lea.w};
-    typedef Dual<kTailN> D;
-    const V4<D> e1 = seed4<kTailN>(ld4d(r.ep1 + 4 * (size_t)i), 0);
-    const V4<D> ev = seed4<kTailN>(ld4d(r.ev + 4 * (size_t)i), 4);
-    V3<D> M = seed3<kTailN>(t.Mc, 8);
-    const V3<D> Tm = seed3<kTailN>(t.Tm, 11);
-    const D Tr = D::input(t.R, 14);
-    if (t.R != 0.0) {
+    const V4<D1> e1 = in4(ld4d(r.ep1 + 4 * (size_t)i), 0, dir);
+    const V4<D1> ev = in4(ld4d(r.ev + 4 * (size_t)i), 4, dir);
+    V3<D1> M = in3(ld3d(sum + 3), 8, dir);
+    const V3<D1> Tm = in3(ld3d(sum + 6), 11, dir);
+    const D1 Tr = in1(sum[9], 14, dir);
+    if (Tr.v != 0.0) {
         const double J = A.flat_inertia ? A.inertia[i] : A.inertia[3 * (size_t)i];
-        rolling<D>(A.dt, J, ang_vel(e1, ev), Tm, Tr, M);
+        rolling<D1>(A.dt, J, ang_vel(e1, ev), Tm, Tr, M);
     }
-    const V4<D> mea = uceom<D>(ld3d(A.inertia + 3 * (size_t)i), e1, ev, to_local(M, e1));
-    double g[kTailN];
-    for (int k = 0; k < kTailN; k++) g[k] = 0.0;
-    vjp_add(g, mea.x, lmea[0]);
-    vjp_add(g, mea.y, lmea[1]);
-    vjp_add(g, mea.z, lmea[2]);
-    vjp_add(g, mea.w, lmea[3]);
-    const double lev_a[4] = {lev.x, lev.y, lev.z, lev.w};
-    for (int q = 0; q < 4; q++) {
-        R.le1[4 * (size_t)i + q] = g[q];
-        lb.ev[4 * (size_t)i + q] = lev_a[q] + g[4 + q];
-        lb.ea[4 * (size_t)i + q] = hdt * lev_a[q];
+    const V4<D1> mea = uceom<D1>(ld3d(A.inertia + 3 * (size_t)i), e1, ev, to_local(M, e1));
+    double g[1] = {0.0};
+    vjp_add(g, mea.x, hdt * lev.x + lea.x);
+    vjp_add(g, mea.y, hdt * lev.y + lea.y);
+    vjp_add(g, mea.z, hdt * lev.z + lea.z);
+    vjp_add(g, mea.w, hdt * lev.w + lea.w);
+    const size_t i3 = 3 * (size_t)i, i4 = 4 * (size_t)i, ib = 10 * (size_t)i;
+    if (dir < 4) {
+        R.le1[i4 + dir] = g[0];
+    } else if (dir < 8) {
+        const double l = la.ev[i4 + dir - 4];
+        lb.ev[i4 + dir - 4] = l + g[0];
+        lb.ea[i4 + dir - 4] = hdt * l;
+    } else if (dir < 11) {
+        const int q = dir - 8;
+        const double l = la.vel[i3 + q];
+        lb.vel[i3 + q] = l;
+        lb.acc[i3 + q] = hdt * l;
+        R.bar[ib + q] = inv_m * (hdt * l + la.acc[i3 + q]);
+        R.bar[ib + 3 + q] = g[0];
+    } else if (dir < 14) {
+        const int q = dir - 11;
+        R.bar[ib + 6 + q] = g[0];
+        R.lom[i3 + q] = 0.0;
+        R.lpos1[i3 + q] = 0.0;
+    } else if (dir == 14) {
+        R.bar[ib + 9] = g[0];
     }
-    const double lv_a[3] = {lv.x, lv.y, lv.z}, lacc_a[3] = {lacc.x, lacc.y, lacc.z};
-    for (int q = 0; q < 3; q++) {
-        lb.vel[3 * (size_t)i + q] = lv_a[q];
-        lb.acc[3 * (size_t)i + q] = hdt * lv_a[q];
-        R.bar[10 * (size_t)i + q] = inv_m * (hdt * lv_a[q] + lacc_a[q]);
-        R.bar[10 * (size_t)i + 3 + q] = g[8 + q];
-        R.bar[10 * (size_t)i + 6 + q] = g[11 + q];
-        R.lom[3 * (size_t)i + q] = 0.0;
-        R.lpos1[3 * (size_t)i + q] = 0.0;
-    }
-    R.bar[10 * (size_t)i + 9] = g[14];
 }
 
-// One sphere-sphere contact differentiated with respect to x_i (0-2), x_j (3-5), v_i (6-8),
-// v_j (9-11), w_i (12-14), w_j (15-17), the history entry read (18-19), theta (20-22); the
-// previous pair's tangential force enters as a constant.
+// The contacts of a sphere, in the forward's order, 32 lanes a sphere. A sphere-sphere contact
+// is differentiated with respect to x_i (directions 0-2), x_j (3-5), v_i (6-8), v_j (9-11), w_i
+// (12-14), w_j (15-17), the history entry read (18-19) and theta (20-22); a wall contact with
+// respect to the same without the j ones; the previous pair's tangential force enters as a
+// constant. Lane e also keeps the cotangent of history value e of the sphere's pair slots (at
+// most 32) and, below 6, of its wall slots: slots that the step did not write pass theirs on.
 constexpr int kPairN = 23;
-// One wall contact: x_i (0-2), v_i (3-5), w_i (6-8), history (9-10), theta (11-13).
-constexpr int kWallN = 14;
+constexpr uint32_t kContactLanes = 32;
+static_assert(2 * XDEM_CALIB_MAX_CAPACITY <= kContactLanes, "a lane for every history value");
 
-__device__ inline void contacts_vjp(const RevArgs& R, uint32_t i, double (&gth)[3])
+__global__ __launch_bounds__(256) void k_cal_rev_contacts(RevArgs R)
 {
     const CalArgs& A = R.A;
     const StepRec& r = R.r;
-    const Theta<double> thd = {A.mu, A.rest, A.s};
-    const V4<double> ip = ld4d(r.pos1 + 4 * (size_t)i);
-    const V3<double> xi = {ip.x, ip.y, ip.z};
-    const double ir = ip.w, im = A.mass[i];
-    const V3<double> vi = ld3d(r.vel + 3 * (size_t)i);
-    const V3<double> wi = ang_vel(ld4d(r.ep1 + 4 * (size_t)i), ld4d(r.ev + 4 * (size_t)i));
-    const double* bar = R.bar + 10 * (size_t)i;
-    const V3<double> bF = {bar[0], bar[1], bar[2]}, bM = {bar[3], bar[4], bar[5]}, bT = {bar[6], bar[7], bar[8]};
-    const double bR = bar[9];
-    const uint32_t nt = r.tape_n[i];
-    const size_t sb = (size_t)i * A.cap;
-    V3<double> Ft = {0.0, 0.0, 0.0};   // the previous pair's tangential force (values)
-    V3<double> gx = {0.0, 0.0, 0.0}, gv = {0.0, 0.0, 0.0}, gw = {0.0, 0.0, 0.0};
-    uint32_t written_pp = 0u, written_pl = 0u;   // slots this step wrote (bit masks)
-    uint32_t m = 0;
-    for (; m < nt; m++) {
-        const uint32_t code = r.tape_code[(size_t)i * kTape + m];
-        if (code & kPlaneTag) break;
-        const uint16_t sl = r.tape_slot[(size_t)i * kTape + m];
-        const int slot_in = (int)(sl & 0xffu) - 1, slot_out = (int)(sl >> 8) - 1;
-        double sd0 = 0.0, sd1 = 0.0;
-        if (slot_in >= 0) {
-            sd0 = r.pp_tsd[2 * (sb + slot_in)];
-            sd1 = r.pp_tsd[2 * (sb + slot_in) + 1];
-        }
-        const uint32_t k = code;
-        const V4<double> jp = ld4d(r.pos1 + 4 * (size_t)k);
-        const V3<double> xj = {jp.x, jp.y, jp.z};
-        const V3<double> vj = ld3d(r.vel + 3 * (size_t)k);
-        const V3<double> wj = ang_vel(ld4d(r.ep1 + 4 * (size_t)k), ld4d(r.ev + 4 * (size_t)k));
-        // cotangents of this pair's new history entry
-        double bs0 = 0.0, bs1 = 0.0;
-        if (slot_out >= 0) {
-            bs0 = R.la.pp_tsd[2 * (sb + slot_out)];
-            bs1 = R.la.pp_tsd[2 * (sb + slot_out) + 1];
-            written_pp |= 1u << slot_out;
-        }
-        {
-            typedef Dual<kPairN> D;
-            const Theta<D> th = {D::input(A.mu, 20), D::input(A.rest, 21), D::input(A.s, 22)};
-            const PairK<D> c = pair_k<D>(A.law.model, A.mat_pp, th, ir, jp.w, im, A.mass[k]);
-            D s0 = D::input(sd0, 18), s1 = D::input(sd1, 19);
-            V3<D> FtD = const3<kPairN>(Ft);
-            Sums<D> acc = zero_sums<D>();
-            pair_side<D>(A.law, c, A.mat_pp.rfric, seed3<kPairN>(xi, 0), ir, seed3<kPairN>(xj, 3), jp.w,
-                         seed3<kPairN>(vi, 6), seed3<kPairN>(vj, 9), seed3<kPairN>(wi, 12), seed3<kPairN>(wj, 15), s0,
-                         s1, FtD, acc);
-            double g[kPairN];
-            for (int q = 0; q < kPairN; q++) g[q] = 0.0;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = t / kContactLanes;
+    const int dir = (int)(t % kContactLanes);
+    double gth = 0.0;   // lanes 20-22: cotangent of theta
+    if (i < A.n) {
+        const V4<double> ip = ld4d(r.pos1 + 4 * (size_t)i);
+        const V3<double> xi = {ip.x, ip.y, ip.z};
+        const double ir = ip.w, im = A.mass[i];
+        const V3<double> vi = ld3d(r.vel + 3 * (size_t)i);
+        const V3<double> wi = ang_vel(ld4d(r.ep1 + 4 * (size_t)i), ld4d(r.ev + 4 * (size_t)i));
+        const double* bar = R.bar + 10 * (size_t)i;
+        const V3<double> bF = {bar[0], bar[1], bar[2]}, bM = {bar[3], bar[4], bar[5]}, bT = {bar[6], bar[7], bar[8]};
+        const double bR = bar[9];
+        const uint32_t nt = r.tape_n[i];
+        const size_t sb = (size_t)i * A.cap, lb = (size_t)i * kPlSlots;
+        const Theta<D1> th = {in1(A.mu, 20, dir), in1(A.rest, 21, dir), in1(A.s, 22, dir)};
+        V3<double> Ft = {0.0, 0.0, 0.0};   // the previous pair's tangential force (values)
+        double own = 0.0;                  // cotangent of x_i, v_i or w_i (lanes 0-2, 6-8, 12-14)
+        double pp = 0.0, pl = 0.0;         // of this lane's history values before the step
+        uint32_t written_pp = 0u, written_pl = 0u;   // slots this step wrote (bit masks)
+        for (uint32_t m = 0; m < nt; m++) {
+            const uint32_t code = r.tape_code[(size_t)i * kTape + m];
+            const uint16_t sl = r.tape_slot[(size_t)i * kTape + m];
+            const int slot_in = (int)(sl & 0xffu) - 1, slot_out = (int)(sl >> 8) - 1;
+            const bool wall = (code & kPlaneTag) != 0u;
+            const double* tsd = wall ? r.pl_tsd + 2 * lb : r.pp_tsd + 2 * sb;
+            const double* lam = wall ? R.la.pl_tsd + 2 * lb : R.la.pp_tsd + 2 * sb;
+            D1 s0 = in1(slot_in >= 0 ? tsd[2 * slot_in] : 0.0, 18, dir);
+            D1 s1 = in1(slot_in >= 0 ? tsd[2 * slot_in + 1] : 0.0, 19, dir);
+            // cotangents of this contact's new history entry
+            const double bs0 = slot_out >= 0 ? lam[2 * slot_out] : 0.0;
+            const double bs1 = slot_out >= 0 ? lam[2 * slot_out + 1] : 0.0;
+            Sums<D1> acc = zero_sums<D1>();
+            uint32_t k = i;
+            if (!wall) {
+                if (slot_out >= 0) written_pp |= 1u << slot_out;
+                k = code;
+                const V4<double> jp = ld4d(r.pos1 + 4 * (size_t)k);
+                const V3<double> vj = ld3d(r.vel + 3 * (size_t)k);
+                const V3<double> wj = ang_vel(ld4d(r.ep1 + 4 * (size_t)k), ld4d(r.ev + 4 * (size_t)k));
+                const PairK<D1> c = pair_k<D1>(A.law.model, A.mat_pp, th, ir, jp.w, im, A.mass[k]);
+                V3<D1> FtD = {D1(Ft.x), D1(Ft.y), D1(Ft.z)};
+                pair_side<D1>(A.law, c, A.mat_pp.rfric, in3(xi, 0, dir), ir, in3(V3<double>{jp.x, jp.y, jp.z}, 3, dir), jp.w,
+                              in3(vi, 6, dir), in3(vj, 9, dir), in3(wi, 12, dir), in3(wj, 15, dir), s0, s1, FtD, acc);
+                Ft = {FtD.x.v, FtD.y.v, FtD.z.v};
+            } else {
+                if (slot_out >= 0) written_pl |= 1u << slot_out;
+                const uint32_t w = code & ~kPlaneTag;
+                const PairK<D1> c = pair_k<D1>(A.law.model, A.mat_pl[w], th, ir, 0.0, im, 0.0);
+                plane_side<D1>(A.law, c, A.mat_pl[w].rfric, A.planes[w], A.plane_dbi + 15 * (size_t)w, in3(xi, 0, dir), ir,
+                               in3(vi, 6, dir), in3(wi, 12, dir), s0, s1, acc);
+            }
+            double g[1] = {0.0};
             vjp_add3(g, acc.F, bF);
             vjp_add3(g, acc.M, bM);
             vjp_add3(g, acc.T, bT);
             vjp_add(g, acc.R, bR);
             vjp_add(g, s0, bs0);
             vjp_add(g, s1, bs1);
-            gx = gx + V3<double>{g[0], g[1], g[2]};
-            atomic_add3(R.lpos1 + 3 * (size_t)k, g[3], g[4], g[5]);
-            gv = gv + V3<double>{g[6], g[7], g[8]};
-            atomic_add3(R.lb.vel + 3 * (size_t)k, g[9], g[10], g[11]);
-            gw = gw + V3<double>{g[12], g[13], g[14]};
-            atomic_add3(R.lom + 3 * (size_t)k, g[15], g[16], g[17]);
-            if (slot_in >= 0) {
-                R.lb.pp_tsd[2 * (sb + slot_in)] += g[18];
-                R.lb.pp_tsd[2 * (sb + slot_in) + 1] += g[19];
+            // x_i, v_i, w_i stay in the lane, x_j, v_j, w_j go to the neighbour
+            if (dir < 18) {
+                const int kind = dir / 6, q = dir % 3;
+                if (dir % 6 < 3) own += g[0];
+                else if (!wall && g[0] != 0.0)
+                    atomicAdd((kind == 0 ? R.lpos1 : (kind == 1 ? R.lb.vel : R.lom)) + 3 * (size_t)k + q, g[0]);
+            } else if (dir >= 20 && dir < kPairN) {
+                gth += g[0];
             }
-            gth[0] += g[20];
-            gth[1] += g[21];
-            gth[2] += g[22];
+            const double g18 = __shfl(g[0], 18, kContactLanes), g19 = __shfl(g[0], 19, kContactLanes);
+            if (slot_in == dir / 2) {
+                if (wall) pl += dir & 1 ? g19 : g18;
+                else pp += dir & 1 ? g19 : g18;
+            }
         }
-        // the value pass, for the next pair's stale tangential force
-        {
-            const PairK<double> c = pair_k<double>(A.law.model, A.mat_pp, thd, ir, jp.w, im, A.mass[k]);
-            Sums<double> acc = zero_sums<double>();
-            double s0 = sd0, s1 = sd1;
-            pair_side<double>(A.law, c, A.mat_pp.rfric, xi, ir, xj, jp.w, vi, vj, wi, wj, s0, s1, Ft, acc);
+        if (dir < 18 && dir % 6 < 3 && own != 0.0) {
+            const int kind = dir / 6;
+            atomicAdd((kind == 0 ? R.lpos1 : (kind == 1 ? R.lb.vel : R.lom)) + 3 * (size_t)i + dir % 3, own);
         }
+        // slots this step did not write keep their values: their cotangents pass through
+        if (dir < (int)(2u * A.cap))
+            R.lb.pp_tsd[2 * sb + dir] = written_pp & (1u << (dir / 2)) ? pp : pp + R.la.pp_tsd[2 * sb + dir];
+        if (dir < 2 * kPlSlots)
+            R.lb.pl_tsd[2 * lb + dir] = written_pl & (1u << (dir / 2)) ? pl : pl + R.la.pl_tsd[2 * lb + dir];
     }
-    const size_t lb = (size_t)i * kPlSlots;
-    for (uint32_t w = 0; w < A.nplane && m < nt; w++) {
-        if (r.tape_code[(size_t)i * kTape + m] != (kPlaneTag | w)) continue;
-        const uint16_t sl = r.tape_slot[(size_t)i * kTape + m];
-        const int slot_in = (int)(sl & 0xffu) - 1, slot_out = (int)(sl >> 8) - 1;
-        m++;
-        double sd0 = 0.0, sd1 = 0.0;
-        if (slot_in >= 0) {
-            sd0 = r.pl_tsd[2 * (lb + slot_in)];
-            sd1 = r.pl_tsd[2 * (lb + slot_in) + 1];
-        }
-        double bs0 = 0.0, bs1 = 0.0;
-        if (slot_out >= 0) {
-            bs0 = R.la.pl_tsd[2 * (lb + slot_out)];
-            bs1 = R.la.pl_tsd[2 * (lb + slot_out) + 1];
-            written_pl |= 1u << slot_out;
-        }
-        typedef Dual<kWallN> D;
-        const Theta<D> th = {D::input(A.mu, 11), D::input(A.rest, 12), D::input(A.s, 13)};
-        const PairK<D> c = pair_k<D>(A.law.model, A.mat_pl[w], th, ir, 0.0, im, 0.0);
-        D s0 = D::input(sd0, 9), s1 = D::input(sd1, 10);
-        Sums<D> acc = zero_sums<D>();
-        plane_side<D>(A.law, c, A.mat_pl[w].rfric, A.planes[w], A.plane_dbi + 15 * (size_t)w, seed3<kWallN>(xi, 0), ir,
-                      seed3<kWallN>(vi, 3), seed3<kWallN>(wi, 6), s0, s1, acc);
-        double g[kWallN];
-        for (int q = 0; q < kWallN; q++) g[q] = 0.0;
-        vjp_add3(g, acc.F, bF);
-        vjp_add3(g, acc.M, bM);
-        vjp_add3(g, acc.T, bT);
-        vjp_add(g, acc.R, bR);
-        vjp_add(g, s0, bs0);
-        vjp_add(g, s1, bs1);
-        gx = gx + V3<double>{g[0], g[1], g[2]};
-        gv = gv + V3<double>{g[3], g[4], g[5]};
-        gw = gw + V3<double>{g[6], g[7], g[8]};
-        if (slot_in >= 0) {
-            R.lb.pl_tsd[2 * (lb + slot_in)] += g[9];
-            R.lb.pl_tsd[2 * (lb + slot_in) + 1] += g[10];
-        }
-        gth[0] += g[11];
-        gth[1] += g[12];
-        gth[2] += g[13];
-    }
-    atomic_add3(R.lpos1 + 3 * (size_t)i, gx.x, gx.y, gx.z);
-    atomic_add3(R.lb.vel + 3 * (size_t)i, gv.x, gv.y, gv.z);
-    atomic_add3(R.lom + 3 * (size_t)i, gw.x, gw.y, gw.z);
-    // slots this step did not write keep their values: their cotangents pass through
-    for (uint32_t q = 0; q < A.cap; q++)
-        if (!(written_pp & (1u << q))) {
-            R.lb.pp_tsd[2 * (sb + q)] += R.la.pp_tsd[2 * (sb + q)];
-            R.lb.pp_tsd[2 * (sb + q) + 1] += R.la.pp_tsd[2 * (sb + q) + 1];
-        }
-    for (int q = 0; q < kPlSlots; q++)
-        if (!(written_pl & (1u << q))) {
-            R.lb.pl_tsd[2 * (lb + q)] += R.la.pl_tsd[2 * (lb + q)];
-            R.lb.pl_tsd[2 * (lb + q) + 1] += R.la.pl_tsd[2 * (lb + q) + 1];
-        }
-}
-
-__global__ __launch_bounds__(64) void k_cal_rev_contacts(RevArgs R)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    double gth[3] = {0.0, 0.0, 0.0};
-    if (i < R.A.n) contacts_vjp(R, i, gth);
-    // theta: a wave sum (every lane takes part), then one atomic per wave and component
-    for (int q = 0; q < 3; q++) {
-        double v = gth[q];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if ((threadIdx.x & 63u) == 0u && v != 0.0) atomicAdd(R.gtheta + q, v);
+    // theta: the block's spheres, then one atomic per component
+    __shared__ double part[256 / kContactLanes][3];
+    if (dir >= 20 && dir < kPairN) part[threadIdx.x / kContactLanes][dir - 20] = gth;
+    __syncthreads();
+    if (threadIdx.x < 3u) {
+        double v = 0.0;
+        for (uint32_t q = 0; q < 256u / kContactLanes; q++) v += part[q][threadIdx.x];
+        if (v != 0.0) atomicAdd(R.gtheta + threadIdx.x, v);
     }
 }
 
@@ -822,9 +726,9 @@ struct xdem_calib {
     }
 
     // record layout of one step: pos1 4n, ep0 4n, ep1 4n, vel 3n, ev 4n, acc 3n, ea 4n, tmax 3n,
-    // rres n, pp_tsd 2 cap n, pl_tsd 6n (doubles); pp_count n, pp_id cap n, pl_count n, pl_id 3n,
+    // rres n, pp_tsd 2 cap n, pl_tsd 6n, sums 10n (doubles); pp_count n, pp_id cap n, pl_count n, pl_id 3n,
     // tape_code kTape n (u32); tape_slot kTape n (u16); tape_n n (u8)
-    size_t rec_doubles() const { return (size_t)n * (4 + 4 + 4 + 3 + 4 + 3 + 4 + 3 + 1 + 2 * cap + 2 * kPlSlots); }
+    size_t rec_doubles() const { return (size_t)n * (4 + 4 + 4 + 3 + 4 + 3 + 4 + 3 + 1 + 2 * cap + 2 * kPlSlots + 10); }
     size_t rec_size() const
     {
         size_t b = sizeof(double) * rec_doubles() + sizeof(uint32_t) * ((size_t)n * (1 + cap + 1 + kPlSlots + kTape));
@@ -849,6 +753,7 @@ struct xdem_calib {
         r.rres = d + o; o += N;
         r.pp_tsd = d + o; o += 2 * cap * N;
         r.pl_tsd = d + o; o += 2 * kPlSlots * N;
+        r.sums = d + o; o += 10 * N;
         uint32_t* u = reinterpret_cast<uint32_t*>(d + o);
         o = 0;
         r.pp_count = u + o; o += N;
@@ -923,6 +828,7 @@ struct xdem_calib {
             A.tape_code = const_cast<uint32_t*>(r.tape_code);
             A.tape_slot = const_cast<uint16_t*>(r.tape_slot);
             A.tape_n = const_cast<uint8_t*>(r.tape_n);
+            A.sums = const_cast<double*>(r.sums);
         }
         hipLaunchKernelGGL(k_cal_contacts, grid, dim3(kThreads), 0, stream, A);
         if ((e = hipGetLastError())) return e;
@@ -1155,6 +1061,8 @@ int xdem_calib_backward(xdem_calib* c, const double* dL_dpos, double grad[3])
     CAL_CHECK(hipMemcpyAsync(c->lam_view(la).pos, dL_dpos, sizeof(double) * 3 * N, hipMemcpyHostToDevice, st));
     const unsigned nsteps = c->last_steps;
     const dim3 grid((c->n + 63) / 64), block(64);
+    const dim3 tail_grid((unsigned)(((size_t)c->n * kTailLanes + 255) / 256));
+    const dim3 contact_grid((unsigned)(((size_t)c->n * kContactLanes + 255) / 256));
     const int seg0 = (int)(c->first_step / c->every);
     for (int seg = (int)((nsteps + c->every - 1) / c->every) - 1; seg >= seg0; seg--) {
         const unsigned k0 = (unsigned)seg * c->every, k1 = std::min(nsteps, k0 + c->every);
@@ -1173,9 +1081,8 @@ int xdem_calib_backward(xdem_calib* c, const double* dL_dpos, double grad[3])
             R.la = c->lam_view(la);
             R.lb = c->lam_view(la ^ 1);
             R.le1 = c->le1; R.lom = c->lom; R.lpos1 = c->lpos1; R.bar = c->bar; R.gtheta = c->gtheta;
-            hipLaunchKernelGGL(k_fill_zero, zg, zb, 0, st, R.lb.pp_tsd, (size_t)(2 * c->cap + 2 * kPlSlots) * N);
-            hipLaunchKernelGGL(k_cal_rev_tail, grid, block, 0, st, R);
-            hipLaunchKernelGGL(k_cal_rev_contacts, grid, block, 0, st, R);
+            hipLaunchKernelGGL(k_cal_rev_tail, tail_grid, dim3(256), 0, st, R);
+            hipLaunchKernelGGL(k_cal_rev_contacts, contact_grid, dim3(256), 0, st, R);
             hipLaunchKernelGGL(k_cal_rev_head, grid, block, 0, st, R);
             CAL_CHECK(hipGetLastError());
             la ^= 1;
