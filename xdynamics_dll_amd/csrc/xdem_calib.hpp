@@ -32,14 +32,14 @@ template <class S> struct PairK {
     double eq_m, eq_r;
 };
 
-template <class S>
-__host__ __device__ inline PairK<S> pair_k(int model, const Material& m, const Theta<S>& th, double ir, double jr,
-                                           double im, double jm)
+// The part of them that no sphere changes: 4/3 E*, 8 G*, beta, the tangential damping factor.
+template <class S> struct MatK {
+    S e43, ks8, beta, vs;
+};
+
+template <class S> __host__ __device__ inline MatK<S> mat_k(const Material& m, const Theta<S>& th)
 {
     const double pi = 3.14159265358979323846;
-    PairK<S> c;
-    c.eq_m = jm ? (im * jm) / (im + jm) : im;
-    c.eq_r = jr ? (ir * jr) / (ir + jr) : ir;
     const S f = exp(th.s);
     const S iE = m.Ei * f, jE = m.Ej * f;
     const double ip = m.pri, jp = m.prj;
@@ -47,13 +47,34 @@ __host__ __device__ inline PairK<S> pair_k(int model, const Material& m, const T
     S Seq = (2.0 * (2.0 - ip) * (1.0 + ip) / iE) + (2.0 * (2.0 - jp) * (1.0 + jp) / jE);
     Seq = 1.0 / Seq;
     const S lne = log(th.rest);
-    const S beta = -lne * sqrt(1.0 / (lne * lne + pi * pi));
-    c.kn = (4.0 / 3.0) * Eeq * sqrt(c.eq_r);
-    c.vn = beta;
-    c.ks = model == 1 ? 8.0 * Seq : c.kn * m.sratio;
-    c.vs = model == 1 ? 2.0 * sqrt(5.0 / 6.0) * beta : c.vn * m.sratio;
+    MatK<S> k;
+    k.beta = -lne * sqrt(1.0 / (lne * lne + pi * pi));
+    k.e43 = (4.0 / 3.0) * Eeq;
+    k.ks8 = 8.0 * Seq;
+    k.vs = 2.0 * sqrt(5.0 / 6.0) * k.beta;
+    return k;
+}
+
+template <class S>
+__host__ __device__ inline PairK<S> pair_k(int model, const Material& m, const MatK<S>& k, const Theta<S>& th, double ir,
+                                           double jr, double im, double jm)
+{
+    PairK<S> c;
+    c.eq_m = jm ? (im * jm) / (im + jm) : im;
+    c.eq_r = jr ? (ir * jr) / (ir + jr) : ir;
+    c.kn = k.e43 * sqrt(c.eq_r);
+    c.vn = k.beta;
+    c.ks = model == 1 ? k.ks8 : c.kn * m.sratio;
+    c.vs = model == 1 ? k.vs : c.vn * m.sratio;
     c.mu = th.mu;
     return c;
+}
+
+template <class S>
+__host__ __device__ inline PairK<S> pair_k(int model, const Material& m, const Theta<S>& th, double ir, double jr,
+                                           double im, double jm)
+{
+    return pair_k<S>(model, m, mat_k<S>(m, th), th, ir, jr, im, jm);
 }
 
 template <class S> __host__ __device__ inline V3<S> s3(double x, double y, double z) { return {S(x), S(y), S(z)}; }

@@ -14,6 +14,15 @@
 
 namespace xdem {
 
+// LDS written by some lanes of a wave and then read by others: the wave's own accesses complete
+// in program order; the fences keep the compiler from moving them across this point.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Material constants of one contact object, computed once (host or device).
 __host__ __device__ inline ContactConst make_contact_const(const xdem_contact_property& p, double reach_radius)
 {

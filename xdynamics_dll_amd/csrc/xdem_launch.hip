@@ -186,15 +186,6 @@ __global__ __launch_bounds__(kThreads) void k_hash(LaunchPrm L, unsigned* hash, 
 }
 
 // --------------------------------------------------------- sphere-sphere (impl:613-733)
-// LDS written by some lanes of a wave and then read by others: the wave's own accesses complete
-// in program order; the fences keep the compiler from moving them across this point.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The material constants, the same in every lane, to scalar registers (computed with vector
 // instructions they would take 32 vector registers for the whole kernel).
 __device__ __forceinline__ ContactConst uniform_const(const xdem_contact_property* cp)

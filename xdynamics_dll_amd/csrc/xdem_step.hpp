@@ -488,15 +488,6 @@ __device__ __forceinline__ OwnState load_own(const StepArgs& A, const SceneDev& 
     return o;
 }
 
-// LDS written by some lanes of a wave and then read by others: the wave's own accesses complete
-// in program order; the fences keep the compiler from moving them across this point.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---------------------------------------------------------------- reference visiting order
 // The reference visits the neighbours of sphere i cell by cell, z, y, x offsets -1..1 in
 // that nesting, spheres of a cell by id (impl:613-733 over the sorted cell table; the stable
