@@ -1,5 +1,5 @@
-"""The full contact pass at the sizes where its division of work changes: a wave takes 4 to 64
-touched spheres, found by sweeping the sorted slots when at least half of them are touched and
+"""The full contact pass at the sizes where its division of work changes: a wave takes 1 to 64
+touched spheres, by whether SIMDs get one wave or two, found by sweeping the sorted slots when at least half of them are touched and
 from the queue otherwise. FP64 states and histories are those of the oracle, bit for bit: the
 pass adds a sphere's pairs in the reference's order whatever the division."""
 import numpy as np
@@ -34,7 +34,7 @@ def pack(n, free, seed=11):
 
 @pytest.mark.parametrize("fuse", [True, False])
 @pytest.mark.parametrize("n, free", [(1, 0), (3, 4), (4, 0), (65, 200), (255, 0), (2049, 3000), (4097, 0),
-                                     (9000, 12000), (70001, 0)])
+                                     (9000, 12000), (26011, 0), (70001, 0)])
 def test_full_pass_equals_oracle(n, free, fuse):
     scene = pack(n, free)
     print(f"[full pass] {n} touching, {free} free, fuse={fuse}", flush=True)

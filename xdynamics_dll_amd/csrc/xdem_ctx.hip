@@ -371,6 +371,7 @@ struct xdem_ctx {
         A.zero_force = 1;
         A.full_blocks = cfg.full_blocks ? std::max(cfg.full_blocks, kQueueSegs) : collide_blocks;
         A.resident_blocks = resident_blocks;
+        A.half_grid = collide_blocks / 2;
         A.group_max_from = cfg.merge_pairs_below ? cfg.merge_pairs_below : UINT32_MAX;
         A.has_cyl = cyls.empty() ? 0 : 1;
         return A;

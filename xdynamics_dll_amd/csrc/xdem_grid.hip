@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_drift(StepArgs A)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= A.np) return;
-    const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+    const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
     drift_sphere(A, S, i, ld4(A.pos + 4 * i), ld4(A.ep + 4 * i), ld3(A.vel + 3 * i), ld3(A.acc + 3 * i),
                  ld4(A.ev + 4 * i), ld4(A.ea + 4 * i));
 }
@@ -325,7 +325,7 @@ __device__ __forceinline__ void count_unit(const StepArgs& A, uint32_t u)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         if (idx[r] >= A.np) continue;
-        const SceneDev& S = A.scenes[scene_index(A, idx[r], MULTI)];
+        const SceneDev& S = table_at(A.scenes, scene_index(A, idx[r], MULTI));
         int gx, gy, gz;
         grid_cell(S.grid, p[r].x, p[r].y, p[r].z, gx, gy, gz);
         const uint32_t key = grid_bucket(S.grid, gx, gy, gz);
@@ -360,7 +360,7 @@ __device__ __forceinline__ void order_gather_slot(const StepArgs& A, uint32_t j)
     if (f >= A.nsorted) { atomicOr(A.err, XDEM_ERR_GRID_SYNC); return; }
     A.svals[f] = k;
     const V4<double> p = ld4(A.pos + 4 * k);
-    const SceneDev& S = A.scenes[scene_index(A, k, MULTI)];
+    const SceneDev& S = table_at(A.scenes, scene_index(A, k, MULTI));
     // exact FP64 reach test against every wall and cylinder of the scene (radius grown by the
     // skin): a sphere with one in reach goes to the full contact pass; and
     // the least displacement that could bring a wall into reach, |dp . uw| / max(1, |uw|) -
@@ -369,7 +369,7 @@ __device__ __forceinline__ void order_gather_slot(const StepArgs& A, uint32_t j)
     bool far = true;
     double wgap = 3.0e38;
     for (uint32_t w = 0; w < S.nwall; w++) {
-        const WallDev& W = A.walls[S.wall_begin + w];
+        const WallDev& W = table_at(A.walls, S.wall_begin + w);
         far = far & wall_out_of_reach(W.cc, W.info, p, S.skin * scale);
         const xdem_plane_info& pl = W.info;
         const double uw2 = pl.uw.x * pl.uw.x + pl.uw.y * pl.uw.y + pl.uw.z * pl.uw.z;
@@ -380,7 +380,7 @@ __device__ __forceinline__ void order_gather_slot(const StepArgs& A, uint32_t j)
     // cylinders: in reach with the radius grown by the skin, and the gap the largest overlap
     // lacks (it changes by at most the distance the sphere or the body moves)
     for (uint32_t c = 0; CYL && c < S.ncyl; c++) {
-        const CylDev& C = A.cyls[S.cyl_begin + c];
+        const CylDev& C = table_at(A.cyls, S.cyl_begin + c);
         far = far & cylinder_out_of_reach(C.cc, C.info, C.dbi, C.margin, p, S.skin * scale);
         const double g = C.cc.coh != 0.0 ? -1.0
                                          : -cylinder_reach(C.info, cylinder_axis(C.info, C.dbi), mk3(p.x, p.y, p.z),

@@ -130,6 +130,14 @@ struct CylDev {
     uint32_t pad_;
 };
 
+// Entry k of a table of scenes or bodies, read through the constant address space: a kernel never
+// changes these tables, so an index that is the same in all lanes gives scalar loads, which do
+// not wait for the lanes' own loads and stores, and keep the constants in scalar registers.
+template <class E> __device__ __forceinline__ const E& table_at(const E* t, uint32_t k)
+{
+    return *(const E*)((const __attribute__((address_space(4))) E*)t + k);
+}
+
 struct StepArgs {
     // state (reference layouts, all scenes concatenated)
     double* pos;  double* vel;  double* acc;  double* ep;  double* ev;  double* ea;
@@ -208,6 +216,7 @@ struct StepArgs {
     uint32_t full_blocks;                    // grid of the full-pass kernels (host side: launch shape)
     uint32_t resident_blocks;                // grid of k_touch: the blocks the device holds at once at
                                              // three waves per SIMD (host side)
+    uint32_t half_grid;                      // k_collide: the blocks that give every SIMD one wave
     uint32_t group_max_from;                 // full passes of this size or more: 64 spheres to a wave
     int has_cyl;                             // a scene has cylinders (host side: the CYL kernels)
     int stale_ft, flat_inertia, keep_velocity, tmax_persist;
@@ -265,7 +274,7 @@ __device__ __forceinline__ uint32_t pairs_slot(const StepArgs& A, uint32_t j, ui
 {
     uint32_t n = 0;
     float pgap = 3.0e38f;
-    const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+    const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
     const float4 fi = A.sposf[j];
     if (S.has_pp) {
         // the sphere's bucket coordinates from its key (dims are powers of two)
@@ -343,7 +352,7 @@ __device__ __forceinline__ uint32_t pairs_slot(const StepArgs& A, uint32_t j, ui
 // skin is within that distance now. Writes the sphere's triangle list and returns its length.
 __device__ __forceinline__ uint32_t mesh_slot(const StepArgs& A, const SceneDev& S, uint32_t i)
 {
-    const MeshDev& M = A.meshes[S.mesh];
+    const MeshDev& M = table_at(A.meshes, S.mesh);
     const V4<double> p = ld4(A.pos + 4 * (size_t)i);
     const V4<double> e = {M.dbi[XDEM_E0], M.dbi[XDEM_E1], M.dbi[XDEM_E2], M.dbi[XDEM_E3]};
     const V3<double> loc = rot_local(mk3(p.x - M.dbi[XDEM_PX], p.y - M.dbi[XDEM_PY], p.z - M.dbi[XDEM_PZ]), e);
@@ -557,18 +566,18 @@ __device__ __forceinline__ bool touch_sphere(const StepArgs& A, const TouchGroup
     bool touch = false;
     uint32_t n = 0;
     V4<double> p = {0.0, 0.0, 0.0, 0.0};
-    const SceneDev& S = A.scenes[i != kInvalid ? scene_index(A, i, MULTI) : 0u];
+    const SceneDev& S = table_at(A.scenes, i != kInvalid ? scene_index(A, i, MULTI) : 0u);
     if (i != kInvalid) {
         p = ld4(A.pos + 4 * (size_t)i);
         touch = (fl & kMeshNear) != 0u;
         if (fl & kWallNear) {
             for (uint32_t w = 0; w < S.nwall; w++) {
-                const WallDev& W = A.walls[S.wall_begin + w];
+                const WallDev& W = table_at(A.walls, S.wall_begin + w);
                 touch = touch || !wall_out_of_reach(W.cc, W.info, p);
             }
             if (CYL)
                 for (uint32_t c = 0; c < S.ncyl; c++) {
-                    const CylDev& C = A.cyls[S.cyl_begin + c];
+                    const CylDev& C = table_at(A.cyls, S.cyl_begin + c);
                     touch = touch || !cylinder_out_of_reach(C.cc, C.info, C.dbi, C.margin, p, 0.0);
                 }
         }
@@ -790,7 +799,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             if (built && i != kInvalid) {
                 fl = pairs_slot<MULTI>(A, j, i);
                 if (MESH) {
-                    const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+                    const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
                     if (S.mesh >= 0 && mesh_slot(A, S, i)) fl |= kMeshNear | kCandidate;
                 }
             }
@@ -916,14 +925,14 @@ __device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S
 // Cohesion-only pairs add their attraction. The first kPairIds slot ids of the previous step
 // are staged in LDS.
 constexpr uint32_t kPairIds = 16;
-constexpr uint32_t kGroupMin = 4;      // k_collide: the fewest spheres to a wave
+constexpr uint32_t kTwoWavesFrom = 26000; // k_collide: the touched spheres from which SIMDs get two waves
 
 // Sphere i's pair with neighbour k: the neighbour's state, the history entry of `slot`, the
-// force law; writes the new slot `rank` and returns the kind.
+// force law; returns the kind and the pair's new history entry in `nh`.
 template <class T, int MODEL, bool GPU_LAW>
 __device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S, uint32_t i, V4<double> ipos,
-                                            V3<double> ivel, V3<double> iom, double imass, uint32_t k, uint32_t rank,
-                                            uint32_t slot, double v[10])
+                                            V3<double> ivel, V3<double> iom, double imass, uint32_t k, uint32_t slot,
+                                            double v[10], double2& nh)
 {
     const uint32_t hb = i * A.cap;
     const V4<double> jpos = ld4(A.pos + 4 * (size_t)k);
@@ -945,10 +954,7 @@ __device__ __forceinline__ uint32_t pair_of(const StepArgs& A, const SceneDev& S
         v[0] = a.x; v[1] = a.y; v[2] = a.z;
         kind = kPairCoh;
     }
-    if (rank < A.cap) {
-        A.pp_id_out[hb + rank] = k;
-        A.pp_tsd_out[hb + rank] = make_double2(sd0, sd1);
-    }
+    nh = make_double2(sd0, sd1);
     return kind;
 }
 
@@ -1023,7 +1029,7 @@ __device__ __forceinline__ void collide_tail(const StepArgs& A, const SceneDev& 
         n_wall = count;
         if (S.wall_dynamic)
             for (uint32_t w = 0; w < S.nwall; w++) {
-                const int32_t slot = A.walls[S.wall_begin + w].wslot;
+                const int32_t slot = table_at(A.walls, S.wall_begin + w).wslot;
                 if (slot < 0) continue;
                 double* wr = A.wrench + (size_t)slot * 6 * A.np;
 #pragma unroll
@@ -1033,7 +1039,7 @@ __device__ __forceinline__ void collide_tail(const StepArgs& A, const SceneDev& 
         // wall slots are read only when a wall needs them and written back only
         // when one changed (the values in memory are the same either way)
         for (uint32_t w = 0; w < S.nwall; w++) {
-            const WallDev& W = A.walls[S.wall_begin + w];
+            const WallDev& W = table_at(A.walls, S.wall_begin + w);
             double bf[6] = {0, 0, 0, 0, 0, 0};
             if (wall_contact<T, MODEL, GPU_LAW>(W.cc, W.info, W.dbi, S.dt, o.pos, o.vel, iom, o.mass, ws, tot, bf))
                 err |= XDEM_ERR_PLANE_OVERFLOW;
@@ -1097,8 +1103,8 @@ template <class T, bool MULTI, int MODEL, bool GPU_LAW>
 __device__ __forceinline__ void mesh_sphere(const StepArgs& A, uint32_t i)
 {
     constexpr uint32_t CAP = XDEM_MAX_P2MS_COUNT;
-    const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
-    const MeshDev& M = A.meshes[S.mesh];
+    const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
+    const MeshDev& M = table_at(A.meshes, S.mesh);
     const V4<double> p4 = ld4(A.pos + 4 * (size_t)i);
     const V3<double> ip = mk3(p4.x, p4.y, p4.z);
     const double ir = p4.w;
@@ -1314,7 +1320,7 @@ __global__ __launch_bounds__(256) void k_collide_lite(StepArgs A)
     reset_rebuild_slots(A);
     uint32_t n_wall = 0;
     lite_spheres(A, [&](uint32_t i, uint32_t skip) {
-        const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+        const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
         LiteIn in;
         lite_load<FUSE>(A, S, i, in);
         lite_sphere<FUSE>(A, S, i, in, skip, n_wall);
@@ -1335,7 +1341,7 @@ __global__ __launch_bounds__(256) void k_lite_move(StepArgs A)
     uint32_t n_wall = 0;
     float dmx = 0.0f;
     lite_spheres(A, [&](uint32_t i, uint32_t skip) {
-        const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+        const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
         const uint32_t flags = A.nbr_count[i];
         // a wave of full-pass spheres only (a dense pack) ends here: the loads below would take
         // bandwidth from the full pass
@@ -1407,7 +1413,7 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
     lite_spheres(A, [&](uint32_t i, uint32_t skip) {
         const uint32_t flags = A.nbr_count[i];
         if (flags & (skip | kSpinStable)) return;
-        const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+        const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
         const V4<double> e = ld4(A.ep + 4 * i);
         const V4<double> ev0 = ld4(A.ev + 4 * i);
         const V4<double> aa = ld4(A.ea + 4 * i);
@@ -1455,16 +1461,23 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
 // sphere_pair_add's operations, so the sums, slots and counts are those of a one-thread walk,
 // and goes on with the walls, the velocity update and the next drift (collide_tail).
 //
-// G: as few spheres as put all of them on half the grid's waves (one per SIMD) in one round,
-// between 4 and 64. A wave issues the same instructions for a few spheres as for 64, so more
-// waves than SIMDs cost issue slots, and fewer cost rounds of pairs one after the other.
+// G: as few spheres as put all of them on one wave per SIMD in one round (1 to 64), from
+// kTwoWavesFrom touched spheres on two waves per SIMD. Two waves share a SIMD's issue slots, but
+// one waits while the other works: a step of 10,000 spheres 47.4 us with one and 50.6 with two,
+// 20,000: 55.5 and 57.0, 25,000: 62.0 and 62.8, 31,000: 67.9 and 64.6, 90,000: 108 and 96. At
+// least four spheres to a wave was slower below 4,000 spheres (1,000: 46.3 and 43.3 us).
 //
 // Bound by the latency of a wave's chain (list entry, neighbour state, the FP64 divisions and
-// roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 29 us for
-// 10,000 touched spheres, 63 us for 61,000 (FP64 and DHS; a thread per sphere walking its own
-// pairs: 44 and 88 us). Beyond, two waves per SIMD wait for the neighbour gathers: 500,000
-// spheres with 3.6M pairs 263 us, half of the line requests missing L2 (a pair pass with a
-// second pass over the spheres for the rest: 172 + 110 us and 160 bytes a sphere between them).
+// roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 18 us for
+// 1,000 touched spheres, 27 us for 10,000, 46 us for 61,000 (FP64 and DHS; a thread per sphere
+// walking its own pairs: 44 us for 10,000 and 88 us for 61,000). Beyond, two waves per SIMD wait
+// for the neighbour gathers: 500,000 spheres with 3.4M pairs 266 us, half of the line requests
+// missing L2 (a pair pass with a second pass over the spheres for the rest: 172 + 110 us and 160
+// bytes a sphere between them). What the chain waits for is kept short: the scene and wall
+// tables are scalar loads (as vector loads each waited for the wave's earlier stores), a
+// sphere's flags, mask, state and slot ids are loaded together, new slots are stored after the
+// sums, and a pair's results are read while the previous pair's are added (29 -> 27, 63 -> 55
+// and 317 -> 266 us for 10,000, 61,000 and 500,000 spheres with the same waves).
 template <class T, bool MULTI, bool FUSE, int MODEL, bool GPU_LAW, bool CYL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_collide(StepArgs A)
 {
@@ -1481,7 +1494,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint32_t qcnt = sweep ? 0u : A.seg_count2[qb.seg * kSegStride];
     const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;   // a multiple of 4
     const uint32_t todo = sweep ? A.nsorted : qcnt;
-    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(kGroupMin, (2u * todo + waves - 1u) / waves));
+    const uint32_t halve = nfull < kTwoWavesFrom && gridDim.x > A.half_grid ? 2u : 1u;
+    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(1u, (halve * todo + waves - 1u) / waves));
     const uint32_t nvb = (A.nsorted + 4u * G - 1u) / (4u * G);
     const uint32_t it0 = sweep ? blockIdx.x : (qb.chunk * 4u + wave) * G;
     const uint32_t it_end = sweep ? nvb : qcnt;
@@ -1498,42 +1512,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                 i = qseg[it + lane];
             }
         }
+        // what the pairs need of the sphere, its slots and its flags, issued together
         uint32_t flags = 0;
-        if (i < A.np) {
-            flags = A.nbr_count[i];
-            if (!(flags & kTouch)) i = kInvalid;
-        } else {
-            i = kInvalid;
-        }
-        // what the pairs need of the sphere and its slot counts, issued together
-        const uint32_t nlist_all = flags & kCountMask;
         unsigned long long m = 0;
         uint32_t old_count = 0, wall_count0 = 0;
         bool has_pp = false;
-        if (i != kInvalid) {
-            const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
-            has_pp = S.has_pp != 0u;
-            if (has_pp && min(nlist_all, A.list_cap)) m = A.pass_mask[i];
-            old_count = min(A.pp_count_in[i], A.cap);
-            wall_count0 = S.nwall ? A.pl_count[i] : 0u;
+        if (i < A.np) {
+            const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
+            flags = A.nbr_count[i];
+            m = A.pass_mask[i];   // of this step for a touched sphere with listed neighbours
+            old_count = A.pp_count_in[i];
+            wall_count0 = A.pl_count[i];
             const V4<double> p = ld4(A.pos + 4 * (size_t)i);
             const V3<double> v = ld3(A.vel + 3 * (size_t)i);
             const V4<double> e = ld4(A.ep + 4 * (size_t)i), d = ld4(A.ev + 4 * (size_t)i);
             const double mass = A.mass[i];
             const uint32_t hb = i * A.cap;
-            const uint32_t nid = m ? min(old_count, kPairIds) : 0u;
             if ((A.cap & 3u) == 0u) {
                 const uint4* p4 = reinterpret_cast<const uint4*>(A.pp_id_in + hb);
-                for (uint32_t q = 0; q < nid; q += 4u) *reinterpret_cast<uint4*>(&st.ids[lane][q]) = p4[q / 4u];
+                // no branch between them: all are in flight together
+                const uint4 q0 = p4[0], q1 = p4[A.cap > 4u ? 1 : 0], q2 = p4[A.cap > 8u ? 2 : 0], q3 = p4[A.cap > 12u ? 3 : 0];
+                uint4* ids = reinterpret_cast<uint4*>(&st.ids[lane][0]);
+                ids[0] = q0; ids[1] = q1; ids[2] = q2; ids[3] = q3;
             } else {
-                for (uint32_t q = 0; q < nid; q++) st.ids[lane][q] = A.pp_id_in[hb + q];
+                for (uint32_t q = 0; q < min(A.cap, kPairIds); q++) st.ids[lane][q] = A.pp_id_in[hb + q];
             }
             const V3<double> w = omega_of(e, d);
             st.own[0][lane] = p.x; st.own[1][lane] = p.y; st.own[2][lane] = p.z; st.own[3][lane] = p.w;
             st.own[4][lane] = v.x; st.own[5][lane] = v.y; st.own[6][lane] = v.z;
             st.own[7][lane] = w.x; st.own[8][lane] = w.y; st.own[9][lane] = w.z;
             st.own[10][lane] = mass;
+            has_pp = S.has_pp != 0u;
+            old_count = min(old_count, A.cap);
+            if (!S.nwall) wall_count0 = 0u;
+            if (!(flags & kTouch)) i = kInvalid;
+        } else {
+            i = kInvalid;
         }
+        const uint32_t nlist_all = flags & kCountMask;
+        if (i == kInvalid || !has_pp || !min(nlist_all, A.list_cap)) m = 0ull;
         const uint32_t c = (uint32_t)__popcll(m);
         // inclusive scan of the counts over the wave
         uint32_t incl = c;
@@ -1575,12 +1592,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             if (b + 64u < total) locate(x + 64u, Ln, rn, kn);
             const uint32_t iL = __shfl(i, (int)L, 64);
             const uint32_t ocL = __shfl(old_count, (int)L, 64);
+            const uint32_t hb = iL * A.cap;
+            double2 nh = make_double2(0.0, 0.0);
+            uint32_t kind = kPairSet;
             if (x < total) {
-                const SceneDev& S = A.scenes[scene_index(A, iL, MULTI)];
+                const SceneDev& S = table_at(A.scenes, scene_index(A, iL, MULTI));
                 const V4<double> ipos = {st.own[0][L], st.own[1][L], st.own[2][L], st.own[3][L]};
                 const V3<double> ivel = mk3(st.own[4][L], st.own[5][L], st.own[6][L]);
                 const V3<double> wL = mk3(st.own[7][L], st.own[8][L], st.own[9][L]);
-                const uint32_t hb = iL * A.cap;
                 uint32_t slot = kInvalid;
 #pragma unroll
                 for (int q = (int)kPairIds - 1; q >= 0; q--)   // downwards: the lowest match stays
@@ -1588,8 +1607,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                 for (uint32_t q = kPairIds; q < ocL && slot == kInvalid; q++)
                     if (A.pp_id_in[hb + q] == k) slot = q;
                 double v[10];
-                const uint32_t kind =
-                    pair_of<T, MODEL, GPU_LAW>(A, S, iL, ipos, ivel, wL, st.own[10][L], k, r, slot, v);
+                kind = pair_of<T, MODEL, GPU_LAW>(A, S, iL, ipos, ivel, wL, st.own[10][L], k, slot, v, nh);
 #pragma unroll
                 for (int q = 0; q < 10; q++) st.v[q][lane] = v[q];
                 st.kind[lane] = kind;
@@ -1599,28 +1617,52 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             // tangential force set, for a pair without one of its own (quirk Q4)
             const uint32_t lo = max(first, b), hi = min(incl, b + 64u);
             uint32_t last = kInvalid;
-            for (uint32_t y = lo; y < hi; y++) {
-                const uint32_t q = y - b;
+            if (!__any(kind != kPairSet)) {
+                // the next pair's values are read while this one's are added
                 double v[7];
+                if (lo < hi) {
 #pragma unroll
-                for (int z = 0; z < 7; z++) v[z] = st.v[z][q];
-                const uint32_t kind = st.kind[q];
-                if (kind == kPairCoh) {
-                    pp.F = pp.F - mk3(v[0], v[1], v[2]);
-                    continue;
+                    for (int z = 0; z < 7; z++) v[z] = st.v[z][lo - b];
+                    last = hi - 1u - b;
                 }
-                if (kind == kPairStale && last != kInvalid && A.stale_ft)
-                    Ft = mk3(T(st.v[7][last]), T(st.v[8][last]), T(st.v[9][last]));
-                sphere_pair_add<T>(v, kind == kPairSet, Ft, pp);
-                if (kind == kPairSet) last = q;
+                for (uint32_t y = lo; y < hi; y++) {
+                    const uint32_t qn = min(y + 1u, hi - 1u) - b;
+                    double vn[7];
+#pragma unroll
+                    for (int z = 0; z < 7; z++) vn[z] = st.v[z][qn];
+                    sphere_pair_add<T>(v, true, Ft, pp);
+#pragma unroll
+                    for (int z = 0; z < 7; z++) v[z] = vn[z];
+                }
+            } else {
+                for (uint32_t y = lo; y < hi; y++) {
+                    const uint32_t q = y - b;
+                    double v[7];
+#pragma unroll
+                    for (int z = 0; z < 7; z++) v[z] = st.v[z][q];
+                    const uint32_t kq = st.kind[q];
+                    if (kq == kPairCoh) {
+                        pp.F = pp.F - mk3(v[0], v[1], v[2]);
+                        continue;
+                    }
+                    if (kq == kPairStale && last != kInvalid && A.stale_ft)
+                        Ft = mk3(T(st.v[7][last]), T(st.v[8][last]), T(st.v[9][last]));
+                    sphere_pair_add<T>(v, kq == kPairSet, Ft, pp);
+                    if (kq == kPairSet) last = q;
+                }
             }
             if (last != kInvalid && A.stale_ft && incl > b + 64u)   // more pairs in the next chunk
                 Ft = mk3(T(st.v[7][last]), T(st.v[8][last]), T(st.v[9][last]));
             wave_lds_sync();
+            // the new slots last: a wait for a load issued after a store waits for the store too
+            if (x < total && r < A.cap) {
+                A.pp_id_out[hb + r] = k;
+                A.pp_tsd_out[hb + r] = nh;
+            }
             L = Ln; r = rn; k = kn;
         }
         if (i != kInvalid) {
-            const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+            const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
             uint32_t err = 0, n_wall = 0;
             if (has_pp) {
                 const uint32_t n_new = min(c, A.cap);
@@ -1653,7 +1695,7 @@ __global__ __launch_bounds__(256) void k_finish(StepArgs A)
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     float dmx = 0.0f;
     if (i < A.np) {
-        const SceneDev& S = A.scenes[scene_index(A, i, MULTI)];
+        const SceneDev& S = table_at(A.scenes, scene_index(A, i, MULTI));
         const V4<double> e = ld4(A.ep + 4 * i);
         V4<double> av = ld4(A.ev + 4 * i);
         V3<double> M = ld3(A.moment + 3 * i);

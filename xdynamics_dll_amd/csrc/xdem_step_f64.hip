@@ -28,8 +28,8 @@ void collide_passes(const StepArgs& A, int pass, hipStream_t s)
 {
     const dim3 g = grid_for(A.np), b(kBlock);
     if (pass == 1) {
-        if (A.has_cyl) hipLaunchKernelGGL((k_collide<double, MULTI, FUSE, MODEL, GPU_LAW, true>), full_grid(A, 4 * kGroupMin), b, 0, s, A);
-        else hipLaunchKernelGGL((k_collide<double, MULTI, FUSE, MODEL, GPU_LAW, false>), full_grid(A, 4 * kGroupMin), b, 0, s, A);
+        if (A.has_cyl) hipLaunchKernelGGL((k_collide<double, MULTI, FUSE, MODEL, GPU_LAW, true>), full_grid(A, 4), b, 0, s, A);
+        else hipLaunchKernelGGL((k_collide<double, MULTI, FUSE, MODEL, GPU_LAW, false>), full_grid(A, 4), b, 0, s, A);
     } else if (pass == 2) {
         // the triangle pass (grid-strided over the mesh queue, whose length is on the device)
         hipLaunchKernelGGL((k_mesh_pass<double, MULTI, MODEL, GPU_LAW>), full_grid(A, kBlock), b, 0, s, A);
