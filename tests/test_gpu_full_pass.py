@@ -1,7 +1,8 @@
 """The full contact pass at the sizes where its division of work changes: a wave takes 1 to 64
-touched spheres, by whether SIMDs get one wave or two, found by sweeping the sorted slots when at least half of them are touched and
-from the queue otherwise. FP64 states and histories are those of the oracle, bit for bit: the
-pass adds a sphere's pairs in the reference's order whatever the division."""
+touched spheres, by whether SIMDs get one wave or two, found by sweeping the sorted slots when at
+least half of them are touched; otherwise at least 32 from the queue. FP64 states and histories
+are those of the oracle, bit for bit: the pass adds a sphere's pairs in the reference's order
+whatever the division."""
 import numpy as np
 import pytest
 
@@ -34,7 +35,7 @@ def pack(n, free, seed=11):
 
 @pytest.mark.parametrize("fuse", [True, False])
 @pytest.mark.parametrize("n, free", [(1, 0), (3, 4), (4, 0), (65, 200), (255, 0), (2049, 3000), (4097, 0),
-                                     (9000, 12000), (26011, 0), (70001, 0)])
+                                     (9000, 12000), (31, 3000), (2113, 40000), (26011, 0), (70001, 0)])
 def test_full_pass_equals_oracle(n, free, fuse):
     scene = pack(n, free)
     print(f"[full pass] {n} touching, {free} free, fuse={fuse}", flush=True)

@@ -733,8 +733,8 @@ __device__ __forceinline__ void queue_append(uint32_t* q, uint32_t* count, uint3
 // kernel waits for dependent loads (the list entries, then the positions they name), so a small
 // set of candidates takes 4 to 16 lanes a sphere, one such round trip on more waves; a large one
 // a lane a sphere. Per launch, against a lane a sphere for every set and a root for every pair:
-// 10,000 candidates with lists of 14: 27 -> 12 us, 61,000: 35 -> 23, 500,000: 109 -> 102 (the
-// build steps among them, with lists sorted by rank in LDS: 440 -> 314).
+// 10,000 candidates with lists of 14: 27 -> 11 us, 61,000: 35 -> 20, 500,000: 109 -> 90 (the
+// build steps among them, with lists sorted by rank in LDS: 440 -> 300).
 template <bool MULTI, bool CYL, bool MESH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_touch(StepArgs A)
 {
@@ -758,6 +758,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const uint32_t* wq = A.work + (size_t)qb.seg * A.seg_cap;
     // on a build step the candidates are not known yet: every slot
     const uint32_t mine = built ? 0u : A.seg_count[qb.seg * kSegStride];
+    // the first queue entries of a wave that takes 64, read together with the counts
+    const uint32_t at64 = (qb.chunk * 4u + wave) * 64u + lane;
+    const uint32_t early = !built && at64 < A.seg_cap ? wq[at64] : kInvalid;
     const uint32_t ncand = queue_total(A.seg_count), nlisted = queue_total(A.seg_count + 1);
     const bool sweep = built || 2ull * ncand >= (unsigned long long)A.nsorted;
     if (!sweep && mine == 0u) return;
@@ -804,7 +807,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                 }
             }
         } else if (lane < per && it + lane < mine) {
-            i = wq[it + lane];
+            i = per == 64u && it == it0 ? early : wq[it + lane];
         }
         if (built) {
             queue_append(A.work, A.seg_count, seg, A.seg_cap, (fl & kCandidate) != 0u, i);
@@ -925,6 +928,7 @@ __device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S
 // Cohesion-only pairs add their attraction. The first kPairIds slot ids of the previous step
 // are staged in LDS.
 constexpr uint32_t kPairIds = 16;
+constexpr uint32_t kQueueGroup = 32;     // k_collide: the fewest spheres to a wave that takes them from the queue
 constexpr uint32_t kTwoWavesFrom = 26000; // k_collide: the touched spheres from which SIMDs get two waves
 
 // Sphere i's pair with neighbour k: the neighbour's state, the history entry of `slot`, the
@@ -1465,7 +1469,12 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
 // kTwoWavesFrom touched spheres on two waves per SIMD. Two waves share a SIMD's issue slots, but
 // one waits while the other works: a step of 10,000 spheres 47.4 us with one and 50.6 with two,
 // 20,000: 55.5 and 57.0, 25,000: 62.0 and 62.8, 31,000: 67.9 and 64.6, 90,000: 108 and 96. At
-// least four spheres to a wave was slower below 4,000 spheres (1,000: 46.3 and 43.3 us).
+// least four spheres to a wave was slower below 4,000 spheres (1,000: 46.3 and 43.3 us). From the
+// queue at least kQueueGroup: most spheres are then in the lite pass beside this kernel, which
+// more waves slow down, and the few have few pairs. Steps of a falling column of 1,000,000 with
+// 1,500 touched spheres, per 50: 4.68 ms from 1 sphere to a wave, 4.50 from 16, 4.44 from 32,
+// 4.48 from 64; 48 scenes with 10,000 to 20,000 touched of 474,000, per 20: 1.88 to 2.25 ms, 1.91
+// to 2.26, 1.91 to 2.12, 2.03 to 2.14.
 //
 // Bound by the latency of a wave's chain (list entry, neighbour state, the FP64 divisions and
 // roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 18 us for
@@ -1485,17 +1494,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     PairStage& st = stage_all[threadIdx.x >> 6];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
+    const QueueBlock qb = queue_block(blockIdx.x, gridDim.x);
+    const uint32_t* qseg = A.work2 + (size_t)qb.seg * A.seg_cap;
+    // the first queue entries of a wave of kQueueGroup, read together with the counts
+    const uint32_t at_first = (qb.chunk * 4u + wave) * kQueueGroup + lane;
+    const uint32_t early = lane < kQueueGroup && at_first < A.seg_cap ? qseg[at_first] : kInvalid;
     const uint32_t nfull = queue_total(A.seg_count2);
     const bool sweep = 2ull * nfull >= (unsigned long long)A.nsorted;
     // the wave's spheres: sorted slots (it = virtual block of 4 G slots) or queue entries (it =
     // the wave's first entry); either way the loop bounds are the same for the whole wave
-    const QueueBlock qb = queue_block(blockIdx.x, gridDim.x);
-    const uint32_t* qseg = A.work2 + (size_t)qb.seg * A.seg_cap;
     const uint32_t qcnt = sweep ? 0u : A.seg_count2[qb.seg * kSegStride];
     const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;   // a multiple of 4
     const uint32_t todo = sweep ? A.nsorted : qcnt;
     const uint32_t halve = nfull < kTwoWavesFrom && gridDim.x > A.half_grid ? 2u : 1u;
-    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(1u, (halve * todo + waves - 1u) / waves));
+    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(sweep ? 1u : kQueueGroup, (halve * todo + waves - 1u) / waves));
     const uint32_t nvb = (A.nsorted + 4u * G - 1u) / (4u * G);
     const uint32_t it0 = sweep ? blockIdx.x : (qb.chunk * 4u + wave) * G;
     const uint32_t it_end = sweep ? nvb : qcnt;
@@ -1509,7 +1521,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                 const uint32_t j = (xcd_block(it, nvb) * 4u + wave) * G + lane;
                 if (j < A.nsorted) i = A.svals[j];
             } else if (it + lane < qcnt) {
-                i = qseg[it + lane];
+                i = G == kQueueGroup && it == it0 ? early : qseg[it + lane];
             }
         }
         // what the pairs need of the sphere, its slots and its flags, issued together
