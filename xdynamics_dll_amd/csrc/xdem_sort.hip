@@ -7,14 +7,16 @@
 //   k_scatter   adds up the counts of the earlier tiles and of all tiles itself (no scan kernel
 //               between: a block reads the whole table, 1 KB a tile, coalesced and from L2), ranks
 //               its pairs among equal digits, reorders the tile in LDS by digit and writes runs of
-//               equal digits
+//               equal digits. That reading grows with the square of the tiles: beyond kTableTiles
+//               of them two kernels between, k_chunk_sums and k_chunk_bases, leave a block one row
+//               and its own chunk's earlier tiles to read.
 // and k_bounds, the first and one-past-last position of every occupied cell. A wave ranks its own 64
 // pairs at a time with wave64 ballots against counters of its own, so the block synchronises only
 // once for all of them; ranks respect input order, which makes the sort stable.
 //
-// Bound by latency: the kernels of a call take 84 -> 48 us for 120,000 pairs and 21 key bits and 131 ->
-// 64 us for 1,048,575
-// (three kernels a digit, one of them a scan by one work-group, and separate copies and fills).
+// Bound by latency up to about a million pairs: the kernels of a call take 84 -> 48 us for 120,000
+// pairs and 21 key bits and 131 -> 64 us for 1,048,575 (three kernels a digit, one of them a scan by
+// one work-group, and separate copies and fills).
 #include "xdem_sort.hpp"
 
 namespace xdem {
@@ -25,9 +27,15 @@ constexpr uint32_t kWaves = kThreads / 64;
 constexpr uint32_t kItems = 4;
 constexpr uint32_t kTile = kThreads * kItems;
 constexpr uint32_t kSmall = kThreads * 8;   // pairs that one block sorts, 2, 4 or 8 a thread
+constexpr uint32_t kChunk = 32;      // tiles whose counts are added up together beyond kTableTiles
+// The most tiles whose whole table every block reads: the reorder launcher takes 67 us either way
+// for 1,000,000 pairs, 109 against 84 for 2,000,000, 240 against 123 for 4,000,000 and 8,540 against
+// 1,004 for 32,000,000 (the kernels of one scan by one work-group 143, 204, 358 and 2,750); 49
+// against 56 for 100,000.
+constexpr uint32_t kTableTiles = 256;
 constexpr uint32_t kNone = 0xffffffffu;
 
-// Both cell tables from entry b * kThreads on, four entries a thread and step, by nb blocks.
+// Both cell tables from entry b * kThreads on, by nb blocks.
 __device__ __forceinline__ void clear_cells(uint32_t* cstart, uint32_t* cend, uint32_t ncell, uint32_t b, uint32_t nb)
 {
     for (size_t i = (size_t)b * kThreads + threadIdx.x; i < ncell; i += (size_t)nb * kThreads) {
@@ -128,10 +136,68 @@ __device__ __forceinline__ void rank_tile(const uint32_t (&digit)[ITEMS], uint32
     for (uint32_t s = 0; s < ITEMS; s++) place[s] += start[digit[s]] + cnt[w][digit[s]];
 }
 
+// The counts of kChunk tiles added up, a chunk a block: a quarter of the block adds up a quarter of
+// the chunk's tiles.
+__device__ __forceinline__ uint32_t chunk_part(const uint32_t* __restrict__ hist, uint32_t chunk, uint32_t end)
+{
+    const uint32_t d = threadIdx.x & 255u, t0 = chunk * kChunk + (threadIdx.x >> 8) * (kChunk / 4u);
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kChunk / 4u; u++) sum += t0 + u < end ? hist[(t0 + u) * 256u + d] : 0u;
+    return sum;
+}
+
+__global__ __launch_bounds__(kThreads) void k_chunk_sums(const uint32_t* __restrict__ hist, uint32_t ntiles,
+                                                         uint32_t* __restrict__ sums)
+{
+    __shared__ uint32_t s_part[kThreads];
+    const uint32_t tid = threadIdx.x;
+    s_part[tid] = chunk_part(hist, blockIdx.x, ntiles);
+    __syncthreads();
+    if (tid < 256u)
+        sums[blockIdx.x * 256u + tid] = s_part[tid] + s_part[256u + tid] + s_part[512u + tid] + s_part[768u + tid];
+}
+
+// The chunks' sums to the first position of each digit of each chunk, in place, by one block: a
+// quarter of it takes a quarter of the chunks.
+__global__ __launch_bounds__(kThreads) void k_chunk_bases(uint32_t* __restrict__ sums, uint32_t nchunk)
+{
+    __shared__ uint32_t s_part[kThreads], s_wsum[4], s_first[256];
+    const uint32_t tid = threadIdx.x, d = tid & 255u, g = tid >> 8, per = (nchunk + 3u) / 4u;
+    const uint32_t lo = min(nchunk, g * per), hi = min(nchunk, lo + per);
+    uint32_t part = 0;
+    for (uint32_t t = lo; t < hi; t += 8u) {
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; u++) part += t + u < hi ? sums[(t + u) * 256u + d] : 0u;
+    }
+    s_part[tid] = part;
+    __syncthreads();
+    const uint32_t all = s_part[d] + s_part[256u + d] + s_part[512u + d] + s_part[768u + d];
+    const uint32_t first = scan256(all, s_wsum);
+    if (tid < 256u) s_first[tid] = first;
+    __syncthreads();
+    uint32_t run = s_first[d];
+    for (uint32_t q = 0; q < g; q++) run += s_part[q * 256u + d];
+    for (uint32_t t = lo; t < hi; t += 8u) {
+        uint32_t c[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; u++) c[u] = t + u < hi ? sums[(t + u) * 256u + d] : 0u;
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; u++) {
+            if (t + u < hi) sums[(t + u) * 256u + d] = run;
+            run += c[u];
+        }
+    }
+}
+
+// BASES: the counts of whole chunks come added up (k_chunk_bases). As a branch of one kernel the
+// other reading's sorts took 1 to 2 percent longer.
+template <bool BASES>
 __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                       uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                       uint32_t* __restrict__ vout2, uint32_t n, uint32_t shift,
-                                                      const uint32_t* __restrict__ hist, uint32_t ntiles)
+                                                      const uint32_t* __restrict__ hist, uint32_t ntiles,
+                                                      const uint32_t* __restrict__ bases)
 {
     __shared__ uint32_t s_keys[kTile], s_vals[kTile];
     __shared__ uint32_t s_cnt[kWaves][256];
@@ -148,7 +214,13 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint32_t* __restrict
     }
     // digit d of this tile goes after all smaller digits and after digit d of the earlier tiles:
     // a quarter of the block adds up a quarter of the tiles' counts
-    {
+    if (BASES) {
+        const uint32_t chunk = blockIdx.x / kChunk;
+        s_keys[tid] = chunk_part(hist, chunk, blockIdx.x);
+        __syncthreads();
+        if (tid < 256u)
+            s_gbase[tid] = bases[chunk * 256u + tid] + s_keys[tid] + s_keys[256u + tid] + s_keys[512u + tid] + s_keys[768u + tid];
+    } else {
         const uint32_t d = tid & 255u, g = tid >> 8, per = (ntiles + 3u) / 4u;
         const uint32_t lo = min(ntiles, g * per), hi = min(ntiles, lo + per);
         uint32_t pre = 0, all = 0, t = lo;
@@ -286,7 +358,7 @@ hipError_t cell_sort(uint32_t* hash, uint32_t* index, uint32_t* sorted_index, ui
     uint32_t bits = 1;
     while (bits < 32u && (1ull << bits) < (unsigned long long)ncell) bits++;
     const uint32_t npass = (bits + 7u) / 8u;
-    const uint32_t clear_blocks = std::min(512u, (ncell + kThreads - 1u) / kThreads);
+    const uint32_t clear_blocks = std::min(512u, (ncell - 1u) / kThreads + 1u);   // ncell > 0
     if (n <= kSmall) {
         hipLaunchKernelGGL(k_clear, dim3(clear_blocks), dim3(kThreads), 0, stream, cstart, cend, ncell);
         if (n > 4u * kThreads)
@@ -308,8 +380,19 @@ hipError_t cell_sort(uint32_t* hash, uint32_t* index, uint32_t* sorted_index, ui
         const uint32_t extra = p == 0u ? clear_blocks : 0u;
         hipLaunchKernelGGL(k_hist, dim3(ntiles + extra), dim3(kThreads), 0, stream, ksrc, n, 8u * p, hist, ntiles, cstart,
                            cend, ncell);
-        hipLaunchKernelGGL(k_scatter, dim3(ntiles), dim3(kThreads), 0, stream, ksrc, vsrc, kdst, vdst,
-                           out ? sorted_index : nullptr, n, 8u * p, hist, ntiles);
+        uint32_t* vcopy = out ? sorted_index : nullptr;
+        if (ntiles <= kTableTiles) {
+            hipLaunchKernelGGL(k_scatter<false>, dim3(ntiles), dim3(kThreads), 0, stream, ksrc, vsrc, kdst, vdst, vcopy, n,
+                               8u * p, hist, ntiles, (const uint32_t*)nullptr);
+        } else {
+            // a row of 256 for each chunk, in an array that this digit neither reads nor writes
+            uint32_t* bases = out ? buf[2u * (p & 1u)] : (p ? sorted_index : buf[2]);
+            const uint32_t nchunk = (ntiles + kChunk - 1u) / kChunk;
+            hipLaunchKernelGGL(k_chunk_sums, dim3(nchunk), dim3(kThreads), 0, stream, hist, ntiles, bases);
+            hipLaunchKernelGGL(k_chunk_bases, dim3(1), dim3(kThreads), 0, stream, bases, nchunk);
+            hipLaunchKernelGGL(k_scatter<true>, dim3(ntiles), dim3(kThreads), 0, stream, ksrc, vsrc, kdst, vdst, vcopy, n,
+                               8u * p, hist, ntiles, (const uint32_t*)bases);
+        }
         ksrc = kdst;
         vsrc = vdst;
     }
