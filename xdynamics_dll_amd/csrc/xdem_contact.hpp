@@ -83,23 +83,27 @@ __device__ __forceinline__ PairGeom pair_geom(V4<double> pi_, V4<double> pj)
     return g;
 }
 
+// Whether a gap d >= 0 lies inside the JKR separation depth at R* = Req (impl:415-423). The depth's
+// cube decides unless the two are within a billionth of each other; there the depth itself does.
+__device__ __forceinline__ bool within_cohesion_depth(const ContactConst& cc, double Req, double d)
+{
+    const double x = (cc.pcc * Req) / cc.ee, v = d / 0.75, v3 = v * v * v;
+    if (x > 1e-280) {   // above it v3 loses nothing to underflow where the two are close
+        if (v3 < x * (1.0 - 1e-9)) return true;
+        if (v3 > x * (1.0 + 1e-9)) return false;
+    }
+    return d < fabs(cohesion_limit_depth(cc, Req));
+}
+
 // The reference's pair predicate: overlap, or inside the JKR separation depth of a cohesive
-// pair (impl:671-718). The depth is 3/4 pow(x, 1.0 / 3.0), x = cohesion_limit_depth's argument; its
-// cube decides but for distances within a billionth of it, and there cbrt(x) with the
-// difference of the rounded exponent to a third (-1.85e-17 ln x) is the same to an ulp, without
-// the registers of pow.
+// pair (impl:671-718).
 __device__ __forceinline__ bool pair_passes(const ContactConst& cc, V4<double> pi, V4<double> pj)
 {
     const PairGeom g = pair_geom(pi, pj);
     if (g.cdist > 0) return true;
     if (!(cc.coh_reach > 0.0 && -g.cdist < cc.coh_reach)) return false;
     const double ir = pi.w, jr = pj.w;
-    const double Req = jr ? (ir * jr) / (ir + jr) : ir;
-    const double x = (cc.pcc * Req) / cc.ee, d = fabs(g.cdist), v = d / 0.75, v3 = v * v * v;
-    if (v3 < x * (1.0 - 1e-9)) return true;
-    if (v3 > x * (1.0 + 1e-9)) return false;
-    const double t = cbrt(x);
-    return d < 0.75 * (t - t * (1.8503717077085941e-17 * (double)__logf(fmaxf((float)x, 1e-37f))));
+    return within_cohesion_depth(cc, jr ? (ir * jr) / (ir + jr) : ir, fabs(g.cdist));
 }
 
 // The predicate where the squared distance decides it without a root: 1 passes, 0 does not, 2

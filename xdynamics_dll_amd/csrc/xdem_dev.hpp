@@ -172,11 +172,15 @@ __device__ __forceinline__ T cohesion_force(const ContactConst& cc, T Req, T Fn)
     return cf;
 }
 
+// Not inlined: pow takes 68 registers, which the contact and pair-test kernels would hold for a
+// call that they hardly make.
+__device__ __attribute__((noinline)) inline double pow_third(double x) { return pow(x, 1.0 / 3.0); }
+
 // Separation depth below which a cohesive pair still attracts (impl:415-423).
 __device__ __forceinline__ double cohesion_limit_depth(const ContactConst& cc, double Req)
 {
     const double c1 = (cc.pcc * Req) / cc.ee;
-    return -(3.0 / 4.0) * pow(c1, 1.0 / 3.0);
+    return -(3.0 / 4.0) * pow_third(c1);
 }
 
 // Normal and tangential force of one pair (impl:432-474; xContact.cpp:210-264).
