@@ -875,20 +875,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 
 // End of a sphere's contact pass. Fused mode: rolling resistance (impl:2420-2454) and the
 // velocity and orientation-rate update (xIntegratorVV.cpp:131-152; impl:192-222). Split
-// mode: the sums are stored for k_finish.
-template <bool FUSE>
-__device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S, uint32_t i, const OwnState& o,
-                                            Accum tot, uint32_t& err, float& dmx)
+// mode: the sums are stored for k_finish. late(o) is called before position, velocity and mass are
+// used: a caller that has them in LDS reads them there again instead of holding 16 registers
+// through uceom, whose 4 x 4 inverse needs most of them.
+template <bool FUSE, class Late>
+__device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S, uint32_t i, OwnState o, Accum tot,
+                                            uint32_t& err, float& dmx, Late&& late)
 {
     if (FUSE) {
         const V4<double> e = o.ep;
         V4<double> av = o.ev;
         const bool consumed = rolling_moment(S.dt, o.J, omega_of(e, av), tot.T, tot.R, tot.M);
         if (A.tmax_persist) st3(A.tmax + 3 * i, consumed ? mk3(0.0, 0.0, 0.0) : tot.T);
-        const double m = o.mass;
         const V4<double> aa = o.ea;
         const V3<double> np_ = rot_local(tot.M, e);
         const V4<double> mea = uceom(o.inertia, e, av, np_);
+        late(o);
+        const double m = o.mass;
         const double inv_m = 1.0 / m;
         const V3<double> a = mk3(inv_m * (tot.F.x + m * S.gx), inv_m * (tot.F.y + m * S.gy),
                                  inv_m * (tot.F.z + m * S.gz));
@@ -1009,11 +1012,12 @@ __device__ __forceinline__ uint32_t collide_cylinders(const CylDev* cyls, uint32
 
 // The rest of sphere i's full contact pass after its sphere pairs (their sums in pp): every wall
 // of the scene in id order, its cylinders, the triangle sums, then sphere_tail. count0: the wall
-// slot count before the step.
+// slot count before the step. own: PairStage::own of the wave, the sphere's in column `lane`.
 template <class T, bool MULTI, bool FUSE, int MODEL, bool GPU_LAW, bool CYL>
 __device__ __forceinline__ void collide_tail(const StepArgs& A, const SceneDev& S, uint32_t i, uint32_t flags,
                                              uint32_t count0, OwnState& o, V3<double> iom, const PairSums& pp,
-                                             uint32_t& n_wall, uint32_t err, float& dmx)
+                                             uint32_t& n_wall, uint32_t err, float& dmx, const double (*own)[64],
+                                             uint32_t lane)
 {
     WallSlots ws;
     ws.init(count0, A.pl_id + XDEM_MAX_P2PL_COUNT * i,
@@ -1089,7 +1093,12 @@ __device__ __forceinline__ void collide_tail(const StepArgs& A, const SceneDev& 
     }
 
     if (FUSE) load_own_fused(A, S, i, o);
-    sphere_tail<FUSE>(A, S, i, o, tot, err, dmx);
+    sphere_tail<FUSE>(A, S, i, o, tot, err, dmx, [&](OwnState& w) {
+        asm volatile("" ::: "memory");   // not earlier
+        w.pos = {own[0][lane], own[1][lane], own[2][lane], own[3][lane]};
+        w.vel = mk3(own[4][lane], own[5][lane], own[6][lane]);
+        w.mass = own[10][lane];
+    });
     if (err) atomicOr(A.err, err);
 }
 
@@ -1295,7 +1304,7 @@ __device__ __forceinline__ void lite_sphere(const StepArgs& A, const SceneDev& S
         n_wall += count;
     }
     float dmx = 0.0f;   // the split lite pass computes no drift
-    sphere_tail<FUSE>(A, S, i, in.o, tot, err, dmx);
+    sphere_tail<FUSE>(A, S, i, in.o, tot, err, dmx, [](OwnState&) {});
     if (err) atomicOr(A.err, err);
 }
 
@@ -1486,7 +1495,10 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
 // tables are scalar loads (as vector loads each waited for the wave's earlier stores), a
 // sphere's flags, mask, state and slot ids are loaded together, new slots are stored after the
 // sums, and a pair's results are read while the previous pair's are added (29 -> 27, 63 -> 55
-// and 317 -> 266 us for 10,000, 61,000 and 500,000 spheres with the same waves).
+// and 317 -> 266 us for 10,000, 61,000 and 500,000 spheres with the same waves). Two waves leave a
+// lane 256 registers: with pow inlined in the walls and the own state held through the update 54 to
+// 66 values went through scratch memory, 6 percent of a dense step (500,000 spheres: 399 -> 374 us)
+// and 34 -> 29 us a launch for 1,500 touched spheres beside a lite pass of 1,000,000.
 template <class T, bool MULTI, bool FUSE, int MODEL, bool GPU_LAW, bool CYL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_collide(StepArgs A)
 {
@@ -1691,7 +1703,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             o.ep = ld4(A.ep + 4 * (size_t)i);
             o.ev = ld4(A.ev + 4 * (size_t)i);
             o.t0 = A.tmax_persist ? ld3(A.tmax + 3 * (size_t)i) : mk3(0.0, 0.0, 0.0);
-            collide_tail<T, MULTI, FUSE, MODEL, GPU_LAW, CYL>(A, S, i, flags, wall_count0, o, iom, pp, n_wall, err, dmx);
+            collide_tail<T, MULTI, FUSE, MODEL, GPU_LAW, CYL>(A, S, i, flags, wall_count0, o, iom, pp, n_wall, err, dmx, st.own,
+                                                              lane);
             c1 += n_wall;
         }
     }
