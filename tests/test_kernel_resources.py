@@ -59,6 +59,6 @@ def test_scratch_of_the_contact_kernels():
     assert max(plain.values()) <= 16, plain
     one = {n: v for n, v in plain.items() if n.split(", ")[1] == "false"}   # one scene
     assert len(one) == 16 and max(one.values()) == 0, one
-    for name in ("k_p2p<", "k_touch<false, false", "k_touch<true, false"):
+    for name in ("k_p2p<", "k_touch<"):
         some = {n: v for n, v in k.items() if n.startswith(name)}
         assert some and max(some.values()) == 0, some
