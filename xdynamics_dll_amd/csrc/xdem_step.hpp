@@ -36,6 +36,7 @@ constexpr uint32_t kCountMask = 0x01ffffffu;
 // slower: its few thousand full-pass spheres then fell into a few segments, on few XCDs.)
 constexpr uint32_t kQueueSegs = 64;
 constexpr uint32_t kSegStride = 32;           // uint32 entries between two segment counters
+constexpr uint32_t kCandTotal = 2, kListedTotal = 3;   // entries of seg_count's first line
 constexpr uint32_t kCounterStride = 16;       // 64-bit entries between two partial contact counts
 constexpr uint32_t kBarFlags = 64;            // release flags of k_rebuild's phases
 constexpr uint32_t kRebuildPhases = 6;        // k_rebuild: count, reduce, parts, apply, scatter, order
@@ -203,7 +204,8 @@ struct StepArgs {
     unsigned long long* counters;  // kQueueSegs partial counts, kCounterStride apart: [0] stored sphere
                                    // contacts, [1] stored wall and cylinder contacts
     uint32_t* seg_count;           // per candidate queue segment (kSegStride apart): its spheres, and
-                                   // the entries of their lists
+                                   // the entries of their lists; in the first line also the totals
+                                   // of both (lite pass of a build step)
     uint32_t* seg_count2;          // spheres per full-pass queue segment (kSegStride apart)
     uint32_t seg_cap;              // entries per queue segment in work and work2
     uint32_t* grid_bar;            // k_rebuild's phase cursors, done counters and release flags,
@@ -766,7 +768,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CYL ? 2 : 3
     // the first queue entries of a wave that takes 64, read together with the counts
     const uint32_t at64 = (qb.chunk * 4u + wave) * 64u + lane;
     const uint32_t early = !built && at64 < A.seg_cap ? wq[at64] : kInvalid;
-    const uint32_t ncand = queue_total(A.seg_count), nlisted = queue_total(A.seg_count + 1);
+    const uint32_t ncand = A.seg_count[kCandTotal], nlisted = A.seg_count[kListedTotal];
     const bool sweep = built || 2ull * ncand >= (unsigned long long)A.nsorted;
     if (!sweep && mine == 0u) return;
     const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;
@@ -817,13 +819,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CYL ? 2 : 3
         if (built) {
             queue_append(A.work, A.seg_count, seg, A.seg_cap, (fl & kCandidate) != 0u, i);
             uint32_t listed_sum = min(fl & kCountMask, A.list_cap);
+            if (__any(listed_sum != 0u)) {
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) listed_sum += __shfl_xor(listed_sum, off, 64);
-            if (lane == 0u && listed_sum) atomicAdd(&A.seg_count[seg * kSegStride + 1u], listed_sum);
+                for (int off = 32; off > 0; off >>= 1) listed_sum += __shfl_xor(listed_sum, off, 64);
+                if (lane == 0u) atomicAdd(&A.seg_count[seg * kSegStride + 1u], listed_sum);
+            }
             if (MESH) queue_append(A.mesh_work, A.mesh_count, 0u, 0u, (fl & kMeshNear) != 0u, i);
-            // the lanes' list and gap stores are read back by other lanes of the wave
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         }
         // whether the sphere has to be tested: one with listed triangles goes to the full pass every
         // step (the triangle pass evaluates its list exactly); a pair can pass only once the two
@@ -835,46 +836,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CYL ? 2 : 3
                 fl = A.nbr_count[i];
                 moved = A.disp[i];
             }
-            gap = A.gap[i];
+            if (!built || (fl & kCandidate)) gap = A.gap[i];
         }
         const bool test = (fl & kCandidate) && ((fl & kMeshNear) || !(gap > (moved + dm) * 1.0001f + 1e-9f));
-        const unsigned long long tests = __ballot(test);
-        const uint32_t ntest = (uint32_t)__popcll(tests);
-        if (test) test_lane[wave][__popcll(tests & ((1ull << lane) - 1ull))] = lane;
-        wave_lds_sync();
-        uint32_t ws = lanes_log2;
-        if (per == 64u) {
-            // a wave of 64 spheres: a lane each, more only where the keys of its longest list need
-            // the room (1,024 keys a wave)
-            uint32_t nmax = test ? min(fl & kCountMask, A.list_cap) : 0u;
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor(nmax, off, 64));
-            nmax = __builtin_amdgcn_readfirstlane(nmax);
-            ws = nmax > 32u ? 2u : (nmax > 16u ? 1u : 0u);
+        bool touch = false;
+        if (__any(test)) {
+            uint32_t ws = lanes_log2;
+            if (per == 64u) {
+                // a wave of 64 spheres: a lane each, more only where the keys of its longest list need
+                // the room (1,024 keys a wave)
+                const uint32_t n = test ? min(fl & kCountMask, A.list_cap) : 0u;
+                ws = __any(n > 32u) ? 2u : (__any(n > 16u) ? 1u : 0u);
+            }
+            TouchGroup T;
+            T.W = 1u << ws;
+            T.l = lane & (T.W - 1u);
+            T.g0 = lane - T.l;
+            const uint32_t g = lane >> ws;
+            T.keys = keys_all[wave] + 16u * T.W * g;
+            if (ws == 0u) {
+                touch = touch_sphere<MULTI, CYL, true>(A, T, test ? i : kInvalid, fl);   // its own
+            } else {
+                if (built) {   // the lists that the lanes have just stored are read back by other lanes
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                }
+                // the spheres to test, dealt to the groups
+                const unsigned long long tests = __ballot(test);
+                const uint32_t ntest = (uint32_t)__popcll(tests), groups = 64u >> ws;
+                const uint32_t place = (uint32_t)__popcll(tests & ((1ull << lane) - 1ull));
+                if (test) test_lane[wave][place] = lane;
+                wave_lds_sync();
+                for (uint32_t r = 0; r < ntest; r += groups) {
+                    const uint32_t q = r + g;
+                    const int src = q < ntest ? (int)test_lane[wave][q] : 0;
+                    const uint32_t fs = __shfl(fl, src, 64), is = __shfl(i, src, 64);
+                    const bool t = touch_sphere<MULTI, CYL, false>(A, T, q < ntest ? is : kInvalid, fs);
+                    if (T.l == 0u && q < ntest) test_lane[wave][q] = t ? 64u + (uint32_t)src : (uint32_t)src;
+                }
+                wave_lds_sync();
+                touch = test && test_lane[wave][place] >= 64u;
+                wave_lds_sync();   // test_lane is written again
+            }
         }
-        TouchGroup T;
-        T.W = 1u << ws;
-        T.l = lane & (T.W - 1u);
-        T.g0 = lane - T.l;
-        const uint32_t g = lane >> ws, groups = 64u >> ws;
-        T.keys = keys_all[wave] + 16u * T.W * g;
-        for (uint32_t r = 0; r < ntest; r += groups) {
-            const uint32_t q = r + g;
-            const int src = q < ntest ? (int)test_lane[wave][q] : 0;
-            const uint32_t fs = __shfl(fl, src, 64), is = __shfl(i, src, 64);
-            const uint32_t it_ = q < ntest ? is : kInvalid;
-            const bool t = T.W == 1u ? touch_sphere<MULTI, CYL, true>(A, T, it_, fs)
-                                     : touch_sphere<MULTI, CYL, false>(A, T, it_, fs);
-            if (T.l == 0u && q < ntest) test_lane[wave][q] = t ? 64u + (uint32_t)src : (uint32_t)src;
-        }
-        wave_lds_sync();
-        const bool touch = test && test_lane[wave][__popcll(tests & ((1ull << lane) - 1ull))] >= 64u;
         // a touched sphere's rotation, acceleration and contact counts are written by the full
         // pass: no longer known stable
         const uint32_t nf = touch ? ((fl & ~kLiteStable) | kTouch) : (fl & ~kTouch);
         if (i < A.np && (built || nf != fl)) A.nbr_count[i] = nf;
         queue_append(A.work2, A.seg_count2, seg, A.seg_cap, touch, i);
-        wave_lds_sync();   // test_lane is written again
     }
 }
 
@@ -1315,11 +1324,20 @@ __device__ __forceinline__ void lite_sphere(const StepArgs& A, const SceneDev& S
 
 // k_rebuild's phase cursors, counters and release flags start at zero: cleared by block 0 of
 // the lite pass (after k_touch has read the release flags, before the next step's
-// k_rebuild).
+// k_rebuild). After a build, it also leaves the candidates and their lists' entries, added up over
+// the segments, to the k_touch of the later steps: the 64 lines of a total, read by each of that
+// kernel's waves, cost a step without contacts 1 us.
 __device__ __forceinline__ void reset_rebuild_slots(const StepArgs& A)
 {
-    if (blockIdx.x == 0)
-        for (uint32_t t = threadIdx.x; t < kBarSlots; t += blockDim.x) A.grid_bar[kSegStride * t] = 0u;
+    if (blockIdx.x != 0) return;
+    for (uint32_t t = threadIdx.x; t < kBarSlots; t += blockDim.x) A.grid_bar[kSegStride * t] = 0u;
+    if (*A.rebuild_cur != 0u && threadIdx.x < 64u) {
+        const uint32_t n = queue_total(A.seg_count), listed = queue_total(A.seg_count + 1);
+        if (threadIdx.x == 0u) {
+            A.seg_count[kCandTotal] = n;
+            A.seg_count[kListedTotal] = listed;
+        }
+    }
 }
 
 // The lite kernels run over every sphere outside this step's full pass (skip kTouch), one
@@ -1516,11 +1534,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     // the first queue entries of a wave of kQueueGroup, read together with the counts
     const uint32_t at_first = (qb.chunk * 4u + wave) * kQueueGroup + lane;
     const uint32_t early = lane < kQueueGroup && at_first < A.seg_cap ? qseg[at_first] : kInvalid;
+    const uint32_t seg_spheres = A.seg_count2[qb.seg * kSegStride];
     const uint32_t nfull = queue_total(A.seg_count2);
     const bool sweep = 2ull * nfull >= (unsigned long long)A.nsorted;
     // the wave's spheres: sorted slots (it = virtual block of 4 G slots) or queue entries (it =
     // the wave's first entry); either way the loop bounds are the same for the whole wave
-    const uint32_t qcnt = sweep ? 0u : A.seg_count2[qb.seg * kSegStride];
+    const uint32_t qcnt = sweep ? 0u : seg_spheres;
     const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;   // a multiple of 4
     const uint32_t todo = sweep ? A.nsorted : qcnt;
     const uint32_t halve = nfull < kTwoWavesFrom && gridDim.x > A.half_grid ? 2u : 1u;
@@ -1529,6 +1548,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint32_t it0 = sweep ? blockIdx.x : (qb.chunk * 4u + wave) * G;
     const uint32_t it_end = sweep ? nvb : qcnt;
     const uint32_t it_step = sweep ? gridDim.x : waves * G;
+    if (it0 >= it_end) return;   // the whole wave
     unsigned long long c0 = 0, c1 = 0;
     float dmx = 0.0f;
     for (uint32_t it = it0; it < it_end; it += it_step) {
