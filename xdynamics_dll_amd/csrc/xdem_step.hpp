@@ -703,6 +703,21 @@ __device__ __forceinline__ uint32_t queue_total(const uint32_t* seg_count)
     return c;
 }
 
+// Whether a kernel over n of the sorted slots finds them by sweeping the slots, each XCD one
+// contiguous eighth (its L2 then holds the positions that its spheres' lists name), rather than
+// from their queue: from half of the slots on, in sets of kSweepLarge slots from three quarters. A
+// sweep gives a small set more waves and its neighbours one L2, but takes lanes for the other
+// slots. A step with 55 percent of the spheres touched, swept and from the queue: 36 and 41 us for
+// 10,000, 44 and 45 for 30,000, 74 and 62 for 100,000, 136 and 108 for 300,000, 440 and 312 for
+// 1,000,000; with 75 percent, scattered over a pack: 83 and 87 for 100,000, 182 and 185 for
+// 300,000; with all: 156 and 163 for 300,000.
+constexpr uint32_t kSweepLarge = 65536;
+
+__device__ __forceinline__ bool sweep_slots(uint32_t n, uint32_t nsorted)
+{
+    return 4ull * n >= (nsorted < kSweepLarge ? 2ull : 3ull) * nsorted;
+}
+
 // Appends the lanes with `on` set to queue segment seg (one atomic per wave, by its first
 // active lane).
 __device__ __forceinline__ void queue_append(uint32_t* q, uint32_t* count, uint32_t seg, uint32_t cap, bool on,
@@ -722,9 +737,8 @@ __device__ __forceinline__ void queue_append(uint32_t* q, uint32_t* count, uint3
 // phases completed), one thread per sorted slot does the pair search for the slot's sphere
 // (pairs_slot: its list, list gap and candidate flags, the candidate queue work), then the wave
 // the exact test of its candidates on the lists it has just written. On the other steps, the
-// candidates of the last build: those of at least half the sorted slots by sweeping the slots,
-// each XCD one contiguous eighth of them (its L2 then holds the positions that its spheres'
-// lists name), fewer from their queue (block b walks segment b mod kQueueSegs); candidates whose
+// candidates of the last build: by sweeping the slots or from their queue (sweep_slots; block b
+// walks segment b mod kQueueSegs); candidates whose
 // gap exceeds their displacement plus the largest displacement since the build cannot touch and
 // are not tested. Touched spheres get kTouch, the pass mask, and a place in the full-pass queue
 // work2 (the segment of their sorted slot, so a segment never holds more than seg_cap); the
@@ -769,7 +783,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CYL ? 2 : 3
     const uint32_t at64 = (qb.chunk * 4u + wave) * 64u + lane;
     const uint32_t early = !built && at64 < A.seg_cap ? wq[at64] : kInvalid;
     const uint32_t ncand = A.seg_count[kCandTotal], nlisted = A.seg_count[kListedTotal];
-    const bool sweep = built || 2ull * ncand >= (unsigned long long)A.nsorted;
+    const bool sweep = built || sweep_slots(ncand, A.nsorted);
     if (!sweep && mine == 0u) return;
     const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;
     const uint32_t todo = sweep ? A.nsorted : mine;
@@ -1485,11 +1499,9 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
     });
 }
 
-// Full pass over the spheres k_touch queued. A wave takes G of them, one per owner lane: when at
-// least half the sorted slots are touched (a dense pack), found in sorted-slot order, each XCD
-// sweeping one contiguous eighth of the slots, so the neighbours a block gathers were mostly
-// fetched into its XCD's L2 by the blocks of adjacent slots; otherwise from the full-pass queue
-// (block b takes segment b mod 64). It numbers their passing pairs consecutively, sphere after
+// Full pass over the spheres k_touch queued. A wave takes G of them, one per owner lane: in
+// sorted-slot order or from the full-pass queue (sweep_slots; block b takes segment b mod 64). It
+// numbers their passing pairs consecutively, sphere after
 // sphere, in rank order (an exclusive scan of the pass-mask counts). The lanes then evaluate the
 // pairs 64 at a time: entry x belongs to the lane L whose range [s_L, s_L + c_L) holds it (a
 // binary search over the scanned ends), its rank is x - s_L and its list entry the rank-th set
@@ -1501,10 +1513,10 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
 // kTwoWavesFrom touched spheres on two waves per SIMD. Two waves share a SIMD's issue slots, but
 // one waits while the other works: a step of 10,000 spheres 47.4 us with one and 50.6 with two,
 // 20,000: 55.5 and 57.0, 25,000: 62.0 and 62.8, 31,000: 67.9 and 64.6, 90,000: 108 and 96. At
-// least four spheres to a wave was slower below 4,000 spheres (1,000: 46.3 and 43.3 us). From the
-// queue at least kQueueGroup: most spheres are then in the lite pass beside this kernel, which
-// more waves slow down, and the few have few pairs. Steps of a falling column of 1,000,000 with
-// 1,500 touched spheres, per 50: 4.68 ms from 1 sphere to a wave, 4.50 from 16, 4.44 from 32,
+// least four spheres to a wave was slower below 4,000 spheres (1,000: 46.3 and 43.3 us).
+// From the queue at least kQueueGroup: most spheres are then in the lite pass beside this kernel,
+// which more waves slow down, and the few have few pairs. Steps of a falling column of 1,000,000
+// with 1,500 touched spheres, per 50: 4.68 ms from 1 sphere to a wave, 4.50 from 16, 4.44 from 32,
 // 4.48 from 64; 48 scenes with 10,000 to 20,000 touched of 474,000, per 20: 1.88 to 2.25 ms, 1.91
 // to 2.26, 1.91 to 2.12, 2.03 to 2.14.
 //
@@ -1536,7 +1548,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint32_t early = lane < kQueueGroup && at_first < A.seg_cap ? qseg[at_first] : kInvalid;
     const uint32_t seg_spheres = A.seg_count2[qb.seg * kSegStride];
     const uint32_t nfull = queue_total(A.seg_count2);
-    const bool sweep = 2ull * nfull >= (unsigned long long)A.nsorted;
+    const bool sweep = sweep_slots(nfull, A.nsorted);
     // the wave's spheres: sorted slots (it = virtual block of 4 G slots) or queue entries (it =
     // the wave's first entry); either way the loop bounds are the same for the whole wave
     const uint32_t qcnt = sweep ? 0u : seg_spheres;
