@@ -1,8 +1,9 @@
 """Scenes of which a part is touched: the pair-test and contact kernels take their spheres by sweeping
 the sorted slots from half of them on, in scenes of 65,536 spheres or more from three quarters, and
-else from a queue. FP64 states, histories and counts are the oracle's at both sides of each line. A
-step's time grows as the touched spheres do: of 1,000,000 with 55 percent touched at most 1.22
-(55 / 45) times that with 45 percent, and a fifth more for what else differs."""
+else from a queue, at least 4 to 32 spheres to a wave by how many are untouched. FP64 states,
+histories and counts are the oracle's at both sides of each line. A step's time grows as the touched
+spheres do: of 1,000,000 with 55 percent touched at most 1.22 (55 / 45) times that with 45 percent,
+and a fifth more for what else differs."""
 import time
 
 import numpy as np

@@ -959,7 +959,7 @@ __device__ __forceinline__ void sphere_tail(const StepArgs& A, const SceneDev& S
 // Cohesion-only pairs add their attraction. The first kPairIds slot ids of the previous step
 // are staged in LDS.
 constexpr uint32_t kPairIds = 16;
-constexpr uint32_t kQueueGroup = 32;     // k_collide: the fewest spheres to a wave that takes them from the queue
+constexpr uint32_t kQueueGroup = 32;     // k_collide: the fewest spheres to a wave beside a long lite pass
 constexpr uint32_t kTwoWavesFrom = 26000; // k_collide: the touched spheres from which SIMDs get two waves
 
 // Sphere i's pair with neighbour k: the neighbour's state, the history entry of `slot`, the
@@ -1514,11 +1514,15 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
 // one waits while the other works: a step of 10,000 spheres 47.4 us with one and 50.6 with two,
 // 20,000: 55.5 and 57.0, 25,000: 62.0 and 62.8, 31,000: 67.9 and 64.6, 90,000: 108 and 96. At
 // least four spheres to a wave was slower below 4,000 spheres (1,000: 46.3 and 43.3 us).
-// From the queue at least kQueueGroup: most spheres are then in the lite pass beside this kernel,
-// which more waves slow down, and the few have few pairs. Steps of a falling column of 1,000,000
-// with 1,500 touched spheres, per 50: 4.68 ms from 1 sphere to a wave, 4.50 from 16, 4.44 from 32,
-// 4.48 from 64; 48 scenes with 10,000 to 20,000 touched of 474,000, per 20: 1.88 to 2.25 ms, 1.91
-// to 2.26, 1.91 to 2.12, 2.03 to 2.14.
+//
+// From the queue at least 4 to kQueueGroup, by the spheres of the lite pass beside this kernel: more
+// waves slow a long lite pass down, and the few touched spheres have few pairs. Steps of a falling
+// column of 1,000,000 with 1,500 touched spheres, per 50: 4.68 ms from 1 sphere to a wave, 4.50
+// from 16, 4.44 from 32, 4.48 from 64; 48 scenes with 10,000 to 20,000 touched of 474,000, per 20:
+// 1.88 to 2.25 ms, 1.91 to 2.26, 1.91 to 2.12, 2.03 to 2.14. A short one does not matter: steps
+// with 10 percent of 10,000 spheres touched 39.7 us from 4 and 42.4 from 32, 45 percent of 30,000
+// 42.5 and 44.4, 2 percent of 100,000 41.0 and 43.5, of 300,000 49.8 and 52.5. From kTwoWavesFrom
+// touched spheres always kQueueGroup: 45 percent of 100,000 56 and 53, 10 of 300,000 57 and 51.
 //
 // Bound by the latency of a wave's chain (list entry, neighbour state, the FP64 divisions and
 // roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 18 us for
@@ -1555,7 +1559,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const uint32_t waves = sweep ? gridDim.x * 4u : qb.nchunk * 4u;   // a multiple of 4
     const uint32_t todo = sweep ? A.nsorted : qcnt;
     const uint32_t halve = nfull < kTwoWavesFrom && gridDim.x > A.half_grid ? 2u : 1u;
-    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(sweep ? 1u : kQueueGroup, (halve * todo + waves - 1u) / waves));
+    const uint32_t least = sweep ? 1u : (nfull >= kTwoWavesFrom ? kQueueGroup : min(kQueueGroup, max(4u, (A.nsorted - nfull) / 16384u)));
+    const uint32_t G = nfull >= A.group_max_from ? 64u : min(64u, max(least, (halve * todo + waves - 1u) / waves));
     const uint32_t nvb = (A.nsorted + 4u * G - 1u) / (4u * G);
     const uint32_t it0 = sweep ? blockIdx.x : (qb.chunk * 4u + wave) * G;
     const uint32_t it_end = sweep ? nvb : qcnt;
