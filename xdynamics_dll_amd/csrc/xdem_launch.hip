@@ -192,9 +192,14 @@ __device__ __forceinline__ ContactConst uniform_const(const xdem_contact_propert
 {
     ContactConst c = make_contact_const(*cp, 0.0);
     static_assert(sizeof(ContactConst) % sizeof(int) == 0, "copied by words");
-    int* w = reinterpret_cast<int*>(&c);
+    char* at = reinterpret_cast<char*>(&c);
 #pragma unroll
-    for (unsigned k = 0; k < sizeof(ContactConst) / sizeof(int); k++) w[k] = __builtin_amdgcn_readfirstlane(w[k]);
+    for (unsigned k = 0; k < sizeof(ContactConst) / sizeof(int); k++) {
+        int w;
+        __builtin_memcpy(&w, at + k * sizeof(int), sizeof(int));
+        w = __builtin_amdgcn_readfirstlane(w);
+        __builtin_memcpy(at + k * sizeof(int), &w, sizeof(int));
+    }
     return c;
 }
 
