@@ -34,65 +34,39 @@ def step_bytes(cbar: float) -> float:
     return 436.0 + 40.0 * cbar
 
 
-def merged_collide_kernel_bytes(spheres: float, wall_contacts: float, pairs: float) -> float:
-    """k_collide walking the pairs too: its own bytes without the pair sums' read (480 - 80),
-    plus the pair walk's pass mask 8 and old and new counts 4 + 4 per sphere and 44 per
-    passing pair (the own state is read once)."""
-    return (480.0 - 80.0 + 16.0) * spheres + 40.0 * wall_contacts + 44.0 * pairs
-
-
 # Algorithmic bytes per sphere of k_lite_move (the translation of every sphere outside the
 # step's full pass): the translational part of the per-sphere state traffic, read pos 32,
 # vel 24, acc 24, mass 8 and write pos 32, vel 24, acc 24.
 LITE_MOVE_BYTES = 168.0
 
 
-def pairs_kernel_bytes(spheres: float, pairs: float) -> float:
-    """Algorithmic bytes of one k_pairs launch: per full-pass sphere its own pos 32, vel 24,
-    mass 8, ep 32, ev 32, list flags 4, pass mask 8, old count 4, new count 4 and the ten pair
-    sums 80 (= 228); per listed pair that passes, its list entry 4, the old history slot read
-    (id 4, tsd 16) and the new one written (id 4, tsd 16) (= 44). A neighbour's state is some
-    other sphere's own state: it is counted once, as that sphere's (re-reads hit the caches
-    or are waste)."""
-    return 228.0 * spheres + 44.0 * pairs
-
-
-def collide_kernel_bytes(spheres: float, wall_contacts: float) -> float:
+def collide_kernel_bytes(spheres: float, wall_contacts: float, pairs: float) -> float:
     """Algorithmic bytes of one fused k_collide launch: per full-pass sphere its state read
-    (pos 32, vel 24, acc 24, ep 32, ev 32, ea 32, mass 8, inertia 24 = 208), the pair sums of
-    k_pairs 80, the list flags 4 and path length 4, the state written (pos 32, vel 24, acc 24,
-    ep 32, ev 32, ea 32 = 176) and the wall-slot count read and written 8 (= 480); per wall
-    contact its slot read and written (id 4 + tsd 16, twice = 40)."""
-    return 480.0 * spheres + 40.0 * wall_contacts
-
-
-# A library with a pair pass of its own walks the pairs inside k_collide when the step's full
-# pass holds fewer spheres than this.
-MERGE_PAIRS_BELOW = 65536
+    (pos 32, vel 24, acc 24, ep 32, ev 32, ea 32, mass 8, inertia 24 = 208), the list flags 4,
+    path length 4, pass mask 8 and old and new pair counts 8, the state written (pos 32, vel 24,
+    acc 24, ep 32, ev 32, ea 32 = 176) and the wall-slot count read and written 8 (= 416); per
+    wall contact its slot read and written (id 4 + tsd 16, twice = 40); per listed pair that
+    passes its list entry 4, the old history slot read and the new one written (20 each) (= 44).
+    A neighbour's state is some other sphere's own state: it is counted once, as that sphere's
+    (re-reads hit the caches or are waste)."""
+    return 416.0 * spheres + 40.0 * wall_contacts + 44.0 * pairs
 
 
 def kernel_rooflines(tm, n, info, n_pp, n_wall, fuse):
     """Per-step time and achieved HBM bandwidth of the step's kernels from the event-timed
-    steps: k_lite_move (spheres outside the full pass), k_pairs and k_collide (the full-pass
-    spheres, contact_spheres of the last step). Without a pair pass of its own (no time for it, or a
-    small full pass) k_collide walks the pairs and their bytes count for it."""
+    steps: k_lite_move (spheres outside the full pass) and k_collide (the full-pass spheres,
+    contact_spheres of the last step, and their pairs)."""
     steps = max(tm["steps"], 1)
     full = info["contact_spheres"]
-    merged = full < MERGE_PAIRS_BELOW or not tm.get("pair_pass_ms", 0) > 0
     out = {}
     if fuse and tm["lite_move_ms"] > 0:
         ms = tm["lite_move_ms"] / steps
         b = LITE_MOVE_BYTES * (n - full)
         out["k_lite_move"] = {"ms": ms, "bytes": b, "units": n - full, "bytes_per_unit": LITE_MOVE_BYTES}
-    if tm.get("pair_pass_ms", 0) > 0 and not merged:
-        ms = tm["pair_pass_ms"] / steps
-        b = pairs_kernel_bytes(full, n_pp)
-        out["k_pairs"] = {"ms": ms, "bytes": b, "units": full, "bytes_per_unit": b / max(full, 1)}
     if fuse and tm.get("collide_ms", 0) > 0:
         ms = tm["collide_ms"] / steps
-        b = merged_collide_kernel_bytes(full, n_wall, n_pp) if merged else collide_kernel_bytes(full, n_wall)
-        out["k_collide"] = {"ms": ms, "bytes": b, "units": full, "bytes_per_unit": b / max(full, 1),
-                            "walks_pairs": merged}
+        b = collide_kernel_bytes(full, n_wall, n_pp)
+        out["k_collide"] = {"ms": ms, "bytes": b, "units": full, "bytes_per_unit": b / max(full, 1)}
     for k in out.values():
         k["gbps"] = k["bytes"] / (k["ms"] * 1e-3) / 1e9
         k["frac"] = k["gbps"] / HBM_PEAK_GBPS
@@ -100,7 +74,10 @@ def kernel_rooflines(tm, n, info, n_pp, n_wall, fuse):
 
 
 def dominant_roofline(kr, traffic=None):
-    """The roofline object of the kernel with the longest time per step."""
+    """The roofline object of the kernel with the longest time per step (None in split mode, whose
+    kernels have no event times of their own)."""
+    if not kr:
+        return None
     name = max(kr, key=lambda k: kr[k]["ms"])
     k = kr[name]
     return {"bound": "hbm", "achieved": k["gbps"], "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": k["frac"],
@@ -274,7 +251,7 @@ def measured_traffic(np_, fused):
 WHEEL_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_wheel_500k.json")
 
 
-def wheel_traffic(np_, kernel="k_pairs"):
+def wheel_traffic(np_, kernel="k_collide"):
     """HBM bytes per dispatch of a full-pass kernel of the wheel workload from the committed
     rocprofv3 --pmc summary (scaled as in measured_traffic), or None when the summary is of
     another bed size."""
@@ -551,9 +528,7 @@ def wheel_main(args):
                                "2 rad/s about y, 200 N load, HHT alpha=-0.1, mu=0.6, dt=1e-5 s, mixed",
                    "np": n, "ntriangle": len(tris), "parallelism": "single GPU + host HHT",
                    "force_law": args.force_law},
-        "roofline": dominant_roofline(kr, {"k_pairs": wheel_traffic(n, "k_pairs"),
-                                           "k_collide": wheel_traffic(n, "k_collide")}
-                                      if args.force_law == "cpu" else None),
+        "roofline": dominant_roofline(kr, {"k_collide": wheel_traffic(n)} if args.force_law == "cpu" else None),
         "kernels": kr,
         "mean_contacts_per_sphere": (n_pp + n_wall + n_mesh) / n,
         "sphere_contacts": n_pp, "wall_contacts": n_wall, "mesh_contacts": n_mesh,
@@ -770,7 +745,7 @@ def main():
     ap.add_argument("--full-blocks", type=int, default=0,
                     help="blocks of the full-pass kernels (0 = library default)")
     ap.add_argument("--merge-below", type=int, default=0,
-                    help="full passes smaller than this walk their pairs in the contact kernel (0 = library default)")
+                    help="full passes of this size or more take 64 spheres to a wave (0 = by size)")
     ap.add_argument("--nscene", type=int, default=256, help="scenes of the batch workload")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
                     help="only run a plain device copy of MIB MiB (counter calibration)")
