@@ -166,12 +166,15 @@ typedef struct xdem_ctx_config {
     unsigned int full_blocks;    /* blocks of the full-pass kernels (pair, triangle and contact
                                     passes), taken to a multiple of 64 (0 = two per CU). They
                                     stride over the queued spheres, so results do not depend on
-                                    it. */
-    unsigned int merge_pairs_below; /* a step's full pass of fewer spheres than this is divided
-                                    into groups of 4 to 64 spheres to a wave, as few as fill the
-                                    device; from this size on every wave takes 64 (0 = the
-                                    first rule for every size; 1 = the second). Results do not
-                                    depend on it. */
+                                    it. The sphere pairs are part of the contact pass: fewer
+                                    blocks than the default slow a large one. */
+    unsigned int merge_pairs_below; /* a step's full pass of fewer spheres than this gives a wave
+                                    1 to 64 spheres (at least 4 to 32 where most are untouched),
+                                    as few as fill the device; from this size on every wave
+                                    takes 64 (0 = the first rule for every size; 1 = the
+                                    second). The name is that of an earlier rule, whether the
+                                    pairs had a pass of their own; they are always part of the
+                                    contact pass. Results do not depend on it. */
     int keep_order;              /* 0 (default): the context stores each scene's spheres in the
                                     bucket order of their initial positions (a stable sort on
                                     the bucket key at commit), so that the neighbours a kernel

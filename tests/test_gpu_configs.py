@@ -37,7 +37,7 @@ def test_box_lattice_10k_fp64_matches_oracle():
     step 2,200 (~700 sphere and 300 wall contacts) the FP64 step is bit-identical to the
     oracle: positions, velocities, accelerations, Euler parameters and their rates."""
     scene = SceneData.build(1, 1001)
-    # the same run with the pairs walked by the pair pass on every step (merge_pairs_below 1)
+    # the same run with 64 spheres to a wave of the contact kernel (merge_pairs_below 1)
     gpus = [DemContext(scene, precision="fp64", fuse_velocity=True, merge_pairs_below=m) for m in (0, 1)]
     ref = xdem_ref.RefSim(scene)
     done = 0
@@ -64,7 +64,7 @@ def test_batch_members_in_one_context_match_oracle():
     equals its own oracle run after 1, 10 and 400 steps."""
     scenes = [SceneData.build(4, 1004, variant=k) for k in range(8)]
     print(f"[cfg4 members] np={[s.np for s in scenes]}", flush=True)
-    # the default context and one whose pairs go through the pair pass on every step
+    # the default context and one with 64 spheres to a wave of the contact kernel
     gpus = [DemContext(scenes, precision="fp64", fuse_velocity=True, merge_pairs_below=m) for m in (0, 1)]
     refs = [xdem_ref.RefSim(s) for s in scenes]
     done = 0

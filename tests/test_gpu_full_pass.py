@@ -1,6 +1,6 @@
 """The full contact pass at the sizes where its division of work changes: a wave takes 1 to 64
-touched spheres, by whether SIMDs get one wave or two, found by sweeping the sorted slots when at
-least half of them are touched; otherwise at least 32 from the queue. FP64 states and histories
+touched spheres, by whether SIMDs get one wave or two, found by sweeping the sorted slots when half
+of them (three quarters in large scenes) are touched; otherwise at least 4 to 32 from the queue. FP64 states and histories
 are those of the oracle, bit for bit: the pass adds a sphere's pairs in the reference's order
 whatever the division."""
 import numpy as np

@@ -1,7 +1,7 @@
 """The launcher layer at the sizes where its division of work changes: the sphere launcher in
 groups of 2 to 16 particles a wave (more candidates and contacts than a round, a half or the slots
 hold). Integers are exact; sums and slots agree to 1e-12 of the largest (the material
-constants come from the device's log and the host's: a rounding of a term, at most 26 terms a sum)."""
+constants come from the device's log and the host's: a rounding of a term, at most 18 terms a sum)."""
 import ctypes as C
 
 import numpy as np
@@ -9,7 +9,7 @@ import pytest
 
 import xdem_ref
 from test_gpu_launchers import Arrays, call, dev, host, ptr, setup_params
-from xdynamics_dll_amd import SceneData, box_walls, contact_property
+from xdynamics_dll_amd import _lib, SceneData, box_walls, contact_property
 
 pytestmark = pytest.mark.gpu
 
@@ -20,8 +20,8 @@ torch = pytest.importorskip("torch")
 @pytest.mark.parametrize("n, pitch", [(1, 1.98e-3), (2, 1.98e-3), (27, 1.2e-3), (2049, 1.98e-3), (4099, 1.55e-3),
                                       (40001, 1.99e-3)])
 def test_sphere_launcher(n, pitch, coh):
-    """1.2 and 1.55 mm pitches overlap second neighbours too: up to 26 contacts a sphere, past the
-    12 slots, and over 64 pairs a group."""
+    """At a pitch of 1.2 mm second neighbours overlap too: up to 18 contacts a sphere, past the 12
+    slots, and over 64 pairs a group; at 1.55 mm six deep ones."""
     rng = np.random.default_rng(n)
     side = max(1, int(np.ceil(n ** (1.0 / 3.0))))
     k, rest = np.divmod(np.arange(n), side * side)
@@ -43,7 +43,7 @@ def test_sphere_launcher(n, pitch, coh):
              ptr(d.mass), ptr(d.tmax), ptr(d.rres), ptr(d.pp_count), ptr(d.pp_id), ptr(d.pp_tsd), ptr(d.sorted),
              ptr(d.cstart), ptr(d.cend), ptr(cp), n)
         ref.grid()
-        xdem_ref.lib().ref_calculate_p2p(*p2p_args(ref))
+        over = xdem_ref.lib().ref_calculate_p2p(*p2p_args(ref))
         torch.cuda.synchronize()
         for name in ("force", "moment", "tmax", "rres"):
             close(host(getattr(d, name)), getattr(ref, name), name)
@@ -54,6 +54,8 @@ def test_sphere_launcher(n, pitch, coh):
         close(host(d.pp_tsd)[used], ref.pp_tsd[used], "slots")
     word = C.c_uint()
     call("xdem_get_error_word", C.byref(word), 1)
+    assert word.value == (_lib.ERR_P2P_OVERFLOW if over else 0), hex(word.value)
+    assert bool(over) == (pitch == 1.2e-3)
 
 
 def close(a, b, name):

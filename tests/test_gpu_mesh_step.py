@@ -134,7 +134,7 @@ def test_terrain_mixed_precision_forces():
 def test_wheel_over_20k_bed_matches_oracle():
     scene, tris, dbi, cp = wheel_over_bed(20000)
     print(f"[wheel 20k] np={scene.np} ntri={len(tris)}", flush=True)
-    # the default context and one whose pairs go through the pair pass on every step
+    # the default context and one with 64 spheres to a wave of the contact kernel
     gpus = [DemContext(scene, precision="fp64", fuse_velocity=True, meshes=[(0, tris, dbi, cp)], merge_pairs_below=m)
             for m in (0, 1)]
     ref = xdem_ref.RefSim(scene)

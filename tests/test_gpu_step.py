@@ -6,10 +6,9 @@ absorbs libm differences in log/pow); pair sets are compared bit-exactly.
 Mixed path: per-sphere net-force error normalised by the sum of that sphere's pair-force
 magnitudes (FP64) <= 1e-4, pair sets bit-exact at the same input state.
 
-Sphere pairs are walked by the contact kernel itself when the full pass is small and by the
-pair pass (k_pairs, lanes packed over the pairs of 64 spheres) when it holds at least
-merge_pairs_below spheres; these scenes are below the default threshold, so the tests run
-with merge_pairs_below = 1 (every step through the pair pass) as well as with the default.
+The contact kernel gives a wave as few spheres as fill the device, or 64 in a full pass of
+merge_pairs_below spheres or more; these scenes are small, so the tests run with
+merge_pairs_below = 1 (64 to a wave on every step) as well as with the default.
 """
 import numpy as np
 import pytest
@@ -52,8 +51,7 @@ def compare_histories(gpu, ref, tol=1e-12):
     assert np.allclose(tsd, ref.pl_tsd, rtol=tol, atol=1e-300)
 
 
-# merge_pairs_below: 0 = the library's threshold (these scenes: the contact kernel walks the
-# pairs), 1 = the pair pass on every step
+# merge_pairs_below: 0 = waves sized to the step, 1 = 64 spheres to a wave on every step
 REGIMES = [0, 1]
 
 
@@ -212,10 +210,9 @@ def test_state_written_between_steps_matches_oracle(fuse):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
-def test_pair_pass_and_contact_kernel_walks_are_bit_identical(precision):
-    """The same scene stepped with the pairs walked by the contact kernel and by the pair pass:
-    states and histories equal bit for bit (both add the pairs in rank order with the same
-    operations)."""
+def test_waves_of_any_size_are_bit_identical(precision):
+    """The same scene stepped with waves sized to the step and with 64 spheres to a wave: states
+    and histories equal bit for bit (a sphere's pairs are added in rank order either way)."""
     scene = random_pack(n=3000)
     a = DemContext(scene, precision=precision, fuse_velocity=True)
     b = DemContext(scene, precision=precision, fuse_velocity=True, merge_pairs_below=1)

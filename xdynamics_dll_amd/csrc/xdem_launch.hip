@@ -1,5 +1,6 @@
 // xdem_launch.hip -- launcher-level C ABI: one gfx950 kernel per launcher of the
-// reference's CUDA layer, on the reference's array layouts (one thread per particle).
+// reference's CUDA layer, on the reference's array layouts: one thread per particle, but a wave for
+// 2 to 16 in the sphere and triangle launchers.
 // Built with -ffp-contract=off: FP64 results follow the reference's operation order.
 #include <algorithm>
 #include <mutex>
@@ -532,7 +533,6 @@ struct MeshStage {
     double own[4][kGroupMax];                        // position and radius
     unsigned hit_id[kGroupMax][kTriList];            // per owner: the contacts of its best kind so far
     double hit_pt[kGroupMax][kTriList][3];
-    int best[kGroupMax];                             // 2 faces, 1 edges, 0 vertices, -1 none
     unsigned hits[kGroupMax];
     double pt[3][64];                                // a round of candidates: closest point, kind, triangle
     int kind[64];                                    // bit 2: overlapping (the repeated-point rule applies)
@@ -567,7 +567,6 @@ __global__ __launch_bounds__(64 * kWaves) void k_mesh(LaunchPrm P, const xdem_tr
     if (lane < n_own) {
         const V4<double> p = ld4(pos + 4 * (size_t)(base + lane));
         st.own[0][lane] = p.x; st.own[1][lane] = p.y; st.own[2][lane] = p.z; st.own[3][lane] = p.w;
-        st.best[lane] = -1;
         st.hits[lane] = 0u;
     }
     wave_lds_sync();
@@ -585,7 +584,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_mesh(LaunchPrm P, const xdem_tr
         // of the half's sphere (kept by its first lane)
         V3<double> prev_line = mk3(0.0, 0.0, 0.0), prev_point = mk3(0.0, 0.0, 0.0);
         unsigned seen[3] = {0u, 0u, 0u}, nhit = 0;
-        int best = -1;
+        int best = -1;   // 2 faces, 1 edges, 0 vertices, -1 none
         for (unsigned r = 0; r < longest; r += 32u) {
             const unsigned x = r + c, at = walk.entry(x);
             const unsigned k = x < walk.total ? sorted_index[at] : 0u;

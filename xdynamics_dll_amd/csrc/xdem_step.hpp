@@ -1,11 +1,17 @@
 // xdem_step.hpp -- kernels of the fused DEM step (the xdem_ctx path).
 //
-// One step is the grid build of xdem_grid.hip (position update, bucket counting sort,
-// sorted copies) followed by
-//   k_collide         one thread per sorted slot: sphere-sphere contacts over the 27
-//                     neighbour buckets in the reference's (z, y, x) order, every wall of
-//                     the scene in id order, then (fused mode) rolling resistance and the
-//                     velocity/orientation-rate update (xIntegratorVV.cpp:131-152);
+// One step is
+//   k_rebuild         (xdem_grid.hip) every step's counters; on a build step the bucket grid;
+//   k_touch           on a build step the pair search, one thread per sorted slot; every step the
+//                     exact test of the candidates, which queues the touched spheres;
+//   k_mesh_pass       triangles of the touched spheres of scenes with a mesh;
+//   k_collide         the touched spheres, 1 to 64 to a wave, their pairs packed over the lanes:
+//                     sphere-sphere contacts in the reference's (z, y, x) order of cells, every wall
+//                     of the scene in id order, cylinders, triangle sums, then (fused mode) rolling
+//                     resistance and the velocity/orientation-rate update
+//                     (xIntegratorVV.cpp:131-152);
+//   k_lite_move, k_lite_turn, k_collide_lite
+//                     the other spheres, beside k_collide;
 //   k_finish          (split mode) rolling resistance and the velocity update.
 // Several independent scenes share the launches: each scene owns a range of buckets, so
 // spheres of different scenes never meet in a bucket.
@@ -131,9 +137,10 @@ struct CylDev {
     uint32_t pad_;
 };
 
-// Entry k of a table of scenes or bodies, read through the constant address space: a kernel never
-// changes these tables, so an index that is the same in all lanes gives scalar loads, which do
-// not wait for the lanes' own loads and stores, and keep the constants in scalar registers.
+// Entry k of a table of scenes or bodies, read through the constant address space: no kernel that
+// reads these tables so writes them (k_set_mesh_pose writes the meshes, in a launch of its own), so
+// an index that is the same in all lanes gives scalar loads, which do not wait for the lanes' own
+// loads and stores, and keep the constants in scalar registers.
 template <class E> __device__ __forceinline__ const E& table_at(const E* t, uint32_t k)
 {
     return *(const E*)((const __attribute__((address_space(4))) E*)t + k);

@@ -44,7 +44,7 @@ class DemContext:
         cfg.step_graph = step_graph   # > 0: step() replays HIP graphs of that many steps; 0: eager launches
         cfg.rebuild_wait_limit = rebuild_wait_limit   # 0: ~1 s before a rebuild phase gives up
         cfg.full_blocks = full_blocks   # 0: two blocks per CU for the full-pass kernels
-        cfg.merge_pairs_below = merge_pairs_below   # 0: 4 to 64 spheres to a wave by size; 1: always 64
+        cfg.merge_pairs_below = merge_pairs_below   # 0: 1 to 64 spheres to a wave by size; k: 64 from full passes of k on
         cfg.keep_order = 1 if keep_order else 0   # 0: spheres stored in bucket order (API calls keep the caller's)
         cfg.skin_cap = skin_cap   # 0: the adaptive skin goes up to 0.4 of the smallest radius
         self.precision = precision
