@@ -661,8 +661,7 @@ int xdem_ctx_add_scene(xdem_ctx* c, const xdem_scene* s, unsigned int* idx)
     D.gx = s->gravity[0]; D.gy = s->gravity[1]; D.gz = s->gravity[2];
     D.grid.wo_x = wo[0]; D.grid.wo_y = wo[1]; D.grid.wo_z = wo[2];
     D.grid.cs = bucket_cs;
-    D.ref_cs = s->cell_size;
-    D.ref_inv = 1.0 / s->cell_size;
+    D.set_ref_cell(s->cell_size);
     D.skin = skin;
     D.grid.mask_x = dims[0] - 1; D.grid.mask_y = dims[1] - 1; D.grid.mask_z = dims[2] - 1;
     D.grid.dim_x = dims[0];
@@ -1645,7 +1644,7 @@ int xdem_ctx_add_mesh(xdem_ctx* c, unsigned int scene, const xdem_mesh* m, unsig
         c->wslots.push_back({sh.dev.p_begin, sh.dev.p_end, kMeshNear, 0u});
     }
     // the reference's cell is twice the largest of the sphere and proxy radii
-    sh.dev.ref_cs = std::max(sh.dev.ref_cs, 2.0 * maxprox);
+    sh.dev.set_ref_cell(std::max(sh.dev.ref_cs, 2.0 * maxprox));
     sh.dev.mesh = (int32_t)c->meshes.size();
     c->ntri += T;
     if (idx) *idx = (unsigned)c->meshes.size();

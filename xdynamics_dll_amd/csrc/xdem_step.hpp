@@ -101,6 +101,12 @@ struct SceneDev {
     uint32_t cyl_begin;       // the scene's cylinder bodies in StepArgs::cyls
     uint32_t ncyl;
     uint32_t cyl_id0;         // a cylinder of the scene has id 0 (it restarts the cylinder slots)
+
+    void set_ref_cell(double cs)
+    {
+        ref_cs = cs;
+        ref_inv = 1.0 / cs;
+    }
 };
 
 // A rigid triangle mesh body of a scene. Triangles keep their body-frame vertices; the
