@@ -406,6 +406,25 @@ __device__ __forceinline__ CylAxis cylinder_axis(const xdem_cylinder_info& cy, c
     return a;
 }
 
+// x and z of the rim circle's point (radius rr) towards (x, z) in the body's frame, by the atan /
+// sin / cos construction of the kernel text. Not inlined: the kernels with cylinders would hold its
+// registers for a point that few spheres need. Inlined, k_collide spilled 66 to 83 of them (24 now)
+// and k_touch, 198 registers, fitted two waves per SIMD (131 now, three): a step of loose spheres in
+// a drum 56 and 51 us (60,000), of a full drum 46 and 42 (10,000), 84 and 76 (60,000), 274 and 259
+// (300,000).
+__device__ __attribute__((noinline)) inline double2 rim_point(double x, double z, double rr)
+{
+    const double phi = atan(x / z);
+    double lx;
+    if (phi < 0 && z < 0) lx = rr * sin(-phi);
+    else if (phi > 0 && x < 0 && z < 0) lx = rr * sin(-phi);
+    else lx = rr * sin(phi);
+    double lz = rr * cos(phi);
+    if (z < 0 && lz > 0) lz = -lz;
+    else if (z > 0 && lz < 0) lz = -lz;
+    return make_double2(lx, lz);
+}
+
 // Overlap of a sphere (centre p, radius r) with the cylinder (impl:1189-1288); u is the unit
 // vector along which the force acts, inner is set for a sphere inside the tube (or on its
 // axis). The regions, in the reference's order:
@@ -451,16 +470,8 @@ __device__ __forceinline__ double cylinder_detection(const xdem_cylinder_info& c
         at = rot_local(p - a.base, a.e);
         rim = a.base;
     }
-    const double rr = cy.len_rr.z;
-    const double phi = atan(at.x / at.z);
-    double lx;
-    if (phi < 0 && at.z < 0) lx = rr * sin(-phi);
-    else if (phi > 0 && at.x < 0 && at.z < 0) lx = rr * sin(-phi);
-    else lx = rr * sin(phi);
-    double lz = rr * cos(phi);
-    if (at.z < 0 && lz > 0) lz = -lz;
-    else if (at.z > 0 && lz < 0) lz = -lz;
-    const V3<double> c = rim + rot_global(mk3(lx, 0.0, lz), a.e);
+    const double2 l = rim_point(at.x, at.z, cy.len_rr.z);
+    const V3<double> c = rim + rot_global(mk3(l.x, 0.0, l.y), a.e);
     const V3<double> dv = c - p;
     const double d = length(dv);
     u = dv / d;

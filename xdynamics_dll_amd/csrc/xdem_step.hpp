@@ -763,14 +763,10 @@ __device__ __forceinline__ void queue_append(uint32_t* q, uint32_t* count, uint3
 // set of candidates takes 4 to 16 lanes a sphere, one such round trip on more waves; a large one
 // a lane a sphere. Per launch, against a lane a sphere for every set and a root for every pair:
 // 10,000 candidates with lists of 14: 27 -> 11 us, 61,000: 35 -> 20, 500,000: 109 -> 90 (the
-// build steps among them, with lists sorted by rank in LDS: 440 -> 300). Three waves per SIMD; two
-// where the reach test of cylinders is in the kernel, which at three spills 38 to 47 registers: a
-// step of loose spheres in a drum 29 us with the kernel of a lane a sphere, 33 with three waves, 31
-// with two (10,000), 32, 36 and 34 (60,000); a drum full of 60,000 142, 88 and 85. (Their grid stays
-// that of three waves, a second round of half the blocks: with two thirds of it a drum of 300,000
-// took 284 us, not 276.)
+// build steps among them, with lists sorted by rank in LDS: 440 -> 300). Three waves per SIMD: the
+// 131 to 134 registers fit, and a fourth wave spills (500,000 candidates 2 percent slower, a fifth 9).
 template <bool MULTI, bool CYL, bool MESH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CYL ? 2 : 3))) void k_touch(StepArgs A)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_touch(StepArgs A)
 {
     const bool built = *A.rebuild_cur != 0u;
     // A build always completes: a rebuild block that stops waiting (XDEM_ERR_GRID_SYNC, a
