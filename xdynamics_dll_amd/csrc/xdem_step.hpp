@@ -1534,11 +1534,11 @@ __global__ __launch_bounds__(256) void k_lite_turn(StepArgs A)
 // touched spheres always kQueueGroup: 45 percent of 100,000 56 and 53, 10 of 300,000 57 and 51.
 //
 // Bound by the latency of a wave's chain (list entry, neighbour state, the FP64 divisions and
-// roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 18 us for
-// 1,000 touched spheres, 27 us for 10,000, 46 us for 61,000 (FP64 and DHS; a thread per sphere
+// roots of a pair, the walls, the update) up to about 100,000 spheres: per launch 17 us for
+// 1,000 touched spheres, 24 us for 10,000, 39 us for 61,000 (FP64 and DHS; a thread per sphere
 // walking its own pairs: 44 us for 10,000 and 88 us for 61,000). Beyond, two waves per SIMD wait
-// for the neighbour gathers: 500,000 spheres with 3.4M pairs 266 us, half of the line requests
-// missing L2 (a pair pass with a second pass over the spheres for the rest: 172 + 110 us and 160
+// for the neighbour gathers: 500,000 spheres with 3.5M pairs 252 us, 644 MB read and 179 written
+// past L2 (a pair pass with a second pass over the spheres for the rest: 172 + 110 us and 160
 // bytes a sphere between them). What the chain waits for is kept short: the scene and wall
 // tables are scalar loads (as vector loads each waited for the wave's earlier stores), a
 // sphere's flags, mask, state and slot ids are loaded together, new slots are stored after the
