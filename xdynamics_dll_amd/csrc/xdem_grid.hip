@@ -83,14 +83,13 @@ __device__ __forceinline__ void st_co(uint32_t* p, uint32_t v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Every step, block 0: clears the step's contact counters, full-pass queue and the next
-// step's rebuild flag.
+// Every step, block 0: clears the step's full-pass queue and the next step's rebuild flag (the
+// contact counters, 64 lines more, are cleared by the last block of k_touch: nothing runs beside
+// this kernel, and here they cost 0.4 us of a step of 1,000,000 spheres, 51.9 -> 51.5).
 __device__ __forceinline__ void step_counters(const StepArgs& A)
 {
     if (blockIdx.x != 0) return;
     if (threadIdx.x < kQueueSegs) {
-        A.counters[threadIdx.x * kCounterStride] = 0ull;
-        A.counters[threadIdx.x * kCounterStride + 1u] = 0ull;
         A.seg_count2[threadIdx.x * kSegStride] = 0u;
         A.dmax_next[threadIdx.x * kSegStride] = 0u;
     }

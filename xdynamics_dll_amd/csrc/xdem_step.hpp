@@ -769,6 +769,8 @@ template <bool MULTI, bool CYL, bool MESH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_touch(StepArgs A)
 {
     const bool built = *A.rebuild_cur != 0u;
+    if (blockIdx.x + 1u == gridDim.x && threadIdx.x < kQueueSegs)   // the step's contact counters
+        *reinterpret_cast<ulonglong2*>(A.counters + threadIdx.x * kCounterStride) = make_ulonglong2(0ull, 0ull);
     // A build always completes: a rebuild block that stops waiting (XDEM_ERR_GRID_SYNC, a
     // warning) has done every unit it claimed, and the block that completes a phase's last
     // unit passes its own wait and goes on, so every later phase still runs to the end. The
